@@ -257,10 +257,11 @@ int mhd_precond_setup(mhd_ctx *ctx, const mhd_solver_opts *opts);
  * result in every run) through a workspace of the context, so calls that
  * overlap each other or a solve of the same context on another stream race. */
 int mhd_smoother_apply_d(mhd_ctx *ctx, const void *d_r, void *d_y, void *stream);
-/* The vertex-patch inversions of mhd_precond_setup (batched Gauss-Jordan)
- * pivot on the diagonal while |a_kk| >= tau max_{i>k} |a_ik| and invert a patch
- * whose diagonal pivot fails that test again with partial pivoting (the
- * largest |a_ik|).  tau in [0, 1]: 1 = every patch with partial pivoting,
+/* The vertex-patch inversions of mhd_precond_setup (batched Gauss-Jordan on
+ * the patch matrices with the cells' interior current dofs eliminated and the
+ * rows scaled by powers of two to a diagonal in [1, 2)) pivot on the diagonal
+ * while |a_kk| >= tau max_{i>k} |a_ik| and invert a patch whose diagonal pivot
+ * fails that test again with partial pivoting (the largest |a_ik|).  tau in [0, 1]: 1 = every patch with partial pivoting,
  * 0 = diagonal pivots unless one is zero.  Default 0.03; applies to the
  * attached coarse levels too.  No counterpart in the reference (its patch
  * solves are library LU factorisations). */
@@ -276,7 +277,8 @@ int mhd_smoother_info(mhd_ctx *ctx, int64_t *npatch, int64_t *patch_dim, int64_t
  * solve (the CPU Newton-step baseline).  out[MHD_NOPS]:
  *   0  nonzeros streamed by SpMVs with FP64 values (A, the A11 / A1x blocks, P, P^T)
  *   1  nonzeros streamed by SpMVs with FP32 values
- *   2  patch-inverse entries applied by the smoother in FP64
+ *   2  patch-inverse entries (and entries of the cells' condensation couplings)
+ *      applied by the smoother in FP64
  *   3  ... in FP32
  *   4  ... in BF16
  *   5  entries of the dense coarsest inverse applied
