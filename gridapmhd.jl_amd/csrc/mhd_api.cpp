@@ -271,7 +271,15 @@ int mhd_create_stabilized(mhd_ctx **out, const mhd_mesh *mesh, const mhd_spaces 
       c->err = "too many cells for the row-assembly index (int32)";
       return -1;
     }
-    std::vector<int32_t> crow(n + 1), centry(ptr[n]);
+    std::vector<int32_t> crow(n + 1), centry(ptr[n]), cfp(c->ncells + 1, 0), cfc(std::max(c->nfaces, 1), 0);
+    for (int f = 0; f < c->nfaces; ++f) ++cfp[mesh->tw_face_cell[f] + 1];
+    for (int32_t cc = 0; cc < c->ncells; ++cc) cfp[cc + 1] += cfp[cc];
+    {
+      std::vector<int32_t> fill3(cfp.begin(), cfp.end() - 1);
+      for (int f = 0; f < c->nfaces; ++f) cfc[fill3[mesh->tw_face_cell[f]]++] = f;
+    }
+    if ((rc = dev_upload(c, &c->d_cfptr, cfp.data(), cfp.size()))) return rc;
+    if ((rc = dev_upload(c, &c->d_cface, cfc.data(), cfc.size()))) return rc;
     for (int64_t i = 0; i <= n; ++i) crow[i] = (int32_t)ptr[i];
     {
       std::vector<int64_t> fill2(ptr.begin(), ptr.end() - 1);
@@ -282,6 +290,7 @@ int mhd_create_stabilized(mhd_ctx **out, const mhd_mesh *mesh, const mhd_spaces 
         }
     }
     if ((rc = dev_upload(c, &c->d_crow, crow.data(), crow.size()))) return rc;
+    c->nhold = (int64_t)centry.size();
     if (centry.empty()) centry.push_back(0);
     if ((rc = dev_upload(c, &c->d_centry, centry.data(), centry.size()))) return rc;
     // a dof listed twice in one cell (periodic direction one cell thick)
@@ -302,6 +311,7 @@ int mhd_create_stabilized(mhd_ctx **out, const mhd_mesh *mesh, const mhd_spaces 
   MHD_HIP(hipMalloc(&c->d_val, sizeof(double) * std::max<int64_t>(c->nnz, 1)));
   MHD_HIP(hipMalloc(&c->d_x, sizeof(double) * std::max<int64_t>(n, 1)));
   MHD_HIP(hipMalloc(&c->d_r, sizeof(double) * std::max<int64_t>(n, 1)));
+  if ((rc = mhd_build_face_matrices(c)) || (rc = mhd_cellop_build(c))) return rc;
   if (nskel > 0) {
     // skeleton entries of every row, in increasing face order
     std::vector<int32_t> srow(n + 1, 0);
@@ -357,7 +367,8 @@ void mhd_destroy(mhd_ctx *c) {
   void *ptrs[] = {c->d_xyz, c->d_dofs, c->d_sign, c->d_dir, c->d_fcell, c->d_flf, c->d_ftau, c->d_fcw, c->d_fjw,
                   c->d_rowptr, c->d_colind, c->d_rank, c->d_val, c->d_tperm, c->d_ref, c->d_fref, c->d_x, c->d_r,
                   c->d_color_cells, c->d_crow, c->d_centry, c->d_ebuf, c->d_rbuf, c->d_skel_dofs, c->d_skel_K,
-                  c->d_srow, c->d_sentry, c->d_skel_rank, c->d_skel_res};
+                  c->d_srow, c->d_sentry, c->d_skel_rank, c->d_skel_res, c->d_gslot, c->d_minv, c->d_state, c->d_cfptr,
+                  c->d_cface, c->d_fK, c->d_fc};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);

@@ -354,76 +354,6 @@ __device__ double jac_entry(const CellLDS &S, const RefTables *__restrict__ T, c
   return acc;
 }
 
-// Residual entry of test function a.
-// mode 0: residual; mode 1: dR/dgamma = -int (j x B).v (u rows only)
-__device__ double res_entry(const CellLDS &S, const RefTables *__restrict__ T, const MhdPhys &ph, int a, int mode) {
-  double acc = 0.0;
-  if (mode == 1) {
-    if (a >= OFF_P) return 0.0;
-    const int ca = a / 27, na = a % 27;
-    const int i1 = ca == 2 ? 0 : ca + 1, i2 = ca == 0 ? 2 : ca - 1;
-#pragma unroll 1
-    for (int q = 0; q < NQ; ++q)
-      acc -= S.W[q] * (S.jv[q][i1] * S.B[i2] - S.jv[q][i2] * S.B[i1]) * S.q2[q][na];
-    return acc;
-  }
-  if (a < OFF_P) {
-    const int ca = a / 27, na = a % 27;
-#pragma unroll 1
-    for (int q = 0; q < NQ; ++q) {
-      const double *gv = S.gphi[q][na];
-      const double phv = S.q2[q][na];
-      // beta grad u : grad v with v = phi e_ca -> sum_i gu[i][ca] dphi_i
-      double t = ph.beta * (S.gu[q][0 * 3 + ca] * gv[0] + S.gu[q][1 * 3 + ca] * gv[1] + S.gu[q][2 * 3 + ca] * gv[2]);
-      if (ph.convection) {
-        // ((grad u)^T u)_ca = sum_i gu[i][ca] u_i
-        const double cv = S.gu[q][0 * 3 + ca] * S.u[q][0] + S.gu[q][1 * 3 + ca] * S.u[q][1] + S.gu[q][2 * 3 + ca] * S.u[q][2];
-        t += ph.alpha * phv * cv;
-      }
-      t -= S.p[q] * gv[ca];
-      const int i1 = ca == 2 ? 0 : ca + 1, i2 = ca == 0 ? 2 : ca - 1;
-      const double jxb = S.jv[q][i1] * S.B[i2] - S.jv[q][i2] * S.B[i1];  // (j x B)_ca
-      t -= ph.gamma * jxb * phv;
-      double f = S.f0[ca];
-      for (int k = 0; k < 3; ++k) f += S.fx[3 * ca + k] * S.xq[q][k];
-      t -= f * phv;
-      acc += S.W[q] * t;
-    }
-    if (ph.zeta_u != 0.0) {
-      double al = 0.0;
-      for (int k = 0; k < 4; ++k) al += S.D[k][a] * S.cu[k];
-      acc += ph.zeta_u * al;
-    }
-  } else if (a < OFF_J) {
-    const int k = a - OFF_P;
-#pragma unroll 1
-    for (int q = 0; q < NQ; ++q) acc -= S.W[q] * S.divu[q] * S.p1[q][k];
-  } else if (a < OFF_PHI) {
-    const int r = a - OFF_J;
-#pragma unroll 1
-    for (int q = 0; q < NQ; ++q) {
-      const double *s = S.psi[q][r];
-      double t = 0.0;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const int i1 = i == 2 ? 0 : i + 1, i2 = i == 0 ? 2 : i - 1;
-        const double uxb = S.u[q][i1] * S.B[i2] - S.u[q][i2] * S.B[i1];
-        double g = S.g0[i];
-        for (int k = 0; k < 3; ++k) g += S.gx[3 * i + k] * S.xq[q][k];
-        t += (S.jv[q][i] - ph.sigma * uxb - g) * s[i];
-      }
-      t -= ph.sigma * S.ph[q] * S.dpsi[q][r];
-      if (ph.zeta_j != 0.0) t += ph.zeta_j * S.divj[q] * S.dpsi[q][r];
-      acc += S.W[q] * t;
-    }
-  } else {
-    const int v = a - OFF_PHI;
-#pragma unroll 1
-    for (int q = 0; q < NQ; ++q) acc -= S.W[q] * S.divj[q] * S.q1[q][v];
-  }
-  return acc;
-}
-
 typedef double d4_t __attribute__((ext_vector_type(4)));
 
 // How a cell's Jacobian entries leave the kernel:
@@ -631,34 +561,6 @@ __global__ __launch_bounds__(WG, 2) void k_cell_jacobian(int ncells, const int32
   }
 }
 
-// Element residuals into rbuf[cell][NDOF] (free rows only); k_res_gather
-// then sums them per dof, so the residual does not depend on the order in
-// which the cells finish.
-__global__ __launch_bounds__(WG, 2) void k_cell_residual(int ncells, const double *__restrict__ xyz,
-                                                      const int32_t *__restrict__ dofs, const int8_t *__restrict__ sign,
-                                                      const double *__restrict__ dir, const double *__restrict__ x,
-                                                      const RefTables *__restrict__ T, double *__restrict__ rbuf,
-                                                      MhdPhys ph, int mode) {
-  __shared__ CellLDS S;
-  for (int c = blockIdx.x; c < ncells; c += gridDim.x) {
-    stage_cell(S, c, xyz, dofs, sign, dir, x, T, nullptr, ph, ph.zeta_u != 0.0);
-    const int a = threadIdx.x;
-    if (a < NDOF && S.g[a] >= 0) rbuf[(int64_t)c * NDOF + a] = res_entry(S, T, ph, a, mode);
-    __syncthreads();
-  }
-}
-
-// r[i] = sum of the element residual rows holding dof i, in increasing cell
-// order (the holder lists of the row assembly)
-__global__ void k_res_gather(int64_t n, const int32_t *__restrict__ crow, const int32_t *__restrict__ centry,
-                             const double *__restrict__ rbuf, double *__restrict__ r) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = 0.0;
-  for (int32_t h = crow[i]; h < crow[i + 1]; ++h) s += rbuf[centry[h]];
-  r[i] = s;
-}
-
 // Per-cell integrals of the state (post-processing, src/Applications/hunt.jl:247-260):
 // out[c] = (int u.u, int grad u : grad u, int j.j, int (div j)^2, int p, |K|).  The 3x3x3
 // Gauss rule integrates these polynomial quantities exactly on affine cells.
@@ -815,67 +717,90 @@ __device__ void stage_face(FaceLDS &S, int f, const double *__restrict__ xyz, co
   __syncthreads();
 }
 
-__global__ __launch_bounds__(64) void k_face_residual(int nfaces, const double *__restrict__ xyz,
-                                                      const int32_t *__restrict__ dofs, const int8_t *__restrict__ sign,
-                                                      const double *__restrict__ dir, const double *__restrict__ x,
-                                                      const FaceTables *__restrict__ F, const int32_t *__restrict__ fcell,
-                                                      const int8_t *__restrict__ flf, const double *__restrict__ ftau,
-                                                      const double *__restrict__ fcw, const double *__restrict__ fjw,
-                                                      double *__restrict__ r, int mode) {
+// dR/dcw of a face: sum_q W tau (s.n) n.(grad j).n
+__global__ __launch_bounds__(64) void k_face_dcw(int nfaces, const double *__restrict__ xyz,
+                                                 const int32_t *__restrict__ dofs, const int8_t *__restrict__ sign,
+                                                 const double *__restrict__ dir, const double *__restrict__ x,
+                                                 const FaceTables *__restrict__ F, const int32_t *__restrict__ fcell,
+                                                 const int8_t *__restrict__ flf, const double *__restrict__ ftau,
+                                                 double *__restrict__ r) {
   __shared__ FaceLDS S;
   for (int f = blockIdx.x; f < nfaces; f += gridDim.x) {
     int cell, lf;
     stage_face(S, f, xyz, dofs, sign, dir, x, F, fcell, flf, nullptr, cell, lf);
     const int a = 4 * lf + threadIdx.x;
     if (threadIdx.x < 4 && S.g[a] >= 0) {
-      const double tau = ftau[f], cw = fcw[f], jw = fjw[f];
+      const double tau = ftau[f];
       const int d = 2 - lf / 2;
       const double sgn = sign ? (double)sign[(int64_t)cell * 6 + lf] : 1.0;
       double acc = 0.0;
-      for (int q = 0; q < NQF; ++q) {
-        const double sn = sgn * F->rt[lf][q][a][d] * S.ndn[q];
-        acc += mode == 2 ? S.W[q] * tau * sn * S.jnn[q] : S.W[q] * tau * sn * (S.jn[q] - jw + cw * S.jnn[q]);
-      }
+      for (int q = 0; q < NQF; ++q) acc += S.W[q] * tau * (sgn * F->rt[lf][q][a][d] * S.ndn[q]) * S.jnn[q];
       atomicAdd(&r[S.g[a]], acc);
     }
     __syncthreads();
   }
 }
 
-__global__ __launch_bounds__(64) void k_face_jacobian(int nfaces, const double *__restrict__ xyz,
-                                                      const int32_t *__restrict__ dofs, const int8_t *__restrict__ sign,
-                                                      const double *__restrict__ dir, const double *__restrict__ x,
-                                                      const FaceTables *__restrict__ F, const int32_t *__restrict__ fcell,
-                                                      const int8_t *__restrict__ flf, const double *__restrict__ ftau,
-                                                      const double *__restrict__ fcw, const int64_t *__restrict__ rowptr,
-                                                      const uint16_t *__restrict__ rank, double *__restrict__ val) {
+// Face matrices K[a][b] = sum_q W tau (s_a.n)(s_b.n + cw n.(grad s_b).n) of the
+// face's four own test functions and the cell's 36 current dofs, and constant
+// parts -jw sum_q W tau (s_a.n), without the orientation signs: the term is
+// linear and depends on the geometry and the face's parameters only, so they
+// are computed once per context (1.2 KB per face).
+__global__ __launch_bounds__(64) void k_face_matrix(int nfaces, const double *__restrict__ xyz,
+                                                    const int32_t *__restrict__ dofs, const double *__restrict__ dir,
+                                                    const double *__restrict__ x, const FaceTables *__restrict__ F,
+                                                    const int32_t *__restrict__ fcell, const int8_t *__restrict__ flf,
+                                                    const double *__restrict__ ftau, const double *__restrict__ fcw,
+                                                    const double *__restrict__ fjw, double *__restrict__ K,
+                                                    double *__restrict__ cst) {
   __shared__ FaceLDS S;
   for (int f = blockIdx.x; f < nfaces; f += gridDim.x) {
     int cell, lf;
-    stage_face(S, f, xyz, dofs, sign, dir, x, F, fcell, flf, rowptr, cell, lf);
-    const double tau = ftau[f], cw = fcw[f];
-    const uint16_t *rk = rank + (int64_t)cell * NENT;
+    stage_face(S, f, xyz, dofs, nullptr, dir, x, F, fcell, flf, nullptr, cell, lf);
+    const double tau = ftau[f], cw = fcw[f], jw = fjw[f];
     const int dax = 2 - lf / 2;
-    const double sgn = sign ? (double)sign[(int64_t)cell * 6 + lf] : 1.0;
     for (int idx = threadIdx.x; idx < 4 * NJ; idx += blockDim.x) {
       const int a = 4 * lf + idx / NJ, b = idx % NJ;
-      if (S.g[a] < 0 || S.g[b] < 0) continue;
       const bool bface = (b >> 2) == lf;
-      double acc = 0.0;
+      double acc = 0.0, one = 0.0;
       for (int q = 0; q < NQF; ++q) {
         const double *n = S.n[q], *gd = S.gpsi[q][b];
-        const double sn = sgn * F->rt[lf][q][a][dax] * S.ndn[q];
-        const double dn = bface ? sgn * F->rt[lf][q][b][dax] * S.ndn[q] : 0.0;
+        const double sn = F->rt[lf][q][a][dax] * S.ndn[q];
+        const double dn = bface ? F->rt[lf][q][b][dax] * S.ndn[q] : 0.0;
         double dnn = 0.0;
         for (int i = 0; i < 3; ++i) dnn += n[i] * (gd[3 * i + 0] * n[0] + gd[3 * i + 1] * n[1] + gd[3 * i + 2] * n[2]);
         acc += S.W[q] * tau * sn * (dn + cw * dnn);
+        one += S.W[q] * tau * sn;
       }
-      // jj block entry of j row a, j column b inside the cell's rank map
-      const int e = E_J + a * ROWS_J_LEN + NU + b;
-      atomicAdd(&val[S.rp[a] + rk[e]], acc);
+      K[(int64_t)f * 4 * NJ + idx] = acc;
+      if (b == 0) cst[4 * (int64_t)f + idx / NJ] = -jw * one;
     }
     __syncthreads();
   }
+}
+
+// The faces' Jacobian entries, added to the assembled values: one thread per
+// entry of the face matrix.  (Recomputing the matrices at every Jacobian took
+// 20 us on 96 faces and 46 us on 2,048, all latency; this takes 3 to 4 us.)
+__global__ __launch_bounds__(256) void k_face_jacobian(int nfaces, const int32_t *__restrict__ dofs,
+                                                       const int8_t *__restrict__ sign,
+                                                       const int32_t *__restrict__ fcell,
+                                                       const int8_t *__restrict__ flf, const double *__restrict__ K,
+                                                       const int64_t *__restrict__ rowptr,
+                                                       const uint16_t *__restrict__ rank, double *__restrict__ val) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t >= (int64_t)nfaces * 4 * NJ) return;
+  const int f = (int)(t / (4 * NJ)), idx = (int)(t % (4 * NJ));
+  const int cell = fcell[f], lf = flf[f], a = 4 * lf + idx / NJ, b = idx % NJ;
+  const int32_t ga = dofs[(int64_t)cell * NDOF + OFF_J + a], gb = dofs[(int64_t)cell * NDOF + OFF_J + b];
+  if (ga < 0 || gb < 0) return;
+  double v = K[t];
+  if (sign) {
+    v *= (double)sign[(int64_t)cell * 6 + lf];
+    if (b < 24) v *= (double)sign[(int64_t)cell * 6 + (b >> 2)];
+  }
+  // jj block entry of j row a, j column b inside the cell's rank map
+  atomicAdd(&val[rowptr[ga] + rank[(int64_t)cell * NENT + E_J + a * ROWS_J_LEN + NU + b]], v);
 }
 
 // Canonical entry range [start, start + len) of local row a of a cell.
@@ -1268,9 +1193,9 @@ int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_
     }
   }
   if (c->nfaces > 0) {
-    hipLaunchKernelGGL(k_face_jacobian, dim3(c->nfaces), dim3(64), 0, s, c->nfaces, c->d_xyz, c->d_dofs, c->d_sign,
-                       c->d_dir, d_x, c->d_fref, c->d_fcell, c->d_flf, c->d_ftau, c->d_fcw, c->d_rowptr, c->d_rank,
-                       d_val);
+    const int64_t ne = (int64_t)c->nfaces * 4 * NJ;
+    hipLaunchKernelGGL(k_face_jacobian, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s, c->nfaces, c->d_dofs,
+                       c->d_sign, c->d_fcell, c->d_flf, c->d_fK, c->d_rowptr, c->d_rank, d_val);
     MHD_HIP(hipGetLastError());
   }
   return mhd_launch_skeleton_jacobian(c, d_val, s);
@@ -1319,22 +1244,33 @@ int mhd_launch_skeleton_jacobian(mhd_ctx *c, double *d_val, hipStream_t s) {
   return 0;
 }
 
+int mhd_build_face_matrices(mhd_ctx *c) {
+  const size_t nf = (size_t)std::max(c->nfaces, 1);
+  MHD_HIP(hipMalloc(&c->d_fK, sizeof(double) * nf * 4 * NJ));
+  MHD_HIP(hipMalloc(&c->d_fc, sizeof(double) * nf * 4));
+  if (c->nfaces <= 0) return 0;
+  // the state that the staging reads plays no part in the matrices
+  MHD_HIP(hipMemsetAsync(c->d_x, 0, sizeof(double) * std::max<int64_t>(c->n, 1), c->stream));
+  hipLaunchKernelGGL(k_face_matrix, dim3((unsigned)std::min(c->nfaces, 1 << 20)), dim3(64), 0, c->stream, c->nfaces,
+                     c->d_xyz, c->d_dofs, c->d_dir, c->d_x, c->d_fref, c->d_fcell, c->d_flf, c->d_ftau, c->d_fcw,
+                     c->d_fjw, c->d_fK, c->d_fc);
+  MHD_HIP(hipGetLastError());
+  return 0;
+}
+
+// mode 0: residual; 1: dR/dgamma; 2: dR/dcw
 int mhd_launch_residual_mode(mhd_ctx *c, const double *d_x, double *d_r, hipStream_t s, int mode) {
-  if (c->ncells > 0 && mode != 2) {
-    if (!c->d_rbuf) MHD_HIP(hipMalloc(&c->d_rbuf, sizeof(double) * (size_t)c->ncells * NDOF));
-    hipLaunchKernelGGL(k_cell_residual, dim3(c->ncells), dim3(WG), 0, s, c->ncells, c->d_xyz, c->d_dofs, c->d_sign,
-                       c->d_dir, d_x, c->d_ref, c->d_rbuf, c->phys, mode);
-    hipLaunchKernelGGL(k_res_gather, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, s, c->n, c->d_crow,
-                       c->d_centry, c->d_rbuf, d_r);
-    MHD_HIP(hipGetLastError());
-  } else {
+  if (mode == 2) {
     MHD_HIP(hipMemsetAsync(d_r, 0, sizeof(double) * c->n, s));
-  }
-  if (c->nfaces > 0 && mode != 1) {
-    hipLaunchKernelGGL(k_face_residual, dim3(c->nfaces), dim3(64), 0, s, c->nfaces, c->d_xyz, c->d_dofs, c->d_sign,
-                       c->d_dir, d_x, c->d_fref, c->d_fcell, c->d_flf, c->d_ftau, c->d_fcw, c->d_fjw, d_r, mode);
+    if (c->nfaces > 0)
+      hipLaunchKernelGGL(k_face_dcw, dim3(c->nfaces), dim3(64), 0, s, c->nfaces, c->d_xyz, c->d_dofs, c->d_sign,
+                         c->d_dir, d_x, c->d_fref, c->d_fcell, c->d_flf, c->d_ftau, d_r);
     MHD_HIP(hipGetLastError());
+    return 0;
   }
+  if (!c->d_rbuf) MHD_HIP(hipMalloc(&c->d_rbuf, sizeof(double) * (size_t)c->ncells * NDOF));
+  int rc = mhd_cellop_residual(c, d_x, d_r, c->d_rbuf, mode, s);
+  if (rc) return rc;
   // the skeleton term depends on neither gamma nor cw (modes 1, 2: dR/dtheta)
   return mode == 0 ? mhd_launch_skeleton_residual(c, d_x, d_r, s) : 0;
 }
@@ -1351,8 +1287,8 @@ int mhd_launch_residual(mhd_ctx *c, const double *d_x, double *d_r, hipStream_t 
 // symbol): the device address of each GPU's copy is looked up once per device
 // with hipGetSymbolAddress while that device is current, and that pointer is
 // what the launches take.  Every call on one GPU shares that GPU's copy, so
-// calls that overlap on one GPU race.  k_cell_residual writes every element
-// residual entry that k_res_gather reads, so nothing is cleared between calls.
+// calls that overlap on one GPU race.  The cell kernel writes every element
+// residual that the gather reads, so nothing is cleared between calls.
 
 namespace {
 constexpr int64_t NOALLOC_DOUBLES = int64_t(1) << 24;
@@ -1360,11 +1296,6 @@ constexpr int NOALLOC_MAX_DEVICES = 64;
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 std::mutex g_scratch_mu;
 double *g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
-
-__global__ void k_fill(int64_t n, double v, double *__restrict__ y) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    y[i] = v;
-}
 }  // namespace
 
 int mhd_noalloc_init(mhd_ctx *c) {
@@ -1392,21 +1323,8 @@ int mhd_launch_residual_noalloc(mhd_ctx *c, const double *d_x, double *d_r, hipS
     c->err = "mhd_residual_d_noalloc: workspace address not set up for this device";
     return -2;
   }
-  if (c->ncells > 0) {
-    hipLaunchKernelGGL(k_cell_residual, dim3(c->ncells), dim3(WG), 0, s, c->ncells, c->d_xyz, c->d_dofs, c->d_sign,
-                       c->d_dir, d_x, c->d_ref, c->d_scratch, c->phys, 0);
-    hipLaunchKernelGGL(k_res_gather, dim3((unsigned)((c->n + 255) / 256)), dim3(256), 0, s, c->n, c->d_crow,
-                       c->d_centry, c->d_scratch, d_r);
-  } else if (c->n > 0) {
-    hipLaunchKernelGGL(k_fill, dim3((unsigned)std::min<int64_t>((c->n + 255) / 256, 65536)), dim3(256), 0, s, c->n,
-                       0.0, d_r);
-  }
-  MHD_HIP(hipGetLastError());
-  if (c->nfaces > 0) {
-    hipLaunchKernelGGL(k_face_residual, dim3(c->nfaces), dim3(64), 0, s, c->nfaces, c->d_xyz, c->d_dofs, c->d_sign,
-                       c->d_dir, d_x, c->d_fref, c->d_fcell, c->d_flf, c->d_ftau, c->d_fcw, c->d_fjw, d_r, 0);
-    MHD_HIP(hipGetLastError());
-  }
+  int rc = mhd_cellop_residual(c, d_x, d_r, c->d_scratch, 0, s);
+  if (rc) return rc;
   // the skeleton face matrices and face products are context memory made at creation
   return mhd_launch_skeleton_residual(c, d_x, d_r, s);
 }

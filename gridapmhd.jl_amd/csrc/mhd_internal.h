@@ -121,9 +121,17 @@ struct mhd_ctx {
   // row assembly: the (cell * NDOF + local row) pairs holding each free dof
   int32_t *d_crow = nullptr;          // [n + 1]
   int32_t *d_centry = nullptr;        // [crow[n]], increasing cell order per row
+  int64_t nhold = 0;                  // crow[n]
   int32_t max_row = 0;                // longest CSR row
   double *d_ebuf = nullptr;           // [ncells][NENT] element buffer (allocated on first use)
-  double *d_rbuf = nullptr;           // [ncells][NDOF] element residuals (allocated on first use)
+  double *d_rbuf = nullptr;           // [ncells][NDOF] element results (allocated on first use)
+  // cell-wise application of the form (mhd_cellop.hip)
+  int32_t *d_gslot = nullptr;         // [crow[n]] element-result slots of every dof's holders
+  double *d_minv = nullptr;           // [ncells][16] inverse dP1 mass matrices
+  double *d_state = nullptr;          // [ncells][12][27] u0, grad u0 of the products' linearisation point
+  int32_t *d_cfptr = nullptr, *d_cface = nullptr;  // thin-wall faces of every cell
+  double *d_fK = nullptr;             // [nfaces][4][36] thin-wall face matrices (without orientation signs)
+  double *d_fc = nullptr;             // [nfaces][4] their constant parts (-jw)
   double *d_scratch = nullptr;        // this device's allocation-free residual workspace (not owned)
   // skeleton stabilisation (mhd_create_stabilized)
   int32_t nskel = 0;
@@ -178,7 +186,20 @@ enum {
 };
 void mhd_solver_free(mhd_ctx *c);
 
+// Cell-wise application (mhd_cellop.hip).  The products use the state of the
+// last mhd_cellop_state and the context's parameters: y = A x, or y = v - A x
+// (v not null), on all rows (MHD_OP_FULL), of the [u,j] block (MHD_OP_UJ) or of
+// the (u,j) rows' p and phi columns (MHD_OP_PPHI); `trans`: of D^-1 A^T D with
+// D = scale on the j and phi dofs.  No skeleton term.
+enum { MHD_OP_FULL = 1, MHD_OP_UJ = 2, MHD_OP_PPHI = 3 };
+int mhd_cellop_build(mhd_ctx *c);
+int mhd_cellop_residual(mhd_ctx *c, const double *d_x, double *d_r, double *buf, int mode, hipStream_t s);
+int mhd_cellop_state(mhd_ctx *c, const double *d_x, hipStream_t s);
+template <class T>
+int mhd_cellop_apply(mhd_ctx *c, int op, bool trans, double scale, const T *x, const T *v, T *y, hipStream_t s);
+
 // Launchers (mhd_assembly.hip)
+int mhd_build_face_matrices(mhd_ctx *c);
 int mhd_launch_residual(mhd_ctx *c, const double *d_x, double *d_r, hipStream_t s);
 int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_t s);
 int mhd_build_rank_map(mhd_ctx *c);
