@@ -1436,6 +1436,9 @@ struct Solver {
   int64_t nnz11 = 0, nnz1x = 0;
   double pent = 0.0, pcube = 0.0;
   double ops[MHD_NOPS] = {};
+  // products without the matrix (mhd_cellop_apply); with a skeleton term they
+  // stream it instead, through the row groups below
+  bool matfree = true;
   // row groups sharing a column list (k_spmv_grp): all rows, and the first
   // ngroups11 groups cover the [u,j] rows exactly
   int64_t ngroups = 0, ngroups11 = 0;
@@ -1454,6 +1457,9 @@ double adjoint_scale(const mhd_ctx *c) {
   const double g = c->phys.gamma, sg = c->phys.sigma;
   return (g > 0.0 && sg > 0.0) ? g / sg : 1.0;
 }
+
+// the scaling of the products: of the transposed ones only
+double op_scale(const mhd_ctx *c) { return c->solver->transposed ? adjoint_scale(c) : 1.0; }
 
 // FGMRES Krylov dimension for a requested restart length
 int krylov_dim(int restart) { return std::max(2, std::min(restart, 2000)); }
@@ -1626,7 +1632,8 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
     S->nnz11 += k;
     S->nnz1x += (e - b) - k;
   }
-  {
+  S->matfree = c->nskel == 0;
+  if (!S->matfree) {
     // runs of consecutive rows with one column list (at most GMAX rows; no run
     // crosses the end of the [u,j] rows)
     std::vector<int64_t> grow, gcp;
@@ -1781,7 +1788,8 @@ int inner_alloc(mhd_ctx *c, int prec) {
   MHD_HIP(hipMalloc(&S->w1, es * n1 + es));
   MHD_HIP(hipMalloc(&S->x1, es * n1 + es));
   MHD_HIP(hipMalloc(&S->r1, es * n1 + es));
-  if (prec >= 1 && !S->d_val32) MHD_HIP(hipMalloc(&S->d_val32, sizeof(float) * std::max<int64_t>(c->nnz, 1)));
+  if (prec >= 1 && !S->matfree && !S->d_val32)
+    MHD_HIP(hipMalloc(&S->d_val32, sizeof(float) * std::max<int64_t>(c->nnz, 1)));
   {
     const size_t ms = prec == 0 ? sizeof(double) : prec == 1 ? sizeof(float) : 2;  // bytes of an inverse's entry
     const int vec = 16 / (int)ms;
@@ -1942,11 +1950,20 @@ int patch_as(mhd_ctx *c, const T *r, T *y, int prec, double w = 1.0, bool accumu
   return patch_as_on<T>(c, r, y, prec, w, accumulate, c->stream);
 }
 
-// y = A11 x (MODE 1) or y = v - A11 x (MODE 3) on the [u,j] rows, FP64 values
-// for precision 0 and the FP32 copy otherwise, through the row groups
+// y = A11 x (MODE 1) or y = v - A11 x (MODE 3) on the [u,j] rows.  Without a
+// skeleton term the form is applied cell by cell: a product reads 0.15 GB at
+// 64 x 64 x 8 where the matrix has 1.7 GB (FP32) or 3.0 GB (FP64).  With one,
+// the matrix is streamed through the row groups, FP64 values for precision 0
+// and the FP32 copy otherwise (the face matrices of the skeleton term alone are
+// as large as the FP32 matrix).
 template <class T, int MODE>
 int a11_product(mhd_ctx *c, const T *x, const T *v, T *y, int prec) {
   Solver *S = c->solver;
+  if (S->matfree) {
+    count(c, prec == 0 ? OP_SPMV64 : OP_SPMV32, (double)S->nnz11);
+    return mhd_cellop_apply<T>(c, MHD_OP_UJ, S->transposed, op_scale(c), x, MODE == 3 ? v : (const T *)nullptr, y,
+                               c->stream);
+  }
   constexpr int LPG = 16;
   const int grid = (int)((S->ngroups11 * LPG + 255) / 256);
   if (prec == 0)
@@ -1960,9 +1977,14 @@ int a11_product(mhd_ctx *c, const T *x, const T *v, T *y, int prec) {
   return 0;
 }
 
-// y = J x with the full FP64 Jacobian of the context, through the row groups
+// y = J x with the full FP64 Jacobian of the context, the same two ways
 int full_product(mhd_ctx *c, const double *x, double *y) {
   Solver *S = c->solver;
+  if (S->matfree) {
+    count(c, OP_SPMV64, (double)c->nnz);
+    return mhd_cellop_apply<double>(c, MHD_OP_FULL, S->transposed, op_scale(c), x, (const double *)nullptr, y,
+                                    c->stream);
+  }
   constexpr int LPG = 16;
   const int grid = (int)((S->ngroups * LPG + 255) / 256);
   hipLaunchKernelGGL((k_spmv_grp<double, double, double, LPG, 0>), dim3(grid), dim3(256), 0, c->stream, S->ngroups,
@@ -2119,19 +2141,20 @@ int precond(mhd_ctx *c, const double *v, double *z, int prec) {
   hipLaunchKernelGGL((k_schur<double>), dim3(nblocks((int64_t)c->ncells * 12)), dim3(TB), 0, c->stream, c->ncells,
                      S->d_pfirst, S->d_phifirst, S->d_Sp, S->d_Sphi, v, z);
   // rhs1 = v1 - A12 z_p - A13 z_phi (FP64)
-  constexpr int LPR = 16;
-  const int grid = (int)((S->n1 * LPR + 255) / 256);
-  if (prec == 0) {
-    hipLaunchKernelGGL((k_spmv_seg<double, double, double, LPR, 2>), dim3(grid), dim3(256), 0, c->stream, S->n1,
-                       c->d_rowptr, S->d_split, c->d_colind, c->d_val, z, v, (double *)S->r1);
-    count(c, OP_SPMV64, (double)S->nnz1x);
+  double *rhs1 = prec == 0 ? (double *)S->r1 : S->t1;
+  count(c, OP_SPMV64, (double)S->nnz1x);
+  if (S->matfree) {
+    if ((rc = mhd_cellop_apply<double>(c, MHD_OP_PPHI, S->transposed, op_scale(c), z, v, rhs1, c->stream))) return rc;
+  } else {
+    constexpr int LPR = 16;
+    hipLaunchKernelGGL((k_spmv_seg<double, double, double, LPR, 2>), dim3((unsigned)((S->n1 * LPR + 255) / 256)),
+                       dim3(256), 0, c->stream, S->n1, c->d_rowptr, S->d_split, c->d_colind, c->d_val, z, v, rhs1);
     MHD_HIP(hipGetLastError());
+  }
+  if (prec == 0) {
     if ((rc = inner_solve<double>(c, 0))) return rc;
     MHD_HIP(hipMemcpyAsync(z, S->x1, sizeof(double) * S->n1, hipMemcpyDeviceToDevice, c->stream));
   } else {
-    hipLaunchKernelGGL((k_spmv_seg<double, double, double, LPR, 2>), dim3(grid), dim3(256), 0, c->stream, S->n1,
-                       c->d_rowptr, S->d_split, c->d_colind, c->d_val, z, v, S->t1);
-    count(c, OP_SPMV64, (double)S->nnz1x);
     hipLaunchKernelGGL((k_convert<double, float>), dim3(nblocks(S->n1)), dim3(TB), 0, c->stream, S->n1, S->t1,
                        (float *)S->r1);
     MHD_HIP(hipGetLastError());
@@ -2286,7 +2309,9 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     S->alpha_p = ap;
     S->alpha_phi = aphi;
   }
-  if (prec >= 1)
+  if (S->matfree) {
+    if ((rc = mhd_cellop_state(c, d_state, c->stream))) return rc;
+  } else if (prec >= 1)
     hipLaunchKernelGGL((k_convert<double, float>), dim3(nblocks(c->nnz)), dim3(TB), 0, c->stream, c->nnz, c->d_val,
                        S->d_val32);
   if ((rc = invert_patches(c, prec))) return rc;

@@ -275,8 +275,9 @@ int mhd_smoother_info(mhd_ctx *ctx, int64_t *npatch, int64_t *patch_dim, int64_t
  * context and its coarse levels.  No counterpart in the reference: a
  * measurement aid that lets other hardware be priced on exactly the work of a
  * solve (the CPU Newton-step baseline).  out[MHD_NOPS]:
- *   0  nonzeros streamed by SpMVs with FP64 values (A, the A11 / A1x blocks, P, P^T)
- *   1  nonzeros streamed by SpMVs with FP32 values
+ *   0  nonzeros of the matrix products with FP64 vectors (A, the A11 / A1x
+ *      blocks, P, P^T), whether the matrix is streamed or the form applied
+ *   1  ... with FP32 vectors
  *   2  patch-inverse entries (and entries of the cells' condensation couplings)
  *      applied by the smoother in FP64
  *   3  ... in FP32

@@ -1,0 +1,40 @@
+"""The Jacobian products that the Krylov solves use (the form applied cell by
+cell; with a skeleton term, the matrix) against the oracle's Jacobian: a
+linear solve with A(x), or with its transpose, to a relative residual of 1e-11
+must satisfy the oracle's system to the same residual.  Odd cell counts (the
+last workgroup holds one cell), non-affine cells, every convection form, a
+state with all fields, the [u,j] V-cycle's products in both precisions."""
+import numpy as np
+import pytest
+
+import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nc,convection,stab,levels", [((3, 3, 3), "newton", 0.0, 1), ((3, 2, 3), "picard", 0.0, 1),
+                                                       ((5, 3, 1), "none", 0.0, 1), ((8, 8, 3), "newton", 0.0, 2),
+                                                       ((3, 3, 3), "newton", 0.1, 1)])
+def test_linear_solves_satisfy_the_oracle_system(nc, convection, stab, levels, precision, orc_mod):
+    import gridapmhd_amd as g
+    from gridapmhd_amd import adjoint
+    sp, phys = adjoint.inlet_duct(nc, 20.0, 5.0, 0.05, convection=convection, jitter=0.15 if levels == 1 else 0.0)
+    phys = dict(phys, stab_mu=stab, f0=np.array([0.2, -0.1, 1.0]))
+    rng = np.random.default_rng(4)
+    x = 0.1 * rng.standard_normal(sp.ndofs)
+    rhs = rng.standard_normal(sp.ndofs)
+    A = orc_mod.Oracle(cases.problem_dict(sp, phys)).jacobian(x).tocsr()
+    ctx = g._lib.context_with_levels(sp, phys, levels=levels)
+    try:
+        o = ctx.default_opts(precision=precision, ls_rtol=1e-11, max_krylov=600, restart=600, inner_iters=4)
+        for name, solve, M in (("A", ctx.linear_solve, A), ("A^T", ctx.adjoint_solve, A.T.tocsr())):
+            s, info, rc = solve(x, rhs, o)
+            res = np.linalg.norm(M @ s - rhs) / np.linalg.norm(rhs)
+            print(f"[products] {nc} {convection} stab={stab} precision={precision} {name}: {info.krylov_iters} "
+                  f"iterations, residual {res:.2e}", flush=True)
+            assert rc == 0
+            # the adjoint solve measures its residual in rows scaled by up to gamma / sigma = Ha^2 / Re = 80
+            assert res < 1e-9
+    finally:
+        ctx.close()
