@@ -162,9 +162,15 @@ struct CoarseLink {
   double *d_Rval = nullptr;
   int64_t nnzP = 0;                // nonzeros of P (and of P^T)
   int coarse_iters = 10;           // Schwarz-GMRES steps on the coarsest level; 0: dense inverse
-  // coarsest level solved exactly: explicit inverse of its [u,j] block (row-major)
-  double *d_Ainv = nullptr;        // [n1c][n1c]
-  double *d_LU = nullptr;          // [n1c][n1c] LU factors (set-up scratch)
+  // coarsest level solved exactly: explicit inverse (row-major) of its [u,j]
+  // block with the cells' interior current dofs condensed out
+  int64_t nb = 0;                  // dofs that are not eliminated
+  int32_t *d_bidx = nullptr, *d_bmap = nullptr;  // [nb] their ids, [n1c] the inverse (-1)
+  int32_t *d_ones = nullptr;       // [ncells of the level]
+  double *d_cF = nullptr, *d_cG = nullptr;       // A_bi D^-1, D^-1 of every cell
+  double *d_rb = nullptr, *d_yb = nullptr;       // [nb] condensed rhs, [n1c] the other dofs' results
+  double *d_Ainv = nullptr;        // [nb][nb]
+  double *d_LU = nullptr;          // [nb][nb] the condensed block, then its LU factors (set-up scratch)
   int32_t *d_piv = nullptr, *d_info = nullptr;
   double *d_gjw = nullptr;         // block Gauss-Jordan workspace (column and row panels, pivot block, check)
   int32_t *d_gjflag = nullptr;     // set when a diagonal block of the block Gauss-Jordan has a zero pivot

@@ -288,18 +288,10 @@ __global__ void k_set_diag(int64_t n, double v, double *__restrict__ D) {
     D[i + i * n] = v;
 }
 
-// dense row-major copy of the [u,j] block (the A11 prefix of each row)
-__global__ void k_dense_a11(int64_t n1, const int64_t *__restrict__ rowptr, const int64_t *__restrict__ split,
-                            const int32_t *__restrict__ colind, const double *__restrict__ val,
-                            double *__restrict__ D) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n1; i += (int64_t)gridDim.x * blockDim.x)
-    for (int64_t p = rowptr[i]; p < split[i]; ++p) D[i * n1 + colind[p]] = val[p];
-}
-
 // ---------------------------------------------------------------------------
-// Dense inverse of the coarsest [u,j] block by block Gauss-Jordan: for each
-// block column K of width BGJ_B, P = A_KK^-1 (one workgroup, Gauss-Jordan with
-// partial pivoting inside the block), then the rank-BGJ_B update
+// Dense inverse of the condensed coarsest [u,j] block by block Gauss-Jordan: for
+// each block column K of width BGJ_B, P = A_KK^-1 (one workgroup, pivoting
+// inside its 32 x 32 diagonal blocks), then the rank-BGJ_B update
 //   A <- A - A[:,K] P A[K,:],  A[K,:] <- P A[K,:],  A[:,K] <- -A[:,K] P,  A_KK <- P
 // on FP64 GEMMs (2 n^3 flops in all, like an LU plus triangular solves, but in
 // n / BGJ_B wide GEMM steps instead of one panel kernel per column).  Pivoting
@@ -307,96 +299,143 @@ __global__ void k_dense_a11(int64_t n1, const int64_t *__restrict__ rowptr, cons
 // redone with the row-pivoted LU if it fails.
 constexpr int BGJ_B = 96;
 
-// One 1024-thread workgroup inverts the kb x kb (kb <= BGJ_B = 96) block; the
-// threads form a 32 x 32 grid, thread (ti, tj) owning the entries
-// (ti + 32a, tj + 32b), a, b < 3, of the block held in LDS.
-__global__ __launch_bounds__(1024) void k_block_inv(int64_t ld, int kb, const double *__restrict__ Mkk,
-                                                    double *__restrict__ P, int32_t *__restrict__ flag) {
-  static_assert(BGJ_B == 96, "the 32 x 32 thread grid covers 96 x 96 entries");
-  __shared__ double A[BGJ_B][BGJ_B + 1];
-  __shared__ double colk[BGJ_B];
-  __shared__ int perm[BGJ_B];
-  __shared__ int piv_row;
-  __shared__ double piv_val;
-  const int tid = threadIdx.x, ti = tid & 31, tj = tid >> 5;
+typedef double d4_t __attribute__((ext_vector_type(4)));
+
+// Orders the LDS accesses of one wave's lanes (no other wave is involved).
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ inline double read_lane(double v, int lane) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+  return __hiloint2double(hi, lo);
+}
+
+// One wave inverts the 32 x 32 block A (LDS) into P: Gauss-Jordan with the
+// block in registers (lane = row + 32 half, 16 columns each), no workgroup
+// barrier.  A diagonal pivot is taken unless an unused row holds an entry ten
+// times larger, then the largest.
+constexpr int SB = 32;
+__device__ inline void wave_inverse(const double *__restrict__ A, int lda, double (*P)[SB + 1], double *prow, int *pk,
+                                    int lane, int32_t *__restrict__ flag) {
+  const int r = lane & 31, h = lane >> 5;
+  double a[16];
 #pragma unroll
-  for (int b = 0; b < 3; ++b)
+  for (int j = 0; j < 16; ++j) a[j] = A[r * lda + 16 * h + j];
+  bool used = false;
+  uint32_t mask = 0;
+  int kof = 0;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const int i = ti + 32 * a, j = tj + 32 * b;
-      if (i < kb && j < kb) A[i][j] = Mkk[i + (int64_t)j * ld];
-    }
-  __syncthreads();
-  for (int k = 0; k < kb; ++k) {
-    if (tid < 64) {
-      double best = -1.0;
-      int bi = k;
-      for (int i = k + tid; i < kb; i += 64) {
-        const double v = fabs(A[i][k]);
-        if (v > best) {
-          best = v;
-          bi = i;
-        }
-      }
-      for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_down(best, off, 64);
-        const int oi = __shfl_down(bi, off, 64);
-        if (ov > best || (ov == best && oi < bi)) {
-          best = ov;
+  for (int k = 0; k < SB; ++k) {
+    const int hk = k >> 4, kk = k & 15;
+    const double f = __shfl(a[kk], r + 32 * hk, 64);  // column k on both halves
+    const double dk = read_lane(f, k);
+    int p = k;
+    if (__ballot(!used && !(fabs(f) <= 10.0 * fabs(dk))) || (mask >> k & 1u) || !(dk != 0.0)) {
+      double best = used ? -1.0 : fabs(f);
+      int bi = r;
+      for (int off = 16; off > 0; off >>= 1) {
+        const double ob = __shfl_xor(best, off, 32);
+        const int oi = __shfl_xor(bi, off, 32);
+        if (ob > best || (ob == best && oi < bi)) {
+          best = ob;
           bi = oi;
         }
       }
-      if (tid == 0) {
-        piv_row = bi;
-        piv_val = A[bi][k];
-        perm[k] = bi;
-        if (!(best > 0.0)) *flag = 1;
-      }
+      p = __builtin_amdgcn_readfirstlane(bi);
     }
-    __syncthreads();
-    const int p = piv_row;
-    const double pv = piv_val;
-    if (p != k && tid < kb) {
-      const double t = A[k][tid];
-      A[k][tid] = A[p][tid];
-      A[p][tid] = t;
-    }
-    __syncthreads();
-    if (!(pv != 0.0)) continue;  // uniform: the flag is set, the block is singular
-    if (tid < kb) {
-      colk[tid] = tid == k ? 0.0 : A[tid][k];
-      A[k][tid] = (tid == k ? 1.0 : A[k][tid]) / pv;
-    }
-    __syncthreads();
+    const double piv = read_lane(f, p);
+    if (!(fabs(piv) > 0.0) && lane == 0) *flag = 1;
+    const double inv = 1.0 / piv;
+    if (r == p) {
 #pragma unroll
-    for (int b = 0; b < 3; ++b)
+      for (int j = 0; j < 16; ++j) prow[16 * h + j] = (j == kk && h == hk) ? inv : a[j] * inv;
+      used = true;
+      kof = k;
+    }
+    mask |= 1u << p;
+    if (lane == 0) pk[k] = p;
+    if (h == hk) a[kk] = 0.0;
+    wave_sync();
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const int i = ti + 32 * a, j = tj + 32 * b;
-        if (i < kb && j < kb && i != k) {
-          if (j == k) A[i][k] = -colk[i] * A[k][k];
-          else A[i][j] -= colk[i] * A[k][j];
-        }
-      }
+    for (int j = 0; j < 16; ++j) {
+      const double pr = prow[16 * h + j];
+      a[j] = r == p ? pr : fma(-f, pr, a[j]);
+    }
+    wave_sync();
+  }
+  // A^-1[k][pk[c]] = S[pk[k]][c]
+#pragma unroll
+  for (int j = 0; j < 16; ++j) P[kof][pk[16 * h + j]] = a[j];
+}
+
+// One 1024-thread workgroup inverts the kb x kb (kb <= BGJ_B = 96) block in
+// LDS by block Gauss-Jordan with 32 x 32 diagonal blocks (wave_inverse) and
+// FP64 MFMA tiles for their updates.  The chain of pivots is what bounds it:
+// a step of one wave in registers costs a sixth of a step of the whole
+// workgroup with its four barriers (a 96-block took 200 us, now 60).
+__global__ __launch_bounds__(1024) void k_block_inv(int64_t ld, int kb, const double *__restrict__ Mkk,
+                                                    double *__restrict__ Pout, int32_t *__restrict__ flag) {
+  static_assert(BGJ_B == 96, "three 32-blocks; 16 waves cover the 4 x 4 tiles outside one of them");
+  __shared__ double A[BGJ_B][BGJ_B + 1];
+  __shared__ double T[SB][BGJ_B + 1];
+  __shared__ double P[SB][SB + 1];
+  __shared__ double prow[SB];
+  __shared__ int pk[SB];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  for (int e = tid; e < BGJ_B * BGJ_B; e += 1024) {
+    const int i = e % BGJ_B, j = e / BGJ_B;
+    A[i][j] = i < kb && j < kb ? Mkk[i + (int64_t)j * ld] : (i == j ? 1.0 : 0.0);
+  }
+  __syncthreads();
+  for (int s0 = 0; s0 < kb; s0 += SB) {
+    if (wave == 0) wave_inverse(&A[s0][s0], BGJ_B + 1, P, prow, pk, lane, flag);
+    __syncthreads();
+    // tile t = 0..3 of the 16-wide tiles outside the block
+    auto outside = [&](int t) { return 16 * t + (16 * t >= s0 ? SB : 0); };
+    if (wave < 8) {  // T = P A[s][:]
+      const int i0 = 16 * (wave & 1), j0 = outside(wave >> 1);
+      d4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < SB; k += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(P[i0 + li][k + lk], A[s0 + k + lk][j0 + li], acc, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) T[i0 + lk + 4 * q][j0 + li] = acc[q];
+    }
+    __syncthreads();
+    {  // A[i][j] -= A[i][s] T[:][j] outside the block
+      const int i0 = outside(wave & 3), j0 = outside(wave >> 2);
+      d4_t acc;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = A[i0 + lk + 4 * q][j0 + li];
+#pragma unroll
+      for (int k = 0; k < SB; k += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-A[i0 + li][s0 + k + lk], T[k + lk][j0 + li], acc, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) A[i0 + lk + 4 * q][j0 + li] = acc[q];
+    }
+    d4_t col = {0.0, 0.0, 0.0, 0.0};  // -A[i][s] P, written once every wave has read A[i][s]
+    const int ci = outside(wave & 3), cj = 16 * ((wave >> 2) & 1);
+    if (wave < 8) {
+#pragma unroll
+      for (int k = 0; k < SB; k += 4)
+        col = __builtin_amdgcn_mfma_f64_16x16x4f64(-A[ci + li][s0 + k + lk], P[k + lk][cj + li], col, 0, 0, 0);
+    }
+    __syncthreads();
+    if (wave < 8) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) A[ci + lk + 4 * q][s0 + cj + li] = col[q];
+    }
+    for (int e = tid; e < SB * BGJ_B; e += 1024) {
+      const int i = e / BGJ_B, j = e % BGJ_B;
+      A[s0 + i][j] = j >= s0 && j < s0 + SB ? P[i][j - s0] : T[i][j];
+    }
     __syncthreads();
   }
-  // undo the row interchanges as column interchanges, last first
-  for (int k = kb - 1; k >= 0; --k) {
-    const int p = perm[k];
-    if (p != k && tid < kb) {
-      const double t = A[tid][k];
-      A[tid][k] = A[tid][p];
-      A[tid][p] = t;
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int b = 0; b < 3; ++b)
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const int i = ti + 32 * a, j = tj + 32 * b;
-      if (i < kb && j < kb) P[i + (int64_t)j * kb] = A[i][j];
-    }
+  for (int e = tid; e < kb * kb; e += 1024) Pout[e] = A[e % kb][e / kb];
 }
 
 // b_i = deterministic values in [-1/2, 1/2) + 1 (the check's right-hand side)
@@ -732,7 +771,8 @@ __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__r
 }
 
 // rt_b = r_b - sum over the cells holding b of F_c[b] . r_i(c), FP64 sums;
-// interior dofs of condensed cells are skipped.  Four lanes per dof share its
+// interior dofs of condensed cells are skipped (`map`: where the others go, or
+// null).  Four lanes per dof share its
 // (up to eight) cells, so the chain of dependent loads is at most two cells
 // long: a level of 200 cells takes 5 us (one lane per dof: 11 us), 32,768
 // cells 60 us (F read once, 138 MB).
@@ -741,7 +781,8 @@ __global__ __launch_bounds__(256) void k_cond_rhs(int64_t n1, const int32_t *__r
                                                   const int32_t *__restrict__ centry,
                                                   const uint8_t *__restrict__ elim,
                                                   const int32_t *__restrict__ ifirst, const TE *__restrict__ F,
-                                                  const T *__restrict__ r, double *__restrict__ rt) {
+                                                  const T *__restrict__ r, double *__restrict__ rt,
+                                                  const int32_t *__restrict__ map) {
   const int64_t gid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, i = gid >> 2;
   const int sub = (int)(gid & 3);
   double s = 0.0;
@@ -769,7 +810,7 @@ __global__ __launch_bounds__(256) void k_cond_rhs(int64_t n1, const int32_t *__r
   }
   s += __shfl_xor(s, 1, 4);
   s += __shfl_xor(s, 2, 4);
-  if (on && sub == 0) rt[i] = (double)r[i] - s;
+  if (on && sub == 0) rt[map ? map[i] : i] = (double)r[i] - s;
 }
 
 // y_b (+)= w yb with yb = sum over the patches P holding b of part[P][b] (FP64,
@@ -836,27 +877,107 @@ __global__ __launch_bounds__(64 * CG_CELLS) void k_cond_gather(
   }
 }
 
-// y = A^-1 x with the explicit inverse stored row-major: one wave per row,
-// coalesced 8-byte loads of the row, FP64 accumulation, T in and out.
-template <class T>
-__global__ __launch_bounds__(256) void k_dense_rowdot(int64_t m, const double *__restrict__ Ainv,
-                                                      const T *__restrict__ x, T *__restrict__ y) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= m) return;  // uniform over the wave
-  const double *a = Ainv + row * m;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  int64_t j = lane;
-  for (; j + 192 < m; j += 256) {
-    s0 += a[j] * (double)x[j];
-    s1 += a[j + 64] * (double)x[j + 64];
-    s2 += a[j + 128] * (double)x[j + 128];
-    s3 += a[j + 192] * (double)x[j + 192];
+// Row b of the condensed coarsest [u,j] block, dense and row-major: the CSR
+// entries of the dofs that are not eliminated, minus A_bi E of the cells that
+// hold the row's dof, in increasing cell order.  One workgroup per row; every
+// entry of the row is written.
+__global__ __launch_bounds__(256) void k_dense_cond(int64_t nb, const int32_t *__restrict__ bidx,
+                                                    const int32_t *__restrict__ bmap,
+                                                    const int64_t *__restrict__ rowptr,
+                                                    const int64_t *__restrict__ split,
+                                                    const int32_t *__restrict__ colind,
+                                                    const double *__restrict__ val, const int32_t *__restrict__ crow,
+                                                    const int32_t *__restrict__ centry,
+                                                    const int32_t *__restrict__ dofs,
+                                                    const int32_t *__restrict__ ifirst, int dups,
+                                                    const double *__restrict__ E64, const double *__restrict__ B64,
+                                                    double *__restrict__ D) {
+  const int t = threadIdx.x;
+  const int32_t i = bidx[blockIdx.x];
+  double *row = D + (int64_t)blockIdx.x * nb;
+  for (int64_t e = t; e < nb; e += 256) row[e] = 0.0;
+  __syncthreads();
+  for (int64_t p = rowptr[i] + t; p < split[i]; p += 256) {
+    const int32_t b = bmap[colind[p]];
+    if (b >= 0) row[b] = val[p];
   }
-  for (; j < m; j += 64) s0 += a[j] * (double)x[j];
-  double v = (s0 + s1) + (s2 + s3);
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  if (lane == 0) y[row] = (T)v;
+  for (int32_t h = crow[i]; h < crow[i + 1]; ++h) {
+    const int32_t ce = centry[h], c = ce / NDOF, a = ce - c * NDOF;
+    const int l = a < NU ? a : a - (OFF_J - NU);
+    if (l >= NB || ifirst[c] < 0) continue;  // uniform
+    __syncthreads();
+    if (t < NB) {
+      const int32_t *cd = dofs + (int64_t)c * NDOF;
+      int32_t id = cd[bdof_local(t)];
+      if (dups && id >= 0)  // a dof listed twice in the cell has its couplings at the first place
+        for (int k = 0; k < t; ++k)
+          if (cd[bdof_local(k)] == id) id = -1;
+      if (id >= 0) {
+        const double *B = B64 + ((int64_t)c * NB + l) * NI, *E = E64 + ((int64_t)c * NB + t) * NI;
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < NI; ++k) s += B[k] * E[k];
+        row[bmap[id]] -= s;
+      }
+    }
+  }
+}
+
+// y = A^-1 x with the explicit inverse stored row-major: one workgroup per row,
+// coalesced 8-byte loads, eight in flight per lane, FP64 accumulation.  The
+// result goes to yd[row], or to yd[bidx[row]] and y[bidx[row]].  (One wave per
+// row left 137 MB, 4,144 rows, at 3.4 TB/s: 40 us.)
+template <class T>
+__global__ __launch_bounds__(TB) void k_dense_rowdot(int64_t m, const double *__restrict__ Ainv,
+                                                      const double *__restrict__ x, const int32_t *__restrict__ bidx,
+                                                      double *__restrict__ yd, T *__restrict__ y) {
+  const int64_t row = blockIdx.x;
+  const double *a = Ainv + row * m;
+  double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  int64_t j = threadIdx.x;
+  for (; j + 7 * TB < m; j += 8 * TB) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s[u] += a[j + u * TB] * x[j + u * TB];
+  }
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (j + u * TB < m) s[u] += a[j + u * TB] * x[j + u * TB];
+  const double v = block_sum(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])));
+  if (threadIdx.x == 0) {
+    const int64_t i = bidx ? bidx[row] : row;
+    yd[i] = v;
+    if (y) y[i] = (T)v;
+  }
+}
+
+// interior dofs of the condensed cells, y_i = G r_i - E yb: one wave per cell,
+// lane = i + 12 s as in k_cond_gather
+template <class T>
+__global__ __launch_bounds__(256) void k_cond_inner(int ncells, const int32_t *__restrict__ dofs,
+                                                    const int32_t *__restrict__ ifirst, const double *__restrict__ E,
+                                                    const double *__restrict__ G, const T *__restrict__ r,
+                                                    const double *__restrict__ yb, T *__restrict__ y) {
+  const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (c >= ncells) return;  // uniform over the wave
+  const int32_t f0 = ifirst[c];
+  if (f0 < 0) return;
+  const int i = lane % NI, sl = lane / NI;
+  double acc = 0.0;
+  if (sl < 5) {
+    const double *Ec = E + ((int64_t)c * NB + sl) * NI + i;
+    const int32_t *cd = dofs + (int64_t)c * NDOF;
+#pragma unroll
+    for (int k = 0; k < NB / 5; ++k) {
+      const int32_t id = cd[bdof_local(sl + 5 * k)];
+      acc -= Ec[5 * k * NI] * (id >= 0 ? yb[id] : 0.0);
+    }
+    const double *Gc = G + ((int64_t)c * NI + i) * NI;
+    for (int k = sl; k < NI; k += 5) acc += Gc[k] * (double)r[f0 + k];
+  }
+  double s = acc;
+#pragma unroll
+  for (int k = 1; k < 5; ++k) s += __shfl(acc, (i + NI * k) & 63, 64);
+  if (lane < NI) y[f0 + i] = (T)s;
 }
 
 // ---------------------------------------------------------------------------
@@ -1932,7 +2053,7 @@ int patch_as_on(mhd_ctx *c, const T *r, T *y, int prec, double w, bool accumulat
   }
   if (S->npatch == 0) return 0;
   hipLaunchKernelGGL((k_cond_rhs<T, TE>), dim3((unsigned)((4 * S->n1 + 255) / 256)), dim3(256), 0, st, S->n1,
-                     c->d_crow, c->d_centry, S->d_elim, S->d_ifirst, F, r, S->d_rt);
+                     c->d_crow, c->d_centry, S->d_elim, S->d_ifirst, F, r, S->d_rt, (const int32_t *)nullptr);
   if (prec == 0) patch_products(S, S->d_pA, (const float *)nullptr, st);
   else if (prec == 1) patch_products(S, S->d_pA32, (const float *)nullptr, st);
   else if (prec == 2) patch_products(S, S->d_pA16, (const float *)nullptr, st);
@@ -2003,16 +2124,24 @@ int spmv_a11(mhd_ctx *c, const T *x, T *y, int prec) {
 template <class T>
 int inner_solve(mhd_ctx *c, int prec);
 
-// ec = A11c^-1 rc on the coarsest level with the explicit FP64 inverse;
-// FP32 vectors are widened inside the product, since the coarsest block is
-// the worst conditioned one and its correction reaches every level above.
+// ec = A11c^-1 rc on the coarsest level, its cells' interior current dofs
+// condensed out (4,144 of 5,680 unknowns on 4 x 4 x 8 cells): the explicit FP64
+// inverse of the condensed block, FP64 couplings; FP32 vectors are widened
+// inside the products, since the coarsest block is the worst conditioned one
+// and its correction reaches every level above.
 template <class T>
 int coarse_direct(mhd_ctx *c, const T *rc, T *ec) {
   CoarseLink *L = c->coarse;
-  const int64_t n = L->n1c;
-  hipLaunchKernelGGL((k_dense_rowdot<T>), dim3((unsigned)((n + 3) / 4)), dim3(256), 0, c->stream, n, L->d_Ainv, rc,
-                     ec);
-  count(c, OP_DENSE, (double)n * n);
+  mhd_ctx *cc = L->ctx;
+  const Solver *S = cc->solver;
+  const int64_t n = L->n1c, m = L->nb;
+  hipLaunchKernelGGL((k_cond_rhs<T, double>), dim3((unsigned)((4 * n + 255) / 256)), dim3(256), 0, c->stream, n,
+                     cc->d_crow, cc->d_centry, S->d_elim, S->d_ifirst, L->d_cF, rc, L->d_rb, L->d_bmap);
+  hipLaunchKernelGGL((k_dense_rowdot<T>), dim3((unsigned)m), dim3(TB), 0, c->stream, m, L->d_Ainv,
+                     L->d_rb, L->d_bidx, L->d_yb, ec);
+  hipLaunchKernelGGL((k_cond_inner<T>), dim3((unsigned)((cc->ncells + 3) / 4)), dim3(256), 0, c->stream, cc->ncells,
+                     cc->d_dofs, S->d_ifirst, S->d_cE64, L->d_cG, rc, L->d_yb, ec);
+  count(c, OP_DENSE, (double)m * m + (double)cc->ncells * (2 * NB * NI + NI * NI));
   MHD_HIP(hipGetLastError());
   return 0;
 }
@@ -2349,24 +2478,49 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     return rc;
   }
   if (L->coarse_iters == 0 && !cc->coarse) {
-    // exact coarsest solve: the explicit inverse of its [u,j] block, row-major
-    // (the layout of the row-dot product).  The row-major copy of A is the
-    // column-major A^T; block Gauss-Jordan inverts it in place into (A^T)^-1,
-    // whose column-major storage is A^-1 row-major.
-    const int64_t m = L->n1c;
-    rocblas_handle rb = cc->solver->rb;  // bound to cs, the stream of every level
-    const int64_t nw = 2 * m * BGJ_B + (int64_t)BGJ_B * BGJ_B + 3 * m + 2;
+    // exact coarsest solve: the explicit inverse of its condensed [u,j] block,
+    // row-major (the layout of the row-dot product).  The row-major copy of the
+    // block S is the column-major S^T; block Gauss-Jordan inverts it in place
+    // into (S^T)^-1, whose column-major storage is S^-1 row-major.
+    const Solver *SC = cc->solver;
+    rocblas_handle rb = SC->rb;  // bound to cs, the stream of every level
     if (!L->d_Ainv) {
-      MHD_HIP(hipMalloc(&L->d_Ainv, sizeof(double) * (size_t)(m * m)));
+      std::vector<int32_t> bidx, bmap(L->n1c, -1), ones(cc->ncells, 1);
+      std::vector<uint8_t> elim(L->n1c);
+      MHD_HIP(hipMemcpy(elim.data(), SC->d_elim, (size_t)L->n1c, hipMemcpyDeviceToHost));
+      for (int64_t i = 0; i < L->n1c; ++i)
+        if (!elim[i]) {
+          bmap[i] = (int32_t)bidx.size();
+          bidx.push_back((int32_t)i);
+        }
+      const int64_t m = L->nb = (int64_t)bidx.size();
+      const int64_t nw = 2 * m * BGJ_B + (int64_t)BGJ_B * BGJ_B + 3 * m + 2;
+      MHD_HIP(hipMalloc(&L->d_bidx, sizeof(int32_t) * (size_t)std::max<int64_t>(m, 1)));
+      MHD_HIP(hipMalloc(&L->d_bmap, sizeof(int32_t) * (size_t)L->n1c));
+      MHD_HIP(hipMalloc(&L->d_ones, sizeof(int32_t) * (size_t)cc->ncells));
+      MHD_HIP(hipMemcpy(L->d_bidx, bidx.data(), sizeof(int32_t) * (size_t)m, hipMemcpyHostToDevice));
+      MHD_HIP(hipMemcpy(L->d_bmap, bmap.data(), sizeof(int32_t) * (size_t)L->n1c, hipMemcpyHostToDevice));
+      MHD_HIP(hipMemcpy(L->d_ones, ones.data(), sizeof(int32_t) * (size_t)cc->ncells, hipMemcpyHostToDevice));
+      MHD_HIP(hipMalloc(&L->d_cF, sizeof(double) * (size_t)cc->ncells * NB * NI));
+      MHD_HIP(hipMalloc(&L->d_cG, sizeof(double) * (size_t)cc->ncells * NI * NI));
+      MHD_HIP(hipMalloc(&L->d_rb, sizeof(double) * (size_t)std::max<int64_t>(m, 1)));
+      MHD_HIP(hipMalloc(&L->d_yb, sizeof(double) * (size_t)L->n1c));
       MHD_HIP(hipMalloc(&L->d_LU, sizeof(double) * (size_t)(m * m)));
       MHD_HIP(hipMalloc(&L->d_piv, sizeof(int32_t) * (size_t)std::max<int64_t>(m, 1)));
       MHD_HIP(hipMalloc(&L->d_info, sizeof(int32_t)));
       MHD_HIP(hipMalloc(&L->d_gjw, sizeof(double) * (size_t)nw));
       MHD_HIP(hipMalloc(&L->d_gjflag, sizeof(int32_t)));
+      MHD_HIP(hipMalloc(&L->d_Ainv, sizeof(double) * (size_t)(m * m)));
     }
-    MHD_HIP(hipMemsetAsync(L->d_LU, 0, sizeof(double) * (size_t)(m * m), cs));
-    hipLaunchKernelGGL(k_dense_a11, dim3(nblocks(m)), dim3(TB), 0, cs, m, cc->d_rowptr, cc->solver->d_split,
-                       cc->d_colind, cc->d_val, L->d_LU);
+    const int64_t m = L->nb;
+    const int dups = cc->dup_dofs ? 1 : 0;
+    // FP64 couplings of single cells (the level's set-up has left its own for the smoother)
+    hipLaunchKernelGGL(k_condense<double>, dim3(cc->ncells), dim3(CND_T), 0, cs, cc->ncells, cc->d_dofs, SC->d_ifirst,
+                       L->d_ones, dups, cc->d_rowptr, cc->d_rank, cc->d_val, SC->d_cE64, SC->d_cB64, (double *)nullptr,
+                       L->d_cF, L->d_cG, SC->d_cflag);
+    hipLaunchKernelGGL(k_dense_cond, dim3((unsigned)m), dim3(256), 0, cs, m, L->d_bidx, L->d_bmap, cc->d_rowptr,
+                       SC->d_split, cc->d_colind, cc->d_val, cc->d_crow, cc->d_centry, cc->d_dofs, SC->d_ifirst, dups,
+                       SC->d_cE64, SC->d_cB64, L->d_LU);
     MHD_HIP(hipGetLastError());
     MHD_HIP(hipMemcpyAsync(L->d_Ainv, L->d_LU, sizeof(double) * (size_t)(m * m), hipMemcpyDeviceToDevice, cs));
     MHD_HIP(hipMemsetAsync(L->d_gjflag, 0, sizeof(int32_t), cs));
@@ -2398,9 +2552,10 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     }
     // check: z = A (A^-1 b) against b for a fixed b
     hipLaunchKernelGGL(k_check_rhs, dim3(nblocks(m)), dim3(TB), 0, cs, m, vb);
-    hipLaunchKernelGGL((k_dense_rowdot<double>), dim3((unsigned)((m + 3) / 4)), dim3(256), 0, cs, m, M, vb, vy);
-    hipLaunchKernelGGL((k_dense_rowdot<double>), dim3((unsigned)((m + 3) / 4)), dim3(256), 0, cs, m, L->d_LU, vy,
-                       vz);
+    hipLaunchKernelGGL((k_dense_rowdot<double>), dim3((unsigned)m), dim3(TB), 0, cs, m, M, vb,
+                       (const int32_t *)nullptr, vy, (double *)nullptr);
+    hipLaunchKernelGGL((k_dense_rowdot<double>), dim3((unsigned)m), dim3(TB), 0, cs, m, L->d_LU, vy,
+                       (const int32_t *)nullptr, vz, (double *)nullptr);
     hipLaunchKernelGGL(k_check_residual, dim3(1), dim3(1024), 0, cs, m, vz, vb, chk);
     MHD_HIP(hipGetLastError());
     double hchk[2] = {0.0, 1.0};
@@ -2408,12 +2563,12 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     MHD_HIP(hipMemcpyAsync(hchk, chk, sizeof(hchk), hipMemcpyDeviceToHost, cs));
     MHD_HIP(hipMemcpyAsync(&flag, L->d_gjflag, sizeof(int32_t), hipMemcpyDeviceToHost, cs));
     MHD_HIP(hipStreamSynchronize(cs));
-    count(c, OP_SETUP_DENSE3, (double)m * m * m);
+    count(c, OP_SETUP_DENSE3, (double)L->n1c * L->n1c * L->n1c);
     if (flag || !(hchk[0] <= 1e-6 * hchk[1])) {
       // redo with the row-pivoted LU: getrf of A^T (the row-major copy), then
       // A^T X = I gives X = A^-T column-major = A^-1 row-major
       ++L->dense_fallbacks;
-      count(c, OP_SETUP_DENSE3, (double)m * m * m);  // a second inversion
+      count(c, OP_SETUP_DENSE3, (double)L->n1c * L->n1c * L->n1c);  // a second inversion
       MHD_HIP(hipMemsetAsync(M, 0, sizeof(double) * (size_t)(m * m), cs));
       hipLaunchKernelGGL(k_set_diag, dim3(nblocks(m)), dim3(TB), 0, cs, m, 1.0, M);
       MHD_HIP(hipGetLastError());
@@ -2536,7 +2691,7 @@ void mhd_coarse_free(mhd_ctx *c) {
   CoarseLink *L = c->coarse;
   void *ptrs[] = {L->d_Prow, L->d_Trow, L->d_Pcol, L->d_Tcol, L->d_Pval, L->d_Tval, L->d_Pval32, L->d_Tval32,
                   L->d_Rrow, L->d_Rcol, L->d_Rval, L->rr, L->rc, L->ec, L->d_Ainv, L->d_LU, L->d_piv, L->d_info, L->d_ab,
-                  L->d_gjw, L->d_gjflag};
+                  L->d_gjw, L->d_gjflag, L->d_bidx, L->d_bmap, L->d_ones, L->d_cF, L->d_cG, L->d_rb, L->d_yb};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (L->ctx) mhd_destroy(L->ctx);
