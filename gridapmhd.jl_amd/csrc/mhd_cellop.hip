@@ -3,23 +3,25 @@
 // with the Jacobian, its [u,j] block, its (u,j) x (p,phi) block, and their
 // transposes.
 //
-// Half a wave (32 lanes) per cell, two cells per 64-thread workgroup.  A lane
-// is first a quadrature point: it evaluates every field of the input there
-// from the cell's 129 values in LDS (broadcast reads) with its own 1-D
-// factors, maps to physical coordinates, forms the fluxes of the weak form and
-// pulls them back to the reference cell (18 numbers per point, LDS).  Then it
-// is a test function: a Q2 node with its three components, then an RT1 face
-// dof, then an RT1 interior / dP1 / dQ1 dof, and sums the fluxes over the 27
-// points, again with 1-D factors.  No basis vector is mapped or stored: a cell
-// costs about 1,300 FMAs per lane and 600 LDS reads, where a kernel that works
-// in physical space pushes 27 x (27 + 36) basis vectors through LDS per cell.
-// Element results go to a buffer [cell][129] and a second kernel adds them per
-// dof in increasing cell order: no atomics, the same bits in every run.
+// Half a wave (32 lanes) per cell, two cells per 64-thread workgroup (one wave:
+// its barriers cost nothing).  The cell's 129 input values go to LDS; the
+// fields at the 27 quadrature points come from them by sum factorisation, one
+// axis per pass: lane (d0, d1, d2) owns row d0 + 3 d1 + 9 d2 of the cell's
+// buffer, and its digits turn from node to point indices axis by axis, in
+// place.  There the lane is a quadrature point: it maps to physical
+// coordinates, forms the fluxes of the weak form and pulls them back to the
+// reference cell (17 numbers).  Three passes back contract them with the test
+// functions, until the lane is a Q2 node and up to three RT1 dofs and a dQ1
+// vertex.  About 550 FMAs and 310 LDS accesses per lane; evaluating every point
+// from all nodal values directly took 1,300 and 610.  Element results go to a
+// buffer [cell][129] and a second kernel adds them per dof in increasing cell
+// order: no atomics, the same bits in every run.
 //
-// Residual at 64 x 64 x 8 (32,768 cells): 2.31 -> 0.158 ms (cell kernel 0.136,
-// sums 0.025), at 8 x 8 x 3: 53 -> 17 us (13 + 4, latency of one cell).  The
-// cell kernel is bound by LDS reads (0.06 ms of them) and their latency at two
-// waves per SIMD.
+// Residual at 64 x 64 x 8 (32,768 cells): 2.31 -> 0.132 ms (cell kernel 0.105,
+// sums 0.025), at 8 x 8 x 3: 53 -> 14 us (10 + 4); an A11 product on 8,192 cells:
+// 132 us streamed in FP32 -> 22 + 7 us on average over the V-cycle's levels.  Bound by
+// latency at two waves per SIMD (200 VGPRs): direct evaluation took 0.136 ms,
+// and a register budget for three waves spills and is slower (0.112 ms).
 #include <algorithm>
 
 #include "mhd_internal.h"
@@ -76,6 +78,7 @@ struct Axis {
   }
 };
 
+constexpr int ROW = 18;  // doubles per row of the cell's buffer
 struct CellIn {
   double x[NDOF + 1];    // input values, RT1 face dofs times their orientation
   double xyz[24];
@@ -83,46 +86,100 @@ struct CellIn {
   double sg[6];
   double dq[4];          // int psi_k div u
   double wd[NQ + 1];     // W div u at the points
-  double fl[NQ][18];     // fluxes: 3 x (S_k, T_0k, T_1k, T_2k), (v_0, v_1, v_2, c), W div j, unused
+  double fl[NQ][ROW];    // pass results; fluxes 3 x (S_k, T_0k, T_1k, T_2k), (v_0, v_1, v_2, c), W div j
 };
 
-// value and reference gradient of one Q2 component from its 27 nodal values
-__device__ inline void q2_eval(const double *__restrict__ v, const Axis &ax, const Axis &ay, const Axis &az, double &f,
-                               double &f0, double &f1, double &f2) {
-  f = f0 = f1 = f2 = 0.0;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    double s = 0.0, s0 = 0.0, s1 = 0.0;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const double *r = v + 3 * j + 9 * k;
-      const double a = ax.b[0] * r[0] + ax.b[1] * r[1] + ax.b[2] * r[2];
-      const double da = ax.d[0] * r[0] + ax.d[1] * r[1] + ax.d[2] * r[2];
-      s += ay.b[j] * a;
-      s0 += ay.b[j] * da;
-      s1 += ay.d[j] * a;
-    }
-    f += az.b[k] * s;
-    f0 += az.b[k] * s0;
-    f1 += az.b[k] * s1;
-    f2 += az.d[k] * s;
-  }
+__device__ inline double dot3(const double *__restrict__ f, const double *__restrict__ v, int stride) {
+  return f[0] * v[0] + f[1] * v[stride] + f[2] * v[2 * stride];
 }
 
-// reference component d of the RT1 field and its derivative along d; the face
-// dofs of the lower / upper side at lo / hi, the interior ones at in
-__device__ inline void rt_eval(const double *__restrict__ lo, const double *__restrict__ hi,
-                               const double *__restrict__ in, const Axis &ad, const Axis &ta, const Axis &tb, double &v,
-                               double &dv) {
-  double s[3];
+// Values and reference gradients out[c] = (f, d0 f, d1 f, d2 f) of the three
+// velocity components from node values v[27 c + node], and with RT the
+// reference components V of the RT1 field and its reference divergence from
+// the 36 dofs xj: three passes through rows of `st` doubles (9, or 14 with RT)
+// for lane digits d.  wr: the lane owns its row.
+template <bool RT>
+__device__ inline void fields_forward(const double *__restrict__ v, const double *__restrict__ xj,
+                                      double *__restrict__ fl, int st, const int *d, bool wr, double (*out)[4],
+                                      double *V, double &div) {
+  double *own = fl + (d[0] + 3 * d[1] + 9 * d[2]) * st;
+  const int t1 = d[1] ? 1 : 0, t2 = d[2] ? 1 : 0;  // tangential index of the RT1 dofs (digit 2: a spare lane)
+  {
+    const Axis a(d[0]);
+    if (wr) {
 #pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    const double *r = m == 0 ? lo : (m == 1 ? in : hi);
-    s[m] = tb.g[0] * (ta.g[0] * r[0] + ta.g[1] * r[1]) + tb.g[1] * (ta.g[0] * r[2] + ta.g[1] * r[3]);
+      for (int c = 0; c < 3; ++c) {
+        const double *r = v + 27 * c + 3 * d[1] + 9 * d[2];
+        own[2 * c] = dot3(a.b, r, 1);
+        own[2 * c + 1] = dot3(a.d, r, 1);
+      }
+      if (RT) {
+        const double *r = xj + t1 + 2 * t2;  // axis x: (normal; y, z), normal dofs at 16, 24, 20
+        own[6] = a.b[0] * r[16] + a.b[1] * r[24] + a.b[2] * r[20];
+        own[7] = a.d[0] * r[16] + a.d[1] * r[24] + a.d[2] * r[20];
+        const double *ry = xj + (d[1] == 0 ? 8 : (d[1] == 1 ? 28 : 12)) + 2 * t2;  // axis y: (x, z)
+        own[8] = a.g[0] * ry[0] + a.g[1] * ry[1];
+        const double *rz = xj + (d[2] == 0 ? 0 : (d[2] == 1 ? 32 : 4)) + 2 * t1;   // axis z: (x, y)
+        own[9] = a.g[0] * rz[0] + a.g[1] * rz[1];
+      }
+    }
   }
-  v = ad.b[0] * s[0] + ad.b[1] * s[1] + ad.b[2] * s[2];
-  dv = ad.d[0] * s[0] + ad.d[1] * s[1] + ad.d[2] * s[2];
+  __syncthreads();
+  {
+    const Axis a(d[1]);
+    const double *r = fl + (d[0] + 9 * d[2]) * st;
+    double y[14];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      y[3 * c] = dot3(a.b, r + 2 * c, 3 * st);
+      y[3 * c + 1] = dot3(a.b, r + 2 * c + 1, 3 * st);
+      y[3 * c + 2] = dot3(a.d, r + 2 * c, 3 * st);
+    }
+    if (RT) {
+      y[9] = a.g[0] * r[6] + a.g[1] * r[3 * st + 6];
+      y[10] = a.g[0] * r[7] + a.g[1] * r[3 * st + 7];
+      y[11] = dot3(a.b, r + 8, 3 * st);
+      y[12] = dot3(a.d, r + 8, 3 * st);
+      y[13] = a.g[0] * r[9] + a.g[1] * r[3 * st + 9];
+    }
+    __syncthreads();
+    if (wr)
+#pragma unroll
+      for (int k = 0; k < (RT ? 14 : 9); ++k) own[k] = y[k];
+  }
+  __syncthreads();
+  const Axis a(d[2]);
+  const double *r = fl + (d[0] + 3 * d[1]) * st;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    out[c][0] = dot3(a.b, r + 3 * c, 9 * st);
+    out[c][1] = dot3(a.b, r + 3 * c + 1, 9 * st);
+    out[c][2] = dot3(a.b, r + 3 * c + 2, 9 * st);
+    out[c][3] = dot3(a.d, r + 3 * c, 9 * st);
+  }
+  if (RT) {
+    V[0] = a.g[0] * r[9] + a.g[1] * r[9 * st + 9];
+    V[1] = a.g[0] * r[11] + a.g[1] * r[9 * st + 11];
+    V[2] = dot3(a.b, r + 13, 9 * st);
+    div = (a.g[0] * r[10] + a.g[1] * r[9 * st + 10]) + (a.g[0] * r[12] + a.g[1] * r[9 * st + 12]) +
+          dot3(a.d, r + 13, 9 * st);
+  }
+  __syncthreads();
 }
+
+// factors of the test functions with index i along one axis at the three points
+struct TestAxis {
+  double b[3], d[3], g[3], l[3];
+  __device__ explicit TestAxis(int i) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      b[q] = q2_val(i, q);
+      d[q] = q2_der(i, q);
+      g[q] = g2_val(i, q);
+      l[q] = i ? GX[q] : 1.0 - GX[q];
+    }
+  }
+};
 
 // Jacobian of the trilinear map at a point: J[3 k + l] = d x_k / d xi_l
 __device__ inline void tri_jacobian(const double *__restrict__ X, double x, double y, double z, double *J) {
@@ -179,7 +236,19 @@ __global__ __launch_bounds__(64) void k_cell_op(CellOpArgs A, MhdPhys ph, const 
   const int c = blockIdx.x * 2 + half;
   const bool live = c < A.ncells;
   CellIn &S = sh[half];
+  constexpr bool LIN = OP == OP_FULL || OP == OP_UJ;
+  double st[12];  // state at the lane's point, on its way during the passes
+  int e0 = 0, e1 = 0;
   if (live) {
+    if (LIN && ph.convection) {
+      const double *sp = A.state + (int64_t)c * 12 * NQ + (hl < NQ ? hl : NQ - 1);
+#pragma unroll
+      for (int k = 0; k < 12; ++k) st[k] = k < 3 || ph.convection == 2 ? sp[k * NQ] : 0.0;
+    }
+    if (UJ) {
+      e0 = A.cfptr[c];
+      e1 = A.cfptr[c + 1];
+    }
     const int32_t *cd = A.dofs + (int64_t)c * NDOF;
     if (hl < 24) S.xyz[hl] = A.xyz[(int64_t)c * 24 + hl];
     if (hl < 16) S.minv[hl] = A.minv[(int64_t)c * 16 + hl];
@@ -203,34 +272,30 @@ __global__ __launch_bounds__(64) void k_cell_op(CellOpArgs A, MhdPhys ph, const 
     }
   }
   __syncthreads();
-  const int q = hl < NQ ? hl : NQ - 1;  // lanes 27..31 repeat the last point and write nothing
-  const int qx = q % 3, qy = (q / 3) % 3, qz = q / 9;
-  const double px = gauss_x(qx), py = gauss_x(qy), pz = gauss_x(qz);
-  double J[9], Ji[9], W, id;
+  const int q = hl < NQ ? hl : NQ - 1;  // lanes 27..31 repeat the last row and write nothing
+  const int d[3] = {q % 3, (q / 3) % 3, q / 9};
+  const bool wr = hl < NQ;
+  const double px = gauss_x(d[0]), py = gauss_x(d[1]), pz = gauss_x(d[2]);
+  double J[9], Ji[9], W = 0.0, id = 0.0;
   double u[3] = {0, 0, 0}, gu[9], j[3] = {0, 0, 0}, dj = 0.0, p = 0.0, phi = 0.0, divu = 0.0;
+  double fw[3][4], V[3], dv = 0.0;
+  if (UJ)  // every lane takes part (the passes hold barriers); a dead half works on its own unused buffer
+    fields_forward<true>(S.x, S.x + OFF_J, &S.fl[0][0], ROW, d, wr, fw, V, dv);
   if (live) {
-    const Axis ax(qx), ay(qy), az(qz);
     tri_jacobian(S.xyz, px, py, pz, J);
     const double det = inv3(J, Ji);
     id = 1.0 / det;
-    W = gauss_w(qx) * gauss_w(qy) * gauss_w(qz) * fabs(det);
+    W = gauss_w(d[0]) * gauss_w(d[1]) * gauss_w(d[2]) * fabs(det);
     if (UJ) {
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        double r0, r1, r2;
-        q2_eval(S.x + 27 * k, ax, ay, az, u[k], r0, r1, r2);
+        u[k] = fw[k][0];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) gu[3 * i + k] = Ji[i] * r0 + Ji[3 + i] * r1 + Ji[6 + i] * r2;
+        for (int i = 0; i < 3; ++i) gu[3 * i + k] = Ji[i] * fw[k][1] + Ji[3 + i] * fw[k][2] + Ji[6 + i] * fw[k][3];
+        j[k] = (J[3 * k] * V[0] + J[3 * k + 1] * V[1] + J[3 * k + 2] * V[2]) * id;
       }
       divu = gu[0] + gu[4] + gu[8];
-      const double *xj = S.x + OFF_J;
-      double r0, r1, r2, d0, d1, d2;
-      rt_eval(xj + 16, xj + 20, xj + 24, ax, ay, az, r0, d0);
-      rt_eval(xj + 8, xj + 12, xj + 28, ay, ax, az, r1, d1);
-      rt_eval(xj, xj + 4, xj + 32, az, ax, ay, r2, d2);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) j[k] = (J[3 * k] * r0 + J[3 * k + 1] * r1 + J[3 * k + 2] * r2) * id;
-      dj = (d0 + d1 + d2) * id;
+      dj = dv * id;
     }
     if (PPHI) {
       const double *xp = S.x + OFF_P, *xf = S.x + OFF_PHI;
@@ -278,17 +343,11 @@ __global__ __launch_bounds__(64) void k_cell_op(CellOpArgs A, MhdPhys ph, const 
     Tk[8] += pr;
     if (UJ) {
       if (ph.convection) {
-        double us[3], gs[9];
         if (RES) {
 #pragma unroll
           for (int k = 0; k < 3; ++k) Sk[k] = ph.alpha * (gu[k] * u[0] + gu[3 + k] * u[1] + gu[6 + k] * u[2]);
         } else {
-          const double *st = A.state + (int64_t)c * 12 * NQ + q;
-#pragma unroll
-          for (int k = 0; k < 3; ++k) us[k] = st[k * NQ];
-          if (ph.convection == 2)
-#pragma unroll
-            for (int e = 0; e < 9; ++e) gs[e] = st[(3 + e) * NQ];
+          const double *us = st, *gs = st + 3;
           if (!TRANS) {  // alpha ((grad du)^T u0 [+ (grad u0)^T du])
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -358,125 +417,92 @@ __global__ __launch_bounds__(64) void k_cell_op(CellOpArgs A, MhdPhys ph, const 
     }
   }
   __syncthreads();
+  // Test functions.  Along x: lane (node / dof index, qy, qz) reads its group's
+  // three rows, all before any lane writes (one wave), then writes its own.
+  double *fl = &S.fl[0][0], *own = fl + q * ROW;
+  {
+    const TestAxis tx(d[0]);
+    const double *r = fl + (3 * d[1] + 9 * d[2]) * ROW;
+    double s[9], w[5];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      s[3 * k] = dot3(tx.b, r + 4 * k, ROW) + dot3(tx.d, r + 4 * k + 1, ROW);
+      s[3 * k + 1] = dot3(tx.b, r + 4 * k + 2, ROW);
+      s[3 * k + 2] = dot3(tx.b, r + 4 * k + 3, ROW);
+    }
+    w[0] = dot3(tx.b, r + 12, ROW) + dot3(tx.d, r + 15, ROW);  // RT1 axis x: done with the normal direction
+    w[1] = dot3(tx.g, r + 13, ROW);
+    w[2] = dot3(tx.g, r + 14, ROW);
+    w[3] = dot3(tx.g, r + 15, ROW);
+    if (ROWS2) w[4] = dot3(tx.l, r + 16, ROW);
+    __syncthreads();
+    if (wr) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) own[k] = s[k];
+#pragma unroll
+      for (int k = 0; k < (ROWS2 ? 5 : 4); ++k) own[9 + k] = w[k];
+    }
+    __syncthreads();
+  }
+  {
+    const TestAxis ty(d[1]);
+    const double *r = fl + (d[0] + 9 * d[2]) * ROW;
+    double s[6], w[5];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      s[2 * k] = dot3(ty.b, r + 3 * k, 3 * ROW) + dot3(ty.d, r + 3 * k + 1, 3 * ROW);
+      s[2 * k + 1] = dot3(ty.b, r + 3 * k + 2, 3 * ROW);
+    }
+    w[0] = dot3(ty.g, r + 9, 3 * ROW);
+    w[1] = dot3(ty.b, r + 10, 3 * ROW) + dot3(ty.d, r + 12, 3 * ROW);
+    w[2] = dot3(ty.g, r + 11, 3 * ROW);
+    w[3] = dot3(ty.g, r + 12, 3 * ROW);
+    if (ROWS2) w[4] = dot3(ty.l, r + 13, 3 * ROW);
+    __syncthreads();
+    if (wr) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) own[k] = s[k];
+#pragma unroll
+      for (int k = 0; k < (ROWS2 ? 5 : 4); ++k) own[6 + k] = w[k];
+    }
+    __syncthreads();
+  }
   if (!live) return;
   double *out = A.out + (int64_t)c * NDOF;
-  // Q2 node hl: three components
-  if (hl < 27) {
-    const int i = hl % 3, jj = (hl / 3) % 3, k = hl / 9;
-    double bx[3], dx[3], by[3], dy[3], bz[3], dz[3];
+  if (ROWS2 && hl >= 28) out[SLOT_P + hl - 28] = RES && A.mode == 1 ? 0.0 : -S.dq[hl - 28];  // p rows: -int psi_k div u
+  if (!wr) return;
+  const TestAxis tz(d[2]);
+  const double *r = fl + (d[0] + 3 * d[1]) * ROW;
 #pragma unroll
-    for (int m = 0; m < 3; ++m) {
-      bx[m] = q2_val(i, m);
-      dx[m] = q2_der(i, m);
-      by[m] = q2_val(jj, m);
-      dy[m] = q2_der(jj, m);
-      bz[m] = q2_val(k, m);
-      dz[m] = q2_der(k, m);
-    }
-#pragma unroll
-    for (int comp = 0; comp < 3; ++comp) {
-      double r = 0.0;
-#pragma unroll
-      for (int c2 = 0; c2 < 3; ++c2) {
-        double t0 = 0.0, t2 = 0.0;
-#pragma unroll
-        for (int c1 = 0; c1 < 3; ++c1) {
-          double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll
-          for (int c0 = 0; c0 < 3; ++c0) {
-            const double *f = &S.fl[c0 + 3 * c1 + 9 * c2][4 * comp];
-            s0 += bx[c0] * f[0] + dx[c0] * f[1];
-            s1 += bx[c0] * f[2];
-            s2 += bx[c0] * f[3];
-          }
-          t0 += by[c1] * s0 + dy[c1] * s1;
-          t2 += by[c1] * s2;
-        }
-        r += bz[c2] * t0 + dz[c2] * t2;
-      }
-      out[3 * hl + comp] = r;
-    }
+  for (int k = 0; k < 3; ++k) out[3 * q + k] = dot3(tz.b, r + 2 * k, 9 * ROW) + dot3(tz.d, r + 2 * k + 1, 9 * ROW);
+  if (ROWS2 && d[0] < 2 && d[1] < 2 && d[2] < 2) {
+    const double t = dot3(tz.l, r + 10, 9 * ROW);
+    out[SLOT_PHI + d[0] + 2 * d[1] + 4 * d[2]] = TRANS ? -ph.sigma * t : -t;
   }
-  // 24 face dofs of RT1, then its 12 interior dofs with the dP1 and dQ1 rows:
-  // sum_q f_x f_y f_z V + g_x g_y g_z C with the lane's own factors
-#pragma unroll 1
-  for (int pass = 0; pass < 2; ++pass) {
-    if (hl >= 24 || (pass && !ROWS2 && hl >= 12)) continue;
-    int d, m, ga, gb, vi;
-    bool rt = true;
-    if (pass == 0) {
-      d = 2 - (hl >> 3);
-      m = (hl >> 2 & 1) ? 2 : 0;
-    } else {
-      d = hl >> 2;
-      m = 1;
-      rt = hl < 12;
-    }
-    ga = hl & 1;
-    gb = (hl & 3) >> 1;
-    vi = 12 + d;
-    if (pass && !rt) {
-      if (hl < 16) {  // p row: -int psi_k div u
-        out[SLOT_P + hl - 12] = RES && A.mode == 1 ? 0.0 : -S.dq[hl - 12];
-        continue;
-      }
-      vi = 16;
-    }
-    double F[3][3], G[3][3];
+  double w[3];
+  w[0] = dot3(tz.g, r + 6, 9 * ROW);
+  w[1] = dot3(tz.g, r + 7, 9 * ROW);
+  w[2] = dot3(tz.b, r + 8, 9 * ROW) + dot3(tz.d, r + 9, 9 * ROW);
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        const double xt = gauss_x(t);
-        if (!rt) {  // dQ1 vertex hl - 16
-          F[a][t] = ((hl - 16) >> a & 1) ? xt : 1.0 - xt;
-          G[a][t] = 0.0;
-        } else if (a == d) {
-          F[a][t] = q2_val(m, t);
-          G[a][t] = q2_der(m, t);
-        } else {
-          const bool low = a == (d == 0 ? 1 : 0);  // the lower of the two tangential axes
-          F[a][t] = G[a][t] = g2_val(low ? ga : gb, t);
-        }
-      }
-    double r = 0.0;
-#pragma unroll
-    for (int c2 = 0; c2 < 3; ++c2) {
-      double t0 = 0.0, t1 = 0.0;
-#pragma unroll
-      for (int c1 = 0; c1 < 3; ++c1) {
-        double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-        for (int c0 = 0; c0 < 3; ++c0) {
-          const double *f = S.fl[c0 + 3 * c1 + 9 * c2];
-          s0 += F[0][c0] * f[vi];
-          s1 += G[0][c0] * f[15];
-        }
-        t0 += F[1][c1] * s0;
-        t1 += G[1][c1] * s1;
-      }
-      r += F[2][c2] * t0 + G[2][c2] * t1;
-    }
-    if (!rt) {
-      out[SLOT_PHI + hl - 16] = TRANS ? -ph.sigma * r : -r;
-      continue;
-    }
-    const int row = pass == 0 ? hl : 24 + hl;
-    if (UJ) {  // thin-wall faces: their own four rows, every current dof of the cell
-      for (int e = A.cfptr[c]; e < A.cfptr[c + 1]; ++e) {
+  for (int a = 0; a < 3; ++a) {
+    const int m = d[a], ga = a == 0 ? d[1] : d[0], gb = a == 2 ? d[1] : d[2];
+    if (ga > 1 || gb > 1) continue;  // spare lanes of this axis
+    const int face = 2 * (2 - a) + (m >> 1);
+    const int row = m == 1 ? 24 + 4 * a + ga + 2 * gb : 4 * face + ga + 2 * gb;
+    double t = w[a];
+    if (UJ)  // thin-wall faces: their own four rows, every current dof of the cell
+      for (int e = e0; e < e1; ++e) {
         const int f = A.cface[e], lf = A.flf[f];
         const double *K = A.fK + (int64_t)f * 4 * NJ;
-        if (!TRANS && (row >> 2) == lf && !(RES && A.mode == 1)) {
-          double t = RES ? A.fc[4 * f + (row & 3)] : 0.0;
+        if (!TRANS && m != 1 && face == lf && !(RES && A.mode == 1)) {
+          if (RES) t += A.fc[4 * f + (row & 3)];
           for (int b = 0; b < NJ; ++b) t += K[(row & 3) * NJ + b] * S.x[OFF_J + b];
-          r += t;
         } else if (TRANS) {
-          for (int a = 0; a < 4; ++a) r += K[a * NJ + row] * S.x[OFF_J + 4 * lf + a];
+          for (int k = 0; k < 4; ++k) t += K[k * NJ + row] * S.x[OFF_J + 4 * lf + k];
         }
       }
-    }
-    if (pass == 0) r *= S.sg[hl >> 2];
-    out[SLOT_J + row] = r;
+    if (m != 1) t *= S.sg[face];
+    out[SLOT_J + row] = t;
   }
 }
 
@@ -485,7 +511,7 @@ __global__ __launch_bounds__(64) void k_cell_op(CellOpArgs A, MhdPhys ph, const 
 __global__ __launch_bounds__(64) void k_cell_state(int ncells, const double *__restrict__ xyz,
                                                    const int32_t *__restrict__ dofs, const double *__restrict__ dir,
                                                    const double *__restrict__ x, double *__restrict__ state) {
-  __shared__ double xs[2][NU], X[2][24];
+  __shared__ double xs[2][NU], X[2][24], fl[2][NQ * 9];
   const int half = threadIdx.x >> 5, hl = threadIdx.x & 31;
   const int c = blockIdx.x * 2 + half;
   if (c < ncells) {
@@ -496,18 +522,19 @@ __global__ __launch_bounds__(64) void k_cell_state(int ncells, const double *__r
     if (hl < 24) X[half][hl] = xyz[(int64_t)c * 24 + hl];
   }
   __syncthreads();
+  const int q = hl < NQ ? hl : NQ - 1;
+  const int d[3] = {q % 3, (q / 3) % 3, q / 9};
+  double fw[3][4], V[3], dv;
+  fields_forward<false>(xs[half], nullptr, fl[half], 9, d, hl < NQ, fw, V, dv);
   if (c >= ncells || hl >= NQ) return;
-  const double px = gauss_x(hl % 3), py = gauss_x((hl / 3) % 3), pz = gauss_x(hl / 9);
-  const Axis ax(hl % 3), ay((hl / 3) % 3), az(hl / 9);
   double J[9], Ji[9];
-  tri_jacobian(X[half], px, py, pz, J);
+  tri_jacobian(X[half], gauss_x(d[0]), gauss_x(d[1]), gauss_x(d[2]), J);
   inv3(J, Ji);
   double *o = state + (int64_t)c * 12 * NQ + hl;
   for (int k = 0; k < 3; ++k) {
-    double f, r0, r1, r2;
-    q2_eval(xs[half] + 27 * k, ax, ay, az, f, r0, r1, r2);
-    o[k * NQ] = f;
-    for (int i = 0; i < 3; ++i) o[(3 + 3 * i + k) * NQ] = Ji[i] * r0 + Ji[3 + i] * r1 + Ji[6 + i] * r2;
+    o[k * NQ] = fw[k][0];
+    for (int i = 0; i < 3; ++i)
+      o[(3 + 3 * i + k) * NQ] = Ji[i] * fw[k][1] + Ji[3 + i] * fw[k][2] + Ji[6 + i] * fw[k][3];
   }
 }
 
