@@ -368,7 +368,7 @@ void mhd_destroy(mhd_ctx *c) {
                   c->d_rowptr, c->d_colind, c->d_rank, c->d_val, c->d_tperm, c->d_ref, c->d_fref, c->d_x, c->d_r,
                   c->d_color_cells, c->d_crow, c->d_centry, c->d_ebuf, c->d_rbuf, c->d_skel_dofs, c->d_skel_K,
                   c->d_srow, c->d_sentry, c->d_skel_rank, c->d_skel_res, c->d_gslot, c->d_minv, c->d_state, c->d_cfptr,
-                  c->d_cface, c->d_fK, c->d_fc};
+                  c->d_cface, c->d_fK, c->d_fc, c->d_sbuf};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
@@ -443,15 +443,13 @@ int mhd_jacobian_d(mhd_ctx *c, const double *d_x, double *d_val, void *stream) {
   // into the context's own storage: the Jacobian mhd_precond_setup factors,
   // with its state (the coarse levels' injected states come from it)
   if (d_x != c->d_x) MHD_HIP(hipMemcpyAsync(c->d_x, d_x, sizeof(double) * c->n, hipMemcpyDeviceToDevice, s));
-  int rc = mhd_launch_jacobian(c, c->d_x, c->d_val, s);
-  c->jac_valid = rc == 0;
-  return rc;
+  return mhd_assemble_own(c, s);
 }
 
 int mhd_spmv_d(mhd_ctx *c, const double *d_x, double *d_y, void *stream) {
   if (!c || !d_x || !d_y) return -1;
   MHD_HIP(hipSetDevice(c->device));
-  return mhd_launch_spmv(c, c->d_val, d_x, d_y, stream ? (hipStream_t)stream : c->stream);
+  return mhd_launch_spmv(c, d_x, d_y, stream ? (hipStream_t)stream : c->stream);
 }
 
 int mhd_cell_integrals(mhd_ctx *c, const double *x, double *out) {
@@ -484,8 +482,7 @@ int mhd_jacobian(mhd_ctx *c, const double *x, double *nzval) {
   if (!c || !x || !nzval) return -1;
   MHD_HIP(hipSetDevice(c->device));
   MHD_HIP(hipMemcpyAsync(c->d_x, x, sizeof(double) * c->n, hipMemcpyHostToDevice, c->stream));
-  int rc = mhd_launch_jacobian(c, c->d_x, c->d_val, c->stream);
-  c->jac_valid = rc == 0;
+  int rc = mhd_assemble_own(c, c->stream);
   if (rc) return rc;
   if (!c->d_tperm) {
     MHD_HIP(hipMalloc(&c->d_tperm, sizeof(int64_t) * std::max<int64_t>(c->nnz, 1)));

@@ -621,7 +621,8 @@ int launch_op(mhd_ctx *c, const T *x, const T *v, T *y, int64_t rows, double *bu
   A.out = buf;
   A.scale = scale;
   A.mode = mode;
-  hipLaunchKernelGGL((k_cell_op<OP, TRANS, T>), dim3((unsigned)((c->ncells + 1) / 2)), dim3(64), 0, s, A, c->phys, x);
+  hipLaunchKernelGGL((k_cell_op<OP, TRANS, T>), dim3((unsigned)((c->ncells + 1) / 2)), dim3(64), 0, s, A,
+                     OP == OP_RES ? c->phys : c->jac_phys, x);
   const dim3 g((unsigned)((rows + 255) / 256));
   const double rs = TRANS ? 1.0 / scale : 1.0;
   if (v)
@@ -654,8 +655,8 @@ int mhd_cellop_residual(mhd_ctx *c, const double *d_x, double *d_r, double *buf,
 }
 
 int mhd_cellop_state(mhd_ctx *c, const double *d_x, hipStream_t s) {
-  if (c->phys.convection == 0) return 0;
   if (!c->d_state) MHD_HIP(hipMalloc(&c->d_state, sizeof(double) * (size_t)c->ncells * 12 * NQ));
+  if (c->phys.convection == 0) return 0;
   hipLaunchKernelGGL(k_cell_state, dim3((unsigned)((c->ncells + 1) / 2)), dim3(64), 0, s, c->ncells, c->d_xyz,
                      c->d_dofs, c->d_dir, d_x, c->d_state);
   MHD_HIP(hipGetLastError());
@@ -663,18 +664,19 @@ int mhd_cellop_state(mhd_ctx *c, const double *d_x, hipStream_t s) {
 }
 
 template <class T>
-int mhd_cellop_apply(mhd_ctx *c, int op, bool trans, double scale, const T *x, const T *v, T *y, hipStream_t s) {
+int mhd_cellop_apply(mhd_ctx *c, int op, bool trans, double scale, const T *x, const T *v, T *y, double *buf,
+                     hipStream_t s) {
   const int64_t rows = op == MHD_OP_FULL ? c->n : (int64_t)c->nfree[0] + c->nfree[2];
-  if (!c->d_rbuf) MHD_HIP(hipMalloc(&c->d_rbuf, sizeof(double) * (size_t)c->ncells * NDOF));
   if (op == MHD_OP_FULL)
-    return trans ? launch_op<OP_FULL, true, T>(c, x, v, y, rows, c->d_rbuf, 0, scale, s)
-                 : launch_op<OP_FULL, false, T>(c, x, v, y, rows, c->d_rbuf, 0, 1.0, s);
+    return trans ? launch_op<OP_FULL, true, T>(c, x, v, y, rows, buf, 0, scale, s)
+                 : launch_op<OP_FULL, false, T>(c, x, v, y, rows, buf, 0, 1.0, s);
   if (op == MHD_OP_UJ)
-    return trans ? launch_op<OP_UJ, true, T>(c, x, v, y, rows, c->d_rbuf, 0, scale, s)
-                 : launch_op<OP_UJ, false, T>(c, x, v, y, rows, c->d_rbuf, 0, 1.0, s);
-  return trans ? launch_op<OP_PPHI, true, T>(c, x, v, y, rows, c->d_rbuf, 0, scale, s)
-               : launch_op<OP_PPHI, false, T>(c, x, v, y, rows, c->d_rbuf, 0, 1.0, s);
+    return trans ? launch_op<OP_UJ, true, T>(c, x, v, y, rows, buf, 0, scale, s)
+                 : launch_op<OP_UJ, false, T>(c, x, v, y, rows, buf, 0, 1.0, s);
+  return trans ? launch_op<OP_PPHI, true, T>(c, x, v, y, rows, buf, 0, scale, s)
+               : launch_op<OP_PPHI, false, T>(c, x, v, y, rows, buf, 0, 1.0, s);
 }
-template int mhd_cellop_apply<double>(mhd_ctx *, int, bool, double, const double *, const double *, double *,
+template int mhd_cellop_apply<double>(mhd_ctx *, int, bool, double, const double *, const double *, double *, double *,
                                       hipStream_t);
-template int mhd_cellop_apply<float>(mhd_ctx *, int, bool, double, const float *, const float *, float *, hipStream_t);
+template int mhd_cellop_apply<float>(mhd_ctx *, int, bool, double, const float *, const float *, float *, double *,
+                                     hipStream_t);

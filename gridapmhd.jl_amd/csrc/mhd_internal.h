@@ -98,6 +98,7 @@ struct mhd_ctx {
   uint16_t *d_rank = nullptr;     // [ncells][NENT] rank of each touched entry inside its row
   double *d_val = nullptr;        // [nnz] CSR values of the last Jacobian assembled into the context
   bool jac_valid = false;         // d_val holds A(d_x): what mhd_precond_setup factors
+  MhdPhys jac_phys{};             // the parameters it was assembled with
   double pivot_tau = 0.03;        // threshold of a diagonal pivot in the patch inversions
   int64_t *d_tperm = nullptr;     // [nnz] CSR position of the transposed entry (CSC export)
   mhd::RefTables *d_ref = nullptr;
@@ -128,7 +129,10 @@ struct mhd_ctx {
   // cell-wise application of the form (mhd_cellop.hip)
   int32_t *d_gslot = nullptr;         // [crow[n]] element-result slots of every dof's holders
   double *d_minv = nullptr;           // [ncells][16] inverse dP1 mass matrices
-  double *d_state = nullptr;          // [ncells][12][27] u0, grad u0 of the products' linearisation point
+  double *d_state = nullptr;          // [ncells][12][27] u0, grad u0 of the Jacobian in d_val
+  double *d_sbuf = nullptr;           // [ncells][NDOF] element results of mhd_spmv_d
+  hipStream_t sbuf_stream = nullptr;  // the one stream whose mhd_spmv_d calls use it
+  bool sbuf_bound = false;
   int32_t *d_cfptr = nullptr, *d_cface = nullptr;  // thin-wall faces of every cell
   double *d_fK = nullptr;             // [nfaces][4][36] thin-wall face matrices (without orientation signs)
   double *d_fc = nullptr;             // [nfaces][4] their constant parts (-jw)
@@ -192,17 +196,22 @@ enum {
 };
 void mhd_solver_free(mhd_ctx *c);
 
-// Cell-wise application (mhd_cellop.hip).  The products use the state of the
-// last mhd_cellop_state and the context's parameters: y = A x, or y = v - A x
+// The Jacobian at d_x into the context's own values, with what the products
+// without the matrix need of it (state, parameters).
+int mhd_assemble_own(mhd_ctx *c, hipStream_t s);
+
+// Cell-wise application (mhd_cellop.hip).  The products are those of the
+// Jacobian last assembled by mhd_assemble_own: y = A x, or y = v - A x
 // (v not null), on all rows (MHD_OP_FULL), of the [u,j] block (MHD_OP_UJ) or of
 // the (u,j) rows' p and phi columns (MHD_OP_PPHI); `trans`: of D^-1 A^T D with
-// D = scale on the j and phi dofs.  No skeleton term.
+// D = scale on the j and phi dofs.  No skeleton term.  buf: [ncells][NDOF].
 enum { MHD_OP_FULL = 1, MHD_OP_UJ = 2, MHD_OP_PPHI = 3 };
 int mhd_cellop_build(mhd_ctx *c);
 int mhd_cellop_residual(mhd_ctx *c, const double *d_x, double *d_r, double *buf, int mode, hipStream_t s);
 int mhd_cellop_state(mhd_ctx *c, const double *d_x, hipStream_t s);
 template <class T>
-int mhd_cellop_apply(mhd_ctx *c, int op, bool trans, double scale, const T *x, const T *v, T *y, hipStream_t s);
+int mhd_cellop_apply(mhd_ctx *c, int op, bool trans, double scale, const T *x, const T *v, T *y, double *buf,
+                     hipStream_t s);
 
 // Launchers (mhd_assembly.hip)
 int mhd_build_face_matrices(mhd_ctx *c);
@@ -210,7 +219,7 @@ int mhd_launch_residual(mhd_ctx *c, const double *d_x, double *d_r, hipStream_t 
 int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_t s);
 int mhd_build_rank_map(mhd_ctx *c);
 int mhd_build_tperm(mhd_ctx *c);
-int mhd_launch_spmv(mhd_ctx *c, const double *d_val, const double *d_x, double *d_y, hipStream_t s);
+int mhd_launch_spmv(mhd_ctx *c, const double *d_x, double *d_y, hipStream_t s);
 int mhd_launch_cell_integrals(mhd_ctx *c, const double *d_x, double *d_out, hipStream_t s);
 int mhd_launch_residual_mode(mhd_ctx *c, const double *d_x, double *d_r, hipStream_t s, int mode);
 int mhd_launch_transpose_values(mhd_ctx *c, const double *d_val, double *d_val_t, hipStream_t s);

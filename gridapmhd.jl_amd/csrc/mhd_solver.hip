@@ -2083,7 +2083,7 @@ int a11_product(mhd_ctx *c, const T *x, const T *v, T *y, int prec) {
   if (S->matfree) {
     count(c, prec == 0 ? OP_SPMV64 : OP_SPMV32, (double)S->nnz11);
     return mhd_cellop_apply<T>(c, MHD_OP_UJ, S->transposed, op_scale(c), x, MODE == 3 ? v : (const T *)nullptr, y,
-                               c->stream);
+                               c->d_rbuf, c->stream);
   }
   constexpr int LPG = 16;
   const int grid = (int)((S->ngroups11 * LPG + 255) / 256);
@@ -2104,7 +2104,7 @@ int full_product(mhd_ctx *c, const double *x, double *y) {
   if (S->matfree) {
     count(c, OP_SPMV64, (double)c->nnz);
     return mhd_cellop_apply<double>(c, MHD_OP_FULL, S->transposed, op_scale(c), x, (const double *)nullptr, y,
-                                    c->stream);
+                                    c->d_rbuf, c->stream);
   }
   constexpr int LPG = 16;
   const int grid = (int)((S->ngroups * LPG + 255) / 256);
@@ -2273,7 +2273,8 @@ int precond(mhd_ctx *c, const double *v, double *z, int prec) {
   double *rhs1 = prec == 0 ? (double *)S->r1 : S->t1;
   count(c, OP_SPMV64, (double)S->nnz1x);
   if (S->matfree) {
-    if ((rc = mhd_cellop_apply<double>(c, MHD_OP_PPHI, S->transposed, op_scale(c), z, v, rhs1, c->stream))) return rc;
+    if ((rc = mhd_cellop_apply<double>(c, MHD_OP_PPHI, S->transposed, op_scale(c), z, v, rhs1, c->d_rbuf,
+                                       c->stream))) return rc;
   } else {
     constexpr int LPR = 16;
     hipLaunchKernelGGL((k_spmv_seg<double, double, double, LPR, 2>), dim3((unsigned)((S->n1 * LPR + 255) / 256)),
@@ -2439,7 +2440,7 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     S->alpha_phi = aphi;
   }
   if (S->matfree) {
-    if ((rc = mhd_cellop_state(c, d_state, c->stream))) return rc;
+    if (!c->d_rbuf) MHD_HIP(hipMalloc(&c->d_rbuf, sizeof(double) * (size_t)c->ncells * NDOF));
   } else if (prec >= 1)
     hipLaunchKernelGGL((k_convert<double, float>), dim3(nblocks(c->nnz)), dim3(TB), 0, c->stream, c->nnz, c->d_val,
                        S->d_val32);
@@ -2453,7 +2454,7 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
   hipLaunchKernelGGL(k_state_restrict, dim3(nblocks(cc->n)), dim3(TB), 0, cs, cc->n, L->nuc, L->d_Rrow, L->d_Rcol,
                      L->d_Rval, d_state, cc->d_x);
   MHD_HIP(hipGetLastError());
-  if ((rc = mhd_launch_jacobian(cc, cc->d_x, cc->d_val, cs))) {
+  if ((rc = mhd_assemble_own(cc, cs))) {
     c->err = "coarse level: " + cc->err;
     return rc;
   }
@@ -2936,8 +2937,7 @@ int linear_solve(mhd_ctx *c, const double *x_state, const double *rhs, double *l
   };
   MHD_HIP(hipMemcpyAsync(c->d_x, x_state, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
   double t = now();
-  if ((rc = mhd_launch_jacobian(c, c->d_x, c->d_val, c->stream))) return finish(rc);
-  c->jac_valid = true;
+  if ((rc = mhd_assemble_own(c, c->stream))) return finish(rc);
   if (transpose && hipMalloc(&d_valT, sizeof(double) * std::max<int64_t>(c->nnz, 1)) != hipSuccess) {
     c->err = "out of device memory for A^T";
     d_valT = nullptr;
@@ -3028,8 +3028,7 @@ int mhd_newton_solve(mhd_ctx *c, double *x_host, const mhd_solver_opts *o, mhd_s
   while (it < o->max_newton) {
     if (rn <= std::max(o->atol, o->rtol * r0)) break;
     t = now();
-    if ((rc = mhd_launch_jacobian(c, c->d_x, c->d_val, c->stream))) return rc;
-    c->jac_valid = true;
+    if ((rc = mhd_assemble_own(c, c->stream))) return rc;
     MHD_HIP(hipStreamSynchronize(c->stream));
     info->t_jacobian += now() - t;
     t = now();

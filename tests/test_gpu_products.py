@@ -38,3 +38,38 @@ def test_linear_solves_satisfy_the_oracle_system(nc, convection, stab, levels, p
             assert res < 1e-9
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("nc,convection,stab", [((3, 3, 3), "newton", 0.0), ((5, 3, 1), "picard", 0.0),
+                                                ((2, 2, 2), "none", 0.0), ((3, 2, 3), "newton", 0.1)])
+def test_spmv_is_the_assembled_jacobian(nc, convection, stab, orc_mod):
+    """mhd_spmv_d on the first stream that calls it (the form applied cell by
+    cell) and on another (the matrix streamed): both are the Jacobian as it was
+    assembled, whatever parameters and states the context has seen since."""
+    import ctypes
+    import gridapmhd_amd as g
+    from devmem import DeviceArray, hip
+    from gridapmhd_amd import adjoint
+    sp, phys = adjoint.inlet_duct(nc, 20.0, 5.0, 0.05, convection=convection, jitter=0.15)
+    phys = dict(phys, stab_mu=stab)
+    rng = np.random.default_rng(8)
+    x, v = 0.3 * rng.standard_normal(sp.ndofs), rng.standard_normal(sp.ndofs)
+    ref = orc_mod.Oracle(cases.problem_dict(sp, phys)).jacobian(x).tocsr() @ v
+    other = ctypes.c_void_p()
+    ctx = g._lib.context_from_spaces(sp, phys)
+    try:
+        assert hip().hipStreamCreate(ctypes.byref(other)) == 0
+        dx, dv, dy = DeviceArray.from_numpy(x), DeviceArray.from_numpy(v), DeviceArray.from_numpy(np.zeros(sp.ndofs))
+        ctx.jacobian_d(dx.ptr)
+        ctx.residual(2.0 * x)                                      # another state in the context
+        ctx.set_params(dict(phys, gamma=3.0, alpha=0.2, convection="newton"))
+        hip().hipDeviceSynchronize()
+        for stream in (0, other.value, 0):
+            dy.copy_from(np.full(sp.ndofs, np.nan))
+            ctx.spmv_d(dv.ptr, dy.ptr, stream)
+            err = np.linalg.norm(dy.numpy() - ref) / np.linalg.norm(ref)
+            print(f"[spmv] {nc} {convection} stab={stab} stream={'own' if not stream else 'other'}: {err:.2e}", flush=True)
+            assert err < 1e-13
+    finally:
+        ctx.close()
+        hip().hipStreamDestroy(other)
