@@ -672,31 +672,37 @@ __global__ __launch_bounds__(CND_T) void k_condense(int ncells, const int32_t *_
 }
 
 // Condensed patch matrices S_P (column-major, identity on the padding): the
-// CSR rows of the patch's dofs restricted to them (each wave takes whole rows,
-// its lanes binary-search the columns among the sorted ids), minus A_bi E of
-// every condensed cell around the vertex, cell by cell in a fixed order.  One
-// 1024-thread workgroup per patch.  LDSM: the matrix is built in LDS
-// (129 x 129 FP64, 133 of the CU's 160 KB) and written once, coalesced; larger
-// patches are built in place in A.  7.5 ms for 33,800 patches (the full
-// 225 x 225 matrices, scattered into cleared memory, took 18 ms).
-template <bool LDSM>
+// entries of A between the patch's dofs, minus A_bi E of every condensed cell
+// around the vertex, cell by cell in a fixed order.  Two dofs of a patch couple
+// only through cells that hold both, and those are around the vertex, so the
+// entries are taken cell by cell through the rank map, without a search (10 K
+// entries per patch, where scanning the CSR rows visits 32 K columns).  SKEL:
+// the skeleton term couples dofs across cells; the rows are scanned then, each
+// by a wave whose lanes binary-search the columns among the sorted ids.  One
+// 1024-thread workgroup per patch.  LDSM: the matrix is built in LDS (129 x 129
+// FP64, 133 of the CU's 160 KB) and written once, coalesced; larger patches are
+// built in place in A.  BUILDFIG
+template <bool LDSM, bool SKEL>
 __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__restrict__ psize,
                                                       const int32_t *__restrict__ pidx,
                                                       const int32_t *__restrict__ pcptr,
                                                       const int32_t *__restrict__ pcell,
                                                       const int64_t *__restrict__ rowptr,
                                                       const int32_t *__restrict__ colind,
+                                                      const uint16_t *__restrict__ rank,
                                                       const double *__restrict__ val,
                                                       const int32_t *__restrict__ dofs,
                                                       const int32_t *__restrict__ ifirst, int dups,
                                                       const double *__restrict__ E64,
                                                       const double *__restrict__ B64, double *__restrict__ A) {
   constexpr int NS = LDSM ? GJSmall::NMAX : 1;
+  constexpr int NUJ = NB + NI;  // [u,j] dofs of a cell
+  constexpr int CB = 8;         // cells in work together: 128 threads each
   __shared__ double lmat[NS * NS];
   __shared__ double Bs[NB][NI + 1], Es[NB][NI + 1];
   __shared__ int32_t sid[256];
-  __shared__ int32_t lpos[NB], lsel[NB];
-  __shared__ int m;
+  __shared__ uint8_t lpos[CB][NUJ], lsel[CB][NUJ];
+  __shared__ int m[CB];
   const int pch = blockIdx.x, t = threadIdx.x;
   const int sz = psize[pch];
   const int32_t *ids = pidx + (int64_t)pch * PS;
@@ -706,62 +712,112 @@ __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__r
   for (int e = t; e < PS * PS; e += 1024) M[e] = 0.0;
   __syncthreads();
   for (int k = sz + t; k < PS; k += 1024) M[k + k * PS] = 1.0;
-  if (sz > 0) {
-    const int32_t first = sid[0], last = sid[sz - 1];
-    auto find = [&](int32_t id) {
-      int lo = 0, hi = sz;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (sid[mid] < id) lo = mid + 1;
-        else hi = mid;
-      }
-      return lo < sz && sid[lo] == id ? lo : -1;
-    };
+  const int32_t first = sz > 0 ? sid[0] : 0, last = sz > 0 ? sid[sz - 1] : -1;
+  auto find = [&](int32_t id) {
+    if (id < first || id > last) return -1;
+    int lo = 0, hi = sz;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (sid[mid] < id) lo = mid + 1;
+      else hi = mid;
+    }
+    return lo < sz && sid[lo] == id ? lo : -1;
+  };
+  if (SKEL) {
     const int wave = t >> 6, lane = t & 63;
     for (int a = wave; a < sz; a += 16) {
       const int32_t row = sid[a];
       const int64_t e = rowptr[row + 1];
       for (int64_t p = rowptr[row] + lane; p < e; p += 64) {
-        const int32_t col = colind[p];
-        if (col < first || col > last) continue;
-        const int b = find(col);
+        const int b = find(colind[p]);
         if (b >= 0) M[a + b * PS] = val[p];
       }
     }
-    for (int q = pcptr[pch]; q < pcptr[pch + 1]; ++q) {
-      const int c = pcell[q];
-      if (ifirst[c] < 0) continue;  // uniform
-      __syncthreads();  // the rows of the first round; the previous cell's tiles
-      if (t == 0) m = 0;
-      __syncthreads();
-      if (t < NB) {
+  }
+  const int q0 = pcptr[pch], q1 = pcptr[pch + 1];
+  // the dofs of the cells qb .. qb + CB - 1 that the patch holds: local index
+  // and position (the order of the lists changes no result)
+  auto locate = [&](int qb) {
+    __syncthreads();  // the previous lists are done with
+    if (t < CB) m[t] = 0;
+    __syncthreads();
+    const int k = t >> 7, l = t & 127;
+    if (qb + k < q1) {
+      const int c = pcell[qb + k];
+      if (l < (ifirst[c] >= 0 ? NB : NUJ)) {
         const int32_t *cd = dofs + (int64_t)c * NDOF;
-        const int32_t id = cd[bdof_local(t)];
+        const int32_t id = cd[bdof_local(l)];
         int pos = id >= 0 ? find(id) : -1;
         if (dups && pos >= 0)
-          for (int l = 0; l < t; ++l)
-            if (cd[bdof_local(l)] == id) pos = -1;
-        if (pos >= 0) {  // the order of the list changes no result: every entry of M is updated once
-          const int k = atomicAdd(&m, 1);
-          lpos[k] = pos;
-          lsel[k] = t;
+          for (int o = 0; o < l; ++o)
+            if (cd[bdof_local(o)] == id) pos = -1;
+        if (pos >= 0) {
+          const int at = atomicAdd(&m[k], 1);
+          lpos[k][at] = (uint8_t)pos;
+          lsel[k][at] = (uint8_t)l;
+        }
+      }
+    }
+    __syncthreads();
+  };
+  // entries of A, all cells at once (an entry of two cells is written twice,
+  // with the same value)
+  if (!SKEL)
+    for (int qb = q0; qb < q1; qb += CB) {
+      locate(qb);
+      const int k = t >> 7, mk = m[k];
+      if (qb + k < q1) {
+        const uint16_t *rk = rank + (int64_t)pcell[qb + k] * NENT;
+        for (int e = t & 127; e < mk * mk; e += 128) {
+          const int ka = e / mk, kb = e - ka * mk;
+          const int la = lsel[k][ka], lb = lsel[k][kb], pa = lpos[k][ka], pb = lpos[k][kb];
+          // u rows hold [u p j], j rows [u j phi]
+          const int ent = la < NU ? la * ROWS_U_LEN + (lb < NU ? lb : lb + NP) : E_J + (la - NU) * ROWS_J_LEN + lb;
+          M[pa + pb * PS] = val[rowptr[sid[pa]] + rk[ent]];
+        }
+      }
+    }
+  // minus A_bi E, cell after cell; the next cell's couplings are loaded meanwhile
+  for (int qb = q0; qb < q1; qb += CB) {
+    if (SKEL || q1 - q0 > CB) locate(qb);
+    else __syncthreads();  // the entries are in place, the lists still hold
+    const int nk = min(CB, q1 - qb);
+    constexpr int PF = (NB * NI + 1023) / 1024;
+    double bn[PF], en[PF];
+    auto fetch = [&](int k) {
+      const int64_t oc = (int64_t)pcell[qb + k] * NB * NI;
+      const int n = ifirst[pcell[qb + k]] >= 0 ? m[k] * NI : 0;
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const int e = t + 1024 * u;
+        if (e < n) {
+          const int64_t at = oc + lsel[k][e / NI] * NI + e % NI;
+          bn[u] = B64[at];
+          en[u] = E64[at];
+        }
+      }
+    };
+    fetch(0);
+    for (int k = 0; k < nk; ++k) {
+      const int mk = ifirst[pcell[qb + k]] >= 0 ? m[k] : 0;  // uniform
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const int e = t + 1024 * u;
+        if (e < mk * NI) {
+          Bs[e / NI][e % NI] = bn[u];
+          Es[e / NI][e % NI] = en[u];
         }
       }
       __syncthreads();
-      const int64_t oc = (int64_t)c * NB * NI;
-      for (int e = t; e < m * NI; e += 1024) {
-        const int k = e / NI, i = e % NI;
-        Bs[k][i] = B64[oc + lsel[k] * NI + i];
-        Es[k][i] = E64[oc + lsel[k] * NI + i];
-      }
-      __syncthreads();
-      for (int e = t; e < m * m; e += 1024) {
-        const int ka = e % m, kb = e / m;
+      if (k + 1 < nk) fetch(k + 1);
+      for (int e = t; e < mk * mk; e += 1024) {
+        const int kb = e / mk, ka = e - kb * mk;
         double s = 0.0;
 #pragma unroll
         for (int i = 0; i < NI; ++i) s += Bs[ka][i] * Es[kb][i];
-        M[lpos[ka] + lpos[kb] * PS] -= s;
+        M[lpos[k][ka] + lpos[k][kb] * PS] -= s;
       }
+      __syncthreads();
     }
   }
   if (LDSM) {
@@ -1135,77 +1191,89 @@ __device__ __forceinline__ void gj_argmax(double &best, double &bval, int &bi, i
 
 // ---- diagonal pivots, rotating tile ----------------------------------------
 
-// Step k = 16 rb + tq (column block cb = k / TC).  colbuf and rowbuf are
-// kept in register order: slot tr + 16 i holds the row of register row i,
-// slot tc + TC j the column of register column j; slot NL is row / column NL.
+// Step k = 16 rb + tq (column block cb = k / TC).  col and row hold the pivot
+// column and row of the step in register order (slot tr + 16 i: the row of
+// register row i; slot tc + TC j: the column of register column j; slot NL: row
+// / column NL), unscaled.  The lanes that own the next step's column and row
+// write them to the other buffer as soon as they have updated them, so a step
+// has one barrier; the pivot's reciprocal is taken by every thread, and the
+// threshold test of the next pivot is off that path.  rot_r / rot_c: the tile
+// rotates after this step, so the next row / column block is the second one.
 template <class G>
-__device__ __forceinline__ void gjd_step(double (&S)[G::RI][G::RJ], GJShared<G> &L, int t, int tr, int tc, int rb,
-                                         int cb, int tq, double tau) {
+__device__ __forceinline__ void gjd_step(double (&S)[G::RI][G::RJ], GJShared<G> &L, const double *col,
+                                         const double *row, double *ncol, double *nrow, int t, int tr, int tc, int rb,
+                                         int cb, int tq, bool rot_r, bool rot_c) {
   const int k = G::TR * rb + tq, kc = k & (G::TC - 1);
-  // ---- pivot column into colbuf (zeroed in place), threshold test
-  if (tc == kc) {  // 16 lanes of one wave
-    double cmax = 0.0, dia = 0.0;
-#pragma unroll
-    for (int i = 0; i < G::RI; ++i) {
-      const double v = S[i][0];
-      L.colbuf[tr + G::TR * i] = v;
-      S[i][0] = 0.0;
-      // register row i holds row block (i + rb) mod RI: unused rows are the
-      // blocks after rb and the rows of block rb after tq
-      if (i < G::RI - rb && (i > 0 || tr > tq)) cmax = fmax(cmax, fabs(v));
-      if (i == 0) dia = v;
-    }
-    if (tr == 0) {
-      const double v = L.Rl[k];
-      L.colbuf[G::NL] = v;
-      cmax = fmax(cmax, fabs(v));
-    }
-    for (int off = G::TR >> 1; off > 0; off >>= 1) cmax = fmax(cmax, __shfl_xor(cmax, off, G::TR));
-    if (tr == tq) {
-      L.piv = dia;
-      if (!(fabs(dia) >= tau * cmax) || dia == 0.0) atomicCAS(&L.bad, 0, k + 1);
-    }
-  }
-  __syncthreads();
-  // ---- pivot row (register row 0 of lanes tr == tq) into rowbuf, zeroed
-  const double piv = L.piv;
+  const double piv = col[tq];
   const double inv = piv != 0.0 ? 1.0 / piv : 0.0;
-  if (tr == tq) {
-#pragma unroll
-    for (int j = 0; j < G::RJ; ++j) {
-      L.rowbuf[tc + G::TC * j] = (j == 0 && tc == kc) ? inv : S[0][j] * inv;
-      S[0][j] = 0.0;
-    }
-    if (tc == 0) L.rowbuf[G::NL] = L.Cl[k] * inv;
-  }
-  if (t == 0) L.colbuf[tq] = -1.0;  // f'_k: the pivot row (zeroed above) becomes the scaled row
-  __syncthreads();
-  // ---- rank-1 update of every entry: a_ij <- a_ij - f'_i r_j
+  // f'_i = f_i (pivot row: -1), r_j = a_kj / a_kk (pivot column: 1 / a_kk);
+  // a_ij <- a_ij - f'_i r_j with the pivot row and column of a zeroed
   double rv[G::RJ];
 #pragma unroll
-  for (int j = 0; j < G::RJ; ++j) rv[j] = L.rowbuf[tc + G::TC * j];
+  for (int j = 0; j < G::RJ; ++j) rv[j] = row[tc + G::TC * j] * inv;
+  const bool mycol = tc == kc, myrow = tr == tq;
+  if (mycol) rv[0] = inv;
 #pragma unroll
   for (int i = 0; i < G::RI; ++i) {
-    const double f = L.colbuf[tr + G::TR * i];
+    const double f = i == 0 && myrow ? -1.0 : col[tr + G::TR * i];
 #pragma unroll
-    for (int j = 0; j < G::RJ; ++j) S[i][j] = fma(-f, rv[j], S[i][j]);
+    for (int j = 0; j < G::RJ; ++j) {
+      const double a = (j == 0 && mycol) || (i == 0 && myrow) ? 0.0 : S[i][j];
+      S[i][j] = fma(-f, rv[j], a);
+    }
   }
+  const double fl = col[G::NL], rl = row[G::NL] * inv;
   if (t < G::NMAX) {  // row NL, physical column t
     int slot = G::NL;
     if (t < G::NL) {
       const int blk = t / G::TC - cb;
       slot = (t & (G::TC - 1)) + G::TC * (blk < 0 ? blk + G::RJ : blk);
     }
-    const double old = t == k ? 0.0 : L.Rl[t];
-    L.Rl[t] = fma(-L.colbuf[G::NL], L.rowbuf[slot], old);
+    L.Rl[t] = fma(-fl, t == k ? inv : row[slot] * inv, t == k ? 0.0 : L.Rl[t]);
   }
   if (t < G::NL) {  // column NL, physical row t
     const int blk = t / G::TR - rb;
     const int slot = (t & (G::TR - 1)) + G::TR * (blk < 0 ? blk + G::RI : blk);
-    const double old = t == k ? 0.0 : L.Cl[t];
-    L.Cl[t] = fma(-L.colbuf[slot], L.rowbuf[G::NL], old);
+    L.Cl[t] = fma(t == k ? 1.0 : -col[slot], rl, t == k ? 0.0 : L.Cl[t]);
+  }
+  // next step: its column (register column 0, or 1 before a rotation) and row
+  const int kn = k + 1;
+  if (kn < G::NL) {
+    if (tc == (kn & (G::TC - 1))) {
+#pragma unroll
+      for (int i = 0; i < G::RI; ++i) {
+        const int i1 = i + 1 < G::RI ? i + 1 : 0;  // every register index a compile-time constant
+        ncol[tr + G::TR * i] = rot_r ? (rot_c ? S[i1][1] : S[i1][0]) : S[i][0];
+      }
+    }
+    if (tr == (kn & (G::TR - 1))) {
+#pragma unroll
+      for (int j = 0; j < G::RJ; ++j) {
+        const int j1 = j + 1 < G::RJ ? j + 1 : 0;
+        nrow[tc + G::TC * j] = rot_r ? (rot_c ? S[1][j1] : S[1][j]) : S[0][j];
+      }
+    }
+    // entries of row / column NL: the threads that have just updated them
+    if (t == kn) {
+      ncol[G::NL] = L.Rl[t];
+      nrow[G::NL] = L.Cl[t];
+    }
   }
   __syncthreads();
+}
+
+// The threshold test of step k's pivot on the column in `col`: 16 lanes.
+// Register row i holds row block (i + rb) mod RI: unused rows are the blocks
+// after rb, the rows of block rb after tq, and row NL.
+template <class G>
+__device__ __forceinline__ void gjd_test(GJShared<G> &L, const double *col, int tr, int rb, int tq, double tau) {
+  double cmax = tr == 0 ? fabs(col[G::NL]) : 0.0;
+#pragma unroll
+  for (int i = 0; i < G::RI; ++i)
+    if (i < G::RI - rb && (i > 0 || tr > tq)) cmax = fmax(cmax, fabs(col[tr + G::TR * i]));
+  for (int off = G::TR >> 1; off > 0; off >>= 1) cmax = fmax(cmax, __shfl_xor(cmax, off, G::TR));
+  const double dia = col[tq];
+  if (tr == tq && (!(fabs(dia) >= tau * cmax) || dia == 0.0)) atomicCAS(&L.bad, 0, G::TR * rb + tq + 1);
 }
 
 template <class G, class OutT>
@@ -1213,15 +1281,34 @@ __global__ __launch_bounds__(G::T) void k_patch_gjd(int PS, int ld, double tau, 
                                                      OutT *__restrict__ out, int16_t *__restrict__ perm,
                                                      int32_t *__restrict__ status, float *__restrict__ pscale) {
   __shared__ GJShared<G> L;
+  __shared__ double buf[2][2][G::NMAX];  // [parity][column, row]
   const int t = threadIdx.x, tr = t % G::TR, tc = t / G::TR;
   const int64_t pch = blockIdx.x;
   double S[G::RI][G::RJ];
   gj_load<G>(S, L, A + pch * PS * PS, PS, t, tr, tc);
   __syncthreads();
+  if (tc == 0)
+#pragma unroll
+    for (int i = 0; i < G::RI; ++i) buf[0][0][tr + G::TR * i] = S[i][0];
+  if (tr == 0)
+#pragma unroll
+    for (int j = 0; j < G::RJ; ++j) buf[0][1][tc + G::TC * j] = S[0][j];
+  if (t == 0) {
+    buf[0][0][G::NL] = L.Rl[0];
+    buf[0][1][G::NL] = L.Cl[0];
+  }
+  __syncthreads();
   for (int cb = 0; cb < G::RJ; ++cb) {
     for (int h = 0; h < G::TC / G::TR; ++h) {
       const int rb = G::TC / G::TR * cb + h;
-      for (int tq = 0; tq < G::TR; ++tq) gjd_step<G>(S, L, t, tr, tc, rb, cb, tq, tau);
+#pragma unroll 2
+      for (int tq = 0; tq < G::TR; ++tq) {
+        const int par = tq & 1;
+        if (tc == G::TC - 1) gjd_test<G>(L, buf[par][0], tr, rb, tq, tau);  // one 16-lane group
+        const bool lr = tq == G::TR - 1;
+        gjd_step<G>(S, L, buf[par][0], buf[par][1], buf[par ^ 1][0], buf[par ^ 1][1], t, tr, tc, rb, cb, tq, lr,
+                    lr && h == G::TC / G::TR - 1);
+      }
       // next row block into register row 0
 #pragma unroll
       for (int j = 0; j < G::RJ; ++j) {
@@ -2350,14 +2437,14 @@ int invert_patches_to(mhd_ctx *c, OutT *inv, float *scale) {
   for (int p0 = 0; p0 < S->npatch; p0 += S->pchunk) {
     const int np = std::min(S->pchunk, S->npatch - p0);
     double *mat = S->d_pscratch;
-    if (S->PS <= GJSmall::NMAX)
-      hipLaunchKernelGGL(k_patch_build<true>, dim3(np), dim3(1024), 0, c->stream, S->PS, S->d_psize + p0,
+    const bool small = S->PS <= GJSmall::NMAX, skel = c->nskel > 0;
+    auto build = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(np), dim3(1024), 0, c->stream, S->PS, S->d_psize + p0,
                          S->d_pidx + (int64_t)p0 * S->PS, S->d_pcptr + p0, S->d_pcell, c->d_rowptr, c->d_colind,
-                         c->d_val, c->d_dofs, S->d_ifirst, dups, S->d_cE64, S->d_cB64, mat);
-    else
-      hipLaunchKernelGGL(k_patch_build<false>, dim3(np), dim3(1024), 0, c->stream, S->PS, S->d_psize + p0,
-                         S->d_pidx + (int64_t)p0 * S->PS, S->d_pcptr + p0, S->d_pcell, c->d_rowptr, c->d_colind,
-                         c->d_val, c->d_dofs, S->d_ifirst, dups, S->d_cE64, S->d_cB64, mat);
+                         c->d_rank, c->d_val, c->d_dofs, S->d_ifirst, dups, S->d_cE64, S->d_cB64, mat);
+    };
+    if (skel) small ? build(k_patch_build<true, true>) : build(k_patch_build<false, true>);
+    else small ? build(k_patch_build<true, false>) : build(k_patch_build<false, false>);
     int16_t *pp = S->d_pperm + (int64_t)p0 * 2 * S->PS;
     int32_t *st = S->d_pstatus + p0;
     OutT *out = inv + p0 * po;
