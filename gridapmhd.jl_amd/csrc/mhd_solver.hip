@@ -681,7 +681,9 @@ __global__ __launch_bounds__(CND_T) void k_condense(int ncells, const int32_t *_
 // by a wave whose lanes binary-search the columns among the sorted ids.  One
 // 1024-thread workgroup per patch.  LDSM: the matrix is built in LDS (129 x 129
 // FP64, 133 of the CU's 160 KB) and written once, coalesced; larger patches are
-// built in place in A.  BUILDFIG
+// built in place in A.  5.1 ms for 33,800 patches; with the rows scanned and the
+// cells taken one after another, each waiting for its loads, 7.5 ms (the full
+// 225 x 225 matrices, scattered into cleared memory, 18 ms).
 template <bool LDSM, bool SKEL>
 __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__restrict__ psize,
                                                       const int32_t *__restrict__ pidx,
@@ -1046,8 +1048,9 @@ __global__ __launch_bounds__(256) void k_cond_inner(int ncells, const int32_t *_
 // rows) and RJ columns (one of every block of TC columns); the last row and
 // column live in LDS.  GJSmall's FP64 tile is 64 values (128 VGPRs) on 256
 // threads, so two to three workgroups share a CU and hide each other's
-// barriers (three per step): 9.6 ms for 33,800 patches, where the full stars
-// took 61 ms on GJLarge's 98 values on 512 threads, one workgroup per CU.
+// barriers (one per step): 12.4 ms for 33,800 patches (13.2 with three barriers
+// per step), where the full stars took 61 ms on GJLarge's 98 values on 512
+// threads, one workgroup per CU.
 //
 // Elimination step k, with the pivot column saved as f and zeroed and the
 // pivot row p saved as r = a_p,: / a_pk (r_k = 1 / a_pk) and zeroed, updates
