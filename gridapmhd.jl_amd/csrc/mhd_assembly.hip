@@ -8,256 +8,19 @@
 // Thin-wall faces (src/weakforms.jl:721-733, residual evaluated at x):
 //   R += int_G tau (s.n)(j.n - jw + cw n.(grad j).n),  J += int_G tau (s.n)(dj.n + cw n.(grad dj).n)
 //
-// One workgroup per cell: quadrature geometry, pushed-forward bases and the
-// state of x at the 27 Gauss points are staged in LDS; the 14913 touched
-// entries of the element matrix are spread over the workgroup in the
-// canonical row-major order of the cell's rank map, so the rank-map reads and
-// the row-local scatter into the CSR values are contiguous.
+// This file: the Jacobian assembly, the thin-wall and skeleton faces, the
+// post-processing integrals; the residual and the matrix-free products are in
+// mhd_cellop.hip.
+#include <algorithm>
 #include <mutex>
 
-#include "mhd_internal.h"
+#include "mhd_cell.h"
 
 using namespace mhd;
 
 namespace {
 
 constexpr int WG = 256;
-
-struct CellLDS {
-  double W[NQ];              // w |det J|
-  union {
-    struct {
-      double Ji[NQ][9];      // (J^-1)[l][i]
-      double Jp[NQ][9];      // J[k][l] / det J
-    };
-    struct {
-      double D[4][NU];       // AL-u: int psi_k div v_b
-      double MD[4][NU];      // AL-u: M^-1 D
-      double Mi[16];         // AL-u: inverse dP1 mass
-      double cu[4];          // AL-u: M^-1 int psi div u
-      double Mq[16];         // AL-u: dP1 mass
-      double dq[4];          // AL-u: int psi div u
-    };
-  };
-  double idet[NQ];           // 1 / det J
-  double xq[NQ][3];          // physical point
-  double q2[NQ][27];         // reference Q2 values
-  double p1[NQ][4];          // reference dP1 values
-  double q1[NQ][8];          // reference dQ1 values
-  double gphi[NQ][27][3];    // physical Q2 gradients
-  double cphi[NQ][27];       // u . grad phi (convective derivative)
-  double psi[NQ][36][3];     // Piola-mapped RT basis (with face signs)
-  double dpsi[NQ][36];       // its divergence
-  double u[NQ][3];           // state of x
-  double gu[NQ][9];          // grad u [i][k] = d u_k / d x_i
-  double wN[NQ][9];          // W alpha d_d u_c  at [3c + d]  (Newton term weights)
-  double p[NQ], jv[NQ][3], divj[NQ], ph[NQ], divu[NQ];
-  double xl[NDOF];
-  double xyz[24];
-  double sg[6];
-  double B[3], f0[3], fx[9], g0[3], gx[9];
-  int64_t rp[NDOF];
-  int32_t g[NDOF];
-};
-
-__device__ inline void inv4(const double *m, double *inv) {
-  // adjugate / determinant of a 4x4 row-major matrix
-  inv[0] = m[5] * m[10] * m[15] - m[5] * m[11] * m[14] - m[9] * m[6] * m[15] + m[9] * m[7] * m[14] + m[13] * m[6] * m[11] - m[13] * m[7] * m[10];
-  inv[4] = -m[4] * m[10] * m[15] + m[4] * m[11] * m[14] + m[8] * m[6] * m[15] - m[8] * m[7] * m[14] - m[12] * m[6] * m[11] + m[12] * m[7] * m[10];
-  inv[8] = m[4] * m[9] * m[15] - m[4] * m[11] * m[13] - m[8] * m[5] * m[15] + m[8] * m[7] * m[13] + m[12] * m[5] * m[11] - m[12] * m[7] * m[9];
-  inv[12] = -m[4] * m[9] * m[14] + m[4] * m[10] * m[13] + m[8] * m[5] * m[14] - m[8] * m[6] * m[13] - m[12] * m[5] * m[10] + m[12] * m[6] * m[9];
-  inv[1] = -m[1] * m[10] * m[15] + m[1] * m[11] * m[14] + m[9] * m[2] * m[15] - m[9] * m[3] * m[14] - m[13] * m[2] * m[11] + m[13] * m[3] * m[10];
-  inv[5] = m[0] * m[10] * m[15] - m[0] * m[11] * m[14] - m[8] * m[2] * m[15] + m[8] * m[3] * m[14] + m[12] * m[2] * m[11] - m[12] * m[3] * m[10];
-  inv[9] = -m[0] * m[9] * m[15] + m[0] * m[11] * m[13] + m[8] * m[1] * m[15] - m[8] * m[3] * m[13] - m[12] * m[1] * m[11] + m[12] * m[3] * m[9];
-  inv[13] = m[0] * m[9] * m[14] - m[0] * m[10] * m[13] - m[8] * m[1] * m[14] + m[8] * m[2] * m[13] + m[12] * m[1] * m[10] - m[12] * m[2] * m[9];
-  inv[2] = m[1] * m[6] * m[15] - m[1] * m[7] * m[14] - m[5] * m[2] * m[15] + m[5] * m[3] * m[14] + m[13] * m[2] * m[7] - m[13] * m[3] * m[6];
-  inv[6] = -m[0] * m[6] * m[15] + m[0] * m[7] * m[14] + m[4] * m[2] * m[15] - m[4] * m[3] * m[14] - m[12] * m[2] * m[7] + m[12] * m[3] * m[6];
-  inv[10] = m[0] * m[5] * m[15] - m[0] * m[7] * m[13] - m[4] * m[1] * m[15] + m[4] * m[3] * m[13] + m[12] * m[1] * m[7] - m[12] * m[3] * m[5];
-  inv[14] = -m[0] * m[5] * m[14] + m[0] * m[6] * m[13] + m[4] * m[1] * m[14] - m[4] * m[2] * m[13] - m[12] * m[1] * m[6] + m[12] * m[2] * m[5];
-  inv[3] = -m[1] * m[6] * m[11] + m[1] * m[7] * m[10] + m[5] * m[2] * m[11] - m[5] * m[3] * m[10] - m[9] * m[2] * m[7] + m[9] * m[3] * m[6];
-  inv[7] = m[0] * m[6] * m[11] - m[0] * m[7] * m[10] - m[4] * m[2] * m[11] + m[4] * m[3] * m[10] + m[8] * m[2] * m[7] - m[8] * m[3] * m[6];
-  inv[11] = -m[0] * m[5] * m[11] + m[0] * m[7] * m[9] + m[4] * m[1] * m[11] - m[4] * m[3] * m[9] - m[8] * m[1] * m[7] + m[8] * m[3] * m[5];
-  inv[15] = m[0] * m[5] * m[10] - m[0] * m[6] * m[9] - m[4] * m[1] * m[10] + m[4] * m[2] * m[9] + m[8] * m[1] * m[6] - m[8] * m[2] * m[5];
-  const double det = m[0] * inv[0] + m[1] * inv[4] + m[2] * inv[8] + m[3] * inv[12];
-  const double id = 1.0 / det;
-  for (int i = 0; i < 16; ++i) inv[i] *= id;
-}
-
-// Load one cell and stage everything the integrands need.  `want_state`
-// evaluates x at the quadrature points (always needed except for a linear
-// Jacobian), `want_al` the zeta_u local projection.
-__device__ void stage_cell(CellLDS &S, int c, const double *__restrict__ xyz, const int32_t *__restrict__ dofs,
-                           const int8_t *__restrict__ sign, const double *__restrict__ dir,
-                           const double *__restrict__ x, const RefTables *__restrict__ T,
-                           const int64_t *__restrict__ rowptr, const MhdPhys &ph, bool want_al) {
-  const int tid = threadIdx.x;
-  if (tid < 24) S.xyz[tid] = xyz[(int64_t)c * 24 + tid];
-  if (tid < 6) S.sg[tid] = sign ? (double)sign[(int64_t)c * 6 + tid] : 1.0;
-  if (tid == 0) {
-    for (int i = 0; i < 3; ++i) {
-      S.B[i] = ph.B[i];
-      S.f0[i] = ph.f0[i];
-      S.g0[i] = ph.g0[i];
-    }
-    for (int i = 0; i < 9; ++i) {
-      S.fx[i] = ph.fx[i];
-      S.gx[i] = ph.gx[i];
-    }
-  }
-  if (tid < NDOF) {
-    const int32_t g = dofs[(int64_t)c * NDOF + tid];
-    S.g[tid] = g;
-    S.xl[tid] = g >= 0 ? x[g] : dir[-g - 1];
-    S.rp[tid] = (g >= 0 && rowptr) ? rowptr[g] : -1;
-  }
-  __syncthreads();
-  // geometry: one thread per quadrature point
-  if (tid < NQ) {
-    const int q = tid;
-    double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, X[3] = {0, 0, 0};
-#pragma unroll
-    for (int v = 0; v < 8; ++v)
-      for (int i = 0; i < 3; ++i) {
-        const double xv = S.xyz[3 * v + i];
-        X[i] += T->q1[q][v] * xv;
-        for (int l = 0; l < 3; ++l) J[i][l] += xv * T->dq1[q][v][l];
-      }
-    const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-    const double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-    const double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-    const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
-    const double id = 1.0 / det;
-    double *Ji = S.Ji[q];
-    Ji[0 * 3 + 0] = c00 * id;
-    Ji[1 * 3 + 0] = c01 * id;
-    Ji[2 * 3 + 0] = c02 * id;
-    Ji[0 * 3 + 1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-    Ji[1 * 3 + 1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-    Ji[2 * 3 + 1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-    Ji[0 * 3 + 2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-    Ji[1 * 3 + 2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-    Ji[2 * 3 + 2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-    for (int k = 0; k < 3; ++k)
-      for (int l = 0; l < 3; ++l) S.Jp[q][3 * k + l] = J[k][l] * id;
-    S.W[q] = T->w[q] * fabs(det);
-    S.idet[q] = id;
-    for (int i = 0; i < 3; ++i) S.xq[q][i] = X[i];
-  }
-  for (int idx = tid; idx < NQ * 27; idx += WG) S.q2[idx / 27][idx % 27] = T->q2[idx / 27][idx % 27];
-  for (int idx = tid; idx < NQ * 4; idx += WG) S.p1[idx / 4][idx % 4] = T->p1[idx / 4][idx % 4];
-  for (int idx = tid; idx < NQ * 8; idx += WG) S.q1[idx / 8][idx % 8] = T->q1[idx / 8][idx % 8];
-  __syncthreads();
-  // push-forward of the Q2 gradients and the RT basis (fixed trip counts, so
-  // the reference-table loads of all rounds are issued together)
-#pragma unroll
-  for (int k = 0; k < (NQ * 27 + WG - 1) / WG; ++k) {
-    const int idx = tid + k * WG;
-    if (idx >= NQ * 27) break;
-    const int q = idx / 27, a = idx % 27;
-    const double *Ji = S.Ji[q];
-    const double d0 = T->dq2[q][a][0], d1 = T->dq2[q][a][1], d2 = T->dq2[q][a][2];
-    for (int i = 0; i < 3; ++i) S.gphi[q][a][i] = Ji[0 * 3 + i] * d0 + Ji[1 * 3 + i] * d1 + Ji[2 * 3 + i] * d2;
-  }
-#pragma unroll
-  for (int k = 0; k < (NQ * 36 + WG - 1) / WG; ++k) {
-    const int idx = tid + k * WG;
-    if (idx >= NQ * 36) break;
-    const int q = idx / 36, r = idx % 36;
-    const double sgn = r < 24 ? S.sg[r >> 2] : 1.0;
-    const double *Jp = S.Jp[q];
-    const double r0 = T->rt[q][r][0], r1 = T->rt[q][r][1], r2 = T->rt[q][r][2];
-    for (int k = 0; k < 3; ++k) S.psi[q][r][k] = sgn * (Jp[3 * k + 0] * r0 + Jp[3 * k + 1] * r1 + Jp[3 * k + 2] * r2);
-    S.dpsi[q][r] = sgn * T->rtdiv[q][r] * S.idet[q];
-  }
-  __syncthreads();
-  // state of x at the quadrature points: 27 x 18 scalar reductions of at most
-  // 36 terms (div u is the trace of grad u, taken after the barrier)
-  for (int idx = tid; idx < NQ * 18; idx += WG) {
-    const int k = idx / NQ, q = idx % NQ;  // quantity-major: a wave's lanes share few branches
-    double acc = 0.0;
-    if (k < 3) {  // u_k
-#pragma unroll
-      for (int a = 0; a < 27; ++a) acc += S.xl[k * 27 + a] * S.q2[q][a];
-      S.u[q][k] = acc;
-    } else if (k < 12) {  // grad u [i][kk]
-      const int i = (k - 3) / 3, kk = (k - 3) % 3;
-#pragma unroll
-      for (int a = 0; a < 27; ++a) acc += S.xl[kk * 27 + a] * S.gphi[q][a][i];
-      S.gu[q][(k - 3)] = acc;
-    } else if (k == 12) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) acc += S.xl[OFF_P + m] * S.p1[q][m];
-      S.p[q] = acc;
-    } else if (k < 16) {
-      const int kk = k - 13;
-#pragma unroll
-      for (int r = 0; r < 36; ++r) acc += S.xl[OFF_J + r] * S.psi[q][r][kk];
-      S.jv[q][kk] = acc;
-    } else if (k == 16) {
-#pragma unroll
-      for (int r = 0; r < 36; ++r) acc += S.xl[OFF_J + r] * S.dpsi[q][r];
-      S.divj[q] = acc;
-    } else {
-#pragma unroll
-      for (int v = 0; v < 8; ++v) acc += S.xl[OFF_PHI + v] * S.q1[q][v];
-      S.ph[q] = acc;
-    }
-  }
-  __syncthreads();
-  if (tid < NQ) S.divu[tid] = S.gu[tid][0] + S.gu[tid][4] + S.gu[tid][8];
-  if (want_al) {
-    __syncthreads();
-    for (int idx = tid; idx < 4 * NU; idx += WG) {
-      const int k = idx / NU, b = idx % NU, cb = b / 27, nb = b % 27;
-      double acc = 0.0;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) acc += S.W[q] * S.p1[q][k] * S.gphi[q][nb][cb];
-      S.D[k][b] = acc;
-    }
-    if (tid < 20) {
-      double acc = 0.0;
-      if (tid < 16) {
-        const int k = tid >> 2, l = tid & 3;
-        for (int q = 0; q < NQ; ++q) acc += S.W[q] * S.p1[q][k] * S.p1[q][l];
-        S.Mq[tid] = acc;
-      } else {
-        const int k = tid - 16;
-        for (int q = 0; q < NQ; ++q) acc += S.W[q] * S.p1[q][k] * S.divu[q];
-        S.dq[k] = acc;
-      }
-    }
-    __syncthreads();
-    if (tid == 0) {
-      inv4(S.Mq, S.Mi);
-      for (int k = 0; k < 4; ++k)
-        S.cu[k] = S.Mi[4 * k + 0] * S.dq[0] + S.Mi[4 * k + 1] * S.dq[1] + S.Mi[4 * k + 2] * S.dq[2] + S.Mi[4 * k + 3] * S.dq[3];
-    }
-    __syncthreads();
-    for (int idx = tid; idx < 4 * NU; idx += WG) {
-      const int k = idx / NU, b = idx % NU;
-      double acc = 0.0;
-      for (int l = 0; l < 4; ++l) acc += S.Mi[4 * k + l] * S.D[l][b];
-      S.MD[k][b] = acc;
-    }
-  }
-  __syncthreads();
-  // convective derivative and Newton weights for the Jacobian tiles
-  for (int idx = tid; idx < NQ * 27; idx += WG) {
-    const int q = idx / 27, a = idx % 27;
-    S.cphi[q][a] = S.u[q][0] * S.gphi[q][a][0] + S.u[q][1] * S.gphi[q][a][1] + S.u[q][2] * S.gphi[q][a][2];
-  }
-  for (int idx = tid; idx < NQ * 9; idx += WG) {
-    const int q = idx / 9, cd = idx % 9, cc = cd / 3, dd = cd % 3;
-    S.wN[q][cd] = S.W[q] * ph.alpha * S.gu[q][3 * dd + cc];
-  }
-  __syncthreads();
-}
-
-__device__ inline void cross3(const double *a, const double *b, double *c) {
-  c[0] = a[1] * b[2] - a[2] * b[1];
-  c[1] = a[2] * b[0] - a[0] * b[2];
-  c[2] = a[0] * b[1] - a[1] * b[0];
-}
 
 // Decode canonical entry e -> (local row a, local column b).
 __device__ inline void decode_entry(int e, int &a, int &b) {
@@ -280,80 +43,6 @@ __device__ inline void decode_entry(int e, int &a, int &b) {
   }
 }
 
-// Jacobian entry (test a, trial b) of the fluid terms.
-__device__ double jac_entry(const CellLDS &S, const RefTables *__restrict__ T, const MhdPhys &ph, int a, int b) {
-  double acc = 0.0;
-  if (a < OFF_P) {  // velocity test v = phi_na e_ca
-    const int ca = a / 27, na = a % 27;
-    if (b < OFF_P) {
-      const int cb = b / 27, nb = b % 27;
-      const bool diag = ca == cb;
-      for (int q = 0; q < NQ; ++q) {
-        double t = 0.0;
-        if (diag) {
-          const double *ga = S.gphi[q][na], *gb = S.gphi[q][nb];
-          t = ph.beta * (ga[0] * gb[0] + ga[1] * gb[1] + ga[2] * gb[2]);
-          if (ph.convection)
-            t += ph.alpha * S.q2[q][na] * (S.u[q][0] * gb[0] + S.u[q][1] * gb[1] + S.u[q][2] * gb[2]);
-        }
-        if (ph.convection == 2) t += ph.alpha * S.q2[q][na] * S.q2[q][nb] * S.gu[q][3 * cb + ca];
-        acc += S.W[q] * t;
-      }
-      if (ph.zeta_u != 0.0) {
-        double al = 0.0;
-        for (int k = 0; k < 4; ++k) {
-          double m = 0.0;
-          for (int l = 0; l < 4; ++l) m += S.Mi[4 * k + l] * S.D[l][b];
-          al += S.D[k][a] * m;
-        }
-        acc += ph.zeta_u * al;
-      }
-    } else if (b < OFF_J) {  // - dp div v
-      const int k = b - OFF_P;
-      for (int q = 0; q < NQ; ++q) acc -= S.W[q] * S.p1[q][k] * S.gphi[q][na][ca];
-    } else {  // - gamma (dj x B).v
-      const int r = b - OFF_J;
-      const int i1 = ca == 2 ? 0 : ca + 1, i2 = ca == 0 ? 2 : ca - 1;
-      const double b1 = S.B[i1], b2 = S.B[i2];
-      for (int q = 0; q < NQ; ++q) {
-        const double cr = S.psi[q][r][i1] * b2 - S.psi[q][r][i2] * b1;  // (psi x B)_ca
-        acc -= ph.gamma * S.W[q] * S.q2[q][na] * cr;
-      }
-    }
-  } else if (a < OFF_J) {  // pressure test: - div du q
-    const int k = a - OFF_P;
-    const int cb = b / 27, nb = b % 27;
-    for (int q = 0; q < NQ; ++q) acc -= S.W[q] * S.p1[q][k] * S.gphi[q][nb][cb];
-  } else if (a < OFF_PHI) {  // current test s = psi_r
-    const int r = a - OFF_J;
-    if (b < OFF_P) {  // - sigma (du x B).s
-      const int cb = b / 27, nb = b % 27;
-      const int i1 = cb == 2 ? 0 : cb + 1, i2 = cb == 0 ? 2 : cb - 1;
-      const double b1 = S.B[i1], b2 = S.B[i2];
-      for (int q = 0; q < NQ; ++q) {
-        // (e_cb x B).s = (B x s)_cb
-        const double t = b1 * S.psi[q][r][i2] - b2 * S.psi[q][r][i1];
-        acc -= ph.sigma * S.W[q] * S.q2[q][nb] * t;
-      }
-    } else if (b < OFF_PHI) {  // dj.s + zeta_j div dj div s
-      const int rb = b - OFF_J;
-      for (int q = 0; q < NQ; ++q) {
-        const double *s = S.psi[q][r], *d = S.psi[q][rb];
-        double t = s[0] * d[0] + s[1] * d[1] + s[2] * d[2];
-        if (ph.zeta_j != 0.0) t += ph.zeta_j * S.dpsi[q][r] * S.dpsi[q][rb];
-        acc += S.W[q] * t;
-      }
-    } else {  // - sigma dphi div s
-      const int v = b - OFF_PHI;
-      for (int q = 0; q < NQ; ++q) acc -= ph.sigma * S.W[q] * S.q1[q][v] * S.dpsi[q][r];
-    }
-  } else {  // potential test: - div dj phi_t
-    const int v = a - OFF_PHI, rb = b - OFF_J;
-    for (int q = 0; q < NQ; ++q) acc -= S.W[q] * S.q1[q][v] * S.dpsi[q][rb];
-  }
-  return acc;
-}
-
 typedef double d4_t __attribute__((ext_vector_type(4)));
 
 // How a cell's Jacobian entries leave the kernel:
@@ -364,9 +53,48 @@ typedef double d4_t __attribute__((ext_vector_type(4)));
 //                   the element buffer (summed into CSR rows by k_row_assemble).
 enum { SCATTER_ATOMIC = 0, SCATTER_COLOUR = 1, SCATTER_EBUF = 2 };
 
+// Reference values at the quadrature points, the same for every cell: loaded
+// into LDS once per workgroup.  Point 27 is all zeros (the padding of K = 27 to
+// 28), and a tile's padding rows and columns read whatever follows.
+struct JacTab {
+  double t4[NQ + 1][4][27];      // d_0, d_1, d_2 and value of the Q2 functions
+  double rv[NQ + 1][NJ];         // RT1: the component along axis d of its dofs, [12 d + i]
+  double rd[NQ + 1][NJ];         // ... their divergence
+  double q1[NQ + 1][8];
+  double p1[NQ + 1][4];
+  double slack[16];
+};
+
+// Weights of one cell at the quadrature points, and what its stores need.
+struct JacCell {
+  double mq[NQ + 1][12];         // W beta G (3 x 3, G = J^-1 J^-T), then W alpha u . J^-T (row 3)
+  double wN[NQ + 1][9];          // W alpha d_d u_c at [3 c + d] (Newton)
+  double wd[NQ + 1][6];          // W / det^2 (J^T J)_{dd'}, d <= d'
+  double wx[NQ + 1][9];          // W / det (J_{:,d} x B)_c at [3 c + d]
+  double wj[NQ + 1][9];          // W J^-1[l][c] at [3 l + c]
+  double wv[NQ + 1];             // W zeta_j / det^2
+  double ws[NQ + 1];             // W / det
+  union {
+    struct {
+      double x[NU], xyz[24], fl[NQ * 9];
+    };
+    struct {
+      double D[4][NU];           // int psi_k div v_b
+      double MD[4][NU];          // zeta_u M^-1 D
+    };
+  };
+  double minv[16];
+  double sg[NJ + 12];            // orientation signs at [12 d + i]
+  int64_t rp[NDOF];
+  int32_t g[NDOF];
+};
+
+// local RT1 dof i of axis d: its two faces' four dofs, then the interior ones
+__device__ inline int rt_local(int d, int i) { return i < 8 ? 8 * (2 - d) + i : 24 + 4 * d + i - 8; }
+
 // Entry e (canonical index) of local row lr / local column lc with value v.
 template <int MODE>
-__device__ inline void emit(const CellLDS &S, const uint16_t *__restrict__ rk, double *__restrict__ out, int e, int lr,
+__device__ inline void emit(const JacCell &S, const uint16_t *__restrict__ rk, double *__restrict__ out, int e, int lr,
                             int lc, double v) {
   if (MODE == SCATTER_EBUF) {
     out[e] = v;
@@ -382,12 +110,12 @@ __device__ inline d4_t mfma16(double a, double b, d4_t c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// Scatter-add one 16x16 MFMA result tile.  Lane l holds rows l/16 + 4 r
-// (r = 0..3), column l%16 of the tile (v_mfma_f64_16x16x4f64 output layout); (row0, col0) are the local dof offsets of the tile,
-// `ent(i, j)` maps tile-local (i, j) to the canonical entry of the rank map.
-template <int MODE, class EntFn>
-__device__ inline void scatter_tile(const CellLDS &S, const d4_t &acc, double scale, int row0, int nrow, int col0,
-                                    int ncol, const uint16_t *__restrict__ rk, double *__restrict__ out, EntFn ent) {
+// One 16x16 MFMA result tile times `scale`.  Lane l holds rows l/16 + 4 r
+// (r = 0..3), column l%16 (v_mfma_f64_16x16x4f64 output layout); `place(i, j, e,
+// lr, lc)` gives the canonical entry and local dofs of tile-local (i, j).
+template <int MODE, class Place>
+__device__ inline void store_tile(const JacCell &S, const d4_t &acc, double scale, int nrow, int ncol,
+                                  const uint16_t *__restrict__ rk, double *__restrict__ out, Place place) {
   const int lane = threadIdx.x & 63;
   const int j = lane & 15;
   if (j >= ncol) return;
@@ -395,203 +123,305 @@ __device__ inline void scatter_tile(const CellLDS &S, const d4_t &acc, double sc
   for (int r = 0; r < 4; ++r) {
     const int i = (lane >> 4) + 4 * r;
     if (i >= nrow) continue;
-    emit<MODE>(S, rk, out, ent(i, j), row0 + i, col0 + j, scale * acc[r]);
+    int e, lr, lc;
+    place(i, j, e, lr, lc);
+    emit<MODE>(S, rk, out, e, lr, lc, scale * acc[r]);
   }
 }
 
-// Jacobian of one cell as FP64 MFMA tiles (16x16x4):
-//   uu(c,d) = delta_cd S + N^{cd} + zeta_u D_c^T M^-1 D_d with
-//     S[a][b]    = sum_q W (beta grad phi_a . grad phi_b + alpha phi_a u.grad phi_b)   (K = 27 q x 4)
-//     N^{cd}[a][b] = sum_q W alpha d_d u_c phi_a phi_b                                (K = 27 q)
-//   X_c[a][r]  = sum_q W phi_a (psi_r x B)_c  ->  uj = -gamma X,  ju = +sigma X^T         (K = 27 q)
-//     (-sigma (e_c phi_a x B).psi_r = +sigma phi_a (psi_r x B)_c, so ju = -(sigma/gamma) uj^T)
-//   jj[r][s]   = sum_q W (psi_r . psi_s + zeta_j div psi_r div psi_s)                    (K = 27 q x 4)
-// The small blocks up / pu (81 x 4) and jphi / phij (36 x 8) run on the vector ALUs.
-// `out` is the CSR value array (atomic / colour modes) or the cell's element
-// buffer slot (NENT doubles, element-buffer mode).
-template <int MODE>
-__device__ void cell_jacobian_tiles(const CellLDS &S, const MhdPhys &ph, const uint16_t *__restrict__ rk,
-                                    double *__restrict__ val) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int li = lane & 15, lk = lane >> 4;
-  const d4_t zero = {0.0, 0.0, 0.0, 0.0};
-  // job list: 4 uu super-tiles, 9 jj tiles, 18 cross tiles; wave w takes jobs w, w+4, ...
-  for (int job = wave; job < 4 + 9 + 18; job += WG / 64) {
-    if (job < 4) {
-      const int ti = job >> 1, tj = job & 1;
-      const int a = 16 * ti + li, b = 16 * tj + li;
-      const bool av = a < 27, bv = b < 27;
-      d4_t Sacc = zero;
-#pragma unroll 9
-      for (int q = 0; q < NQ; ++q) {
-        double A = 0.0, Bv = 0.0;
-        if (av) A = lk < 3 ? S.gphi[q][a][lk] : S.q2[q][a];
-        if (bv) Bv = S.W[q] * (lk < 3 ? ph.beta * S.gphi[q][b][lk] : (ph.convection ? ph.alpha * S.cphi[q][b] : 0.0));
-        Sacc = mfma16(A, Bv, Sacc);
-      }
-      // Q2 values of this lane's rows / columns at its 7 quadrature points,
-      // shared by the nine (c, d) blocks
-      double qa[7], qb[7];
-#pragma unroll
-      for (int st = 0; st < 7; ++st) {
-        const int q = 4 * st + lk;
-        qa[st] = (av && q < NQ) ? S.q2[q][a] : 0.0;
-        qb[st] = (bv && q < NQ) ? S.q2[q][b] : 0.0;
-      }
-#pragma unroll 1
-      for (int cd = 0; cd < 9; ++cd) {
-        const int c = cd / 3, d = cd % 3;
-        d4_t acc = c == d ? Sacc : zero;
-        if (ph.convection == 2) {
-          double wq[7];
-#pragma unroll
-          for (int st = 0; st < 7; ++st) wq[st] = 4 * st + lk < NQ ? S.wN[4 * st + lk][cd] : 0.0;
-#pragma unroll
-          for (int st = 0; st < 7; ++st) acc = mfma16(qa[st], wq[st] * qb[st], acc);
-        }
-        if (ph.zeta_u != 0.0) {
-          const double A = av ? S.D[lk][c * 27 + a] : 0.0;
-          const double Bv = bv ? ph.zeta_u * S.MD[lk][d * 27 + b] : 0.0;
-          acc = mfma16(A, Bv, acc);
-        }
-        const int r0 = c * 27 + 16 * ti, c0 = d * 27 + 16 * tj;
-        scatter_tile<MODE>(S, acc, 1.0, r0, min(16, 27 - 16 * ti), c0, min(16, 27 - 16 * tj), rk, val,
-                     [&](int i, int j) { return (r0 + i) * ROWS_U_LEN + (c0 + j); });
-      }
-    } else if (job < 13) {
-      const int t = job - 4, ti = t / 3, tj = t % 3;
-      const int r = 16 * ti + li, sidx = 16 * tj + li;
-      const bool rv = r < 36, sv = sidx < 36;
-      d4_t acc = zero;
-#pragma unroll 9
-      for (int q = 0; q < NQ; ++q) {
-        double A = 0.0, Bv = 0.0;
-        if (rv) A = lk < 3 ? S.psi[q][r][lk] : S.dpsi[q][r];
-        if (sv) Bv = S.W[q] * (lk < 3 ? S.psi[q][sidx][lk] : ph.zeta_j * S.dpsi[q][sidx]);
-        acc = mfma16(A, Bv, acc);
-      }
-      const int r0 = 16 * ti, s0 = 16 * tj;
-      scatter_tile<MODE>(S, acc, 1.0, OFF_J + r0, min(16, 36 - r0), OFF_J + s0, min(16, 36 - s0), rk, val,
-                   [&](int i, int j) { return E_J + (r0 + i) * ROWS_J_LEN + NU + (s0 + j); });
-    } else {
-      const int t = job - 13, c = t / 6, tt = t % 6, ti = tt / 3, tj = tt % 3;
-      const int c1 = c == 2 ? 0 : c + 1, c2 = c == 0 ? 2 : c - 1;
-      const double b1 = S.B[c1], b2 = S.B[c2];
-      const int a = 16 * ti + li, r = 16 * tj + li;
-      const bool av = a < 27, rv = r < 36;
-      d4_t acc = zero, accT = zero;
-#pragma unroll
-      for (int st = 0; st < 7; ++st) {
-        const int q = 4 * st + lk;
-        const double A = (av && q < NQ) ? S.q2[q][a] : 0.0;
-        const double Bv = (rv && q < NQ) ? S.W[q] * (S.psi[q][r][c1] * b2 - S.psi[q][r][c2] * b1) : 0.0;
-        acc = mfma16(A, Bv, acc);
-        // A and B share the lane -> (index, k) layout, so swapping them gives X^T
-        if (MODE == SCATTER_EBUF) accT = mfma16(Bv, A, accT);
-      }
-      const int a0 = 16 * ti, r0 = 16 * tj;
-      const int na = min(16, 27 - a0), nr = min(16, 36 - r0);
-      // uj = -gamma X   (u row c*27 + a, j column r)
-      scatter_tile<MODE>(S, acc, -ph.gamma, c * 27 + a0, na, OFF_J + r0, nr, rk, val,
-                   [&](int i, int j) { return (c * 27 + a0 + i) * ROWS_U_LEN + OFF_J + r0 + j; });
-      // ju = +sigma X^T (j row r, u column c*27 + a)
-      if (MODE == SCATTER_EBUF) {
-        // accT lane holds X^T[r0 + i][a0 + j]: rows of the j block, contiguous u columns
-        scatter_tile<MODE>(S, accT, ph.sigma, OFF_J + r0, nr, c * 27 + a0, na, rk, val,
-                           [&](int i, int j) { return E_J + (r0 + i) * ROWS_J_LEN + c * 27 + a0 + j; });
-      } else {
-        // lane holds X[a0+i][r0+j] -> entry (j row r0+j, u col a0+i)
-        const int j = lane & 15;
-        if (j < nr && S.g[OFF_J + r0 + j] >= 0) {
-          const int lr = OFF_J + r0 + j;
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) {
-            const int i = (lane >> 4) + 4 * rr;
-            if (i >= na) continue;
-            const int lc = c * 27 + a0 + i;
-            if (S.g[lc] < 0) continue;
-            emit<MODE>(S, rk, val, E_J + (r0 + j) * ROWS_J_LEN + lc, lr, lc, ph.sigma * acc[rr]);
-          }
-        }
-      }
-    }
-  }
-  // up / pu (81 x 4) and jphi / phij (36 x 8) on the vector ALUs
-  for (int t = threadIdx.x; t < NU * 4 + NJ * 8; t += WG) {
-    if (t < NU * 4) {
-      const int row = t >> 2, k = t & 3, ca = row / 27, na = row % 27;
-      if (MODE != SCATTER_EBUF && (S.g[row] < 0 || S.g[OFF_P + k] < 0)) continue;
-      double acc = 0.0;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) acc -= S.W[q] * S.p1[q][k] * S.gphi[q][na][ca];
-      emit<MODE>(S, rk, val, row * ROWS_U_LEN + OFF_P + k, row, OFF_P + k, acc);     // - dp div v
-      emit<MODE>(S, rk, val, E_P + k * ROWS_P_LEN + row, OFF_P + k, row, acc);       // - div du q
-    } else {
-      const int tt = t - NU * 4, r = tt >> 3, v = tt & 7;
-      if (MODE != SCATTER_EBUF && (S.g[OFF_J + r] < 0 || S.g[OFF_PHI + v] < 0)) continue;
-      double acc = 0.0;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) acc -= S.W[q] * S.q1[q][v] * S.dpsi[q][r];
-      emit<MODE>(S, rk, val, E_J + r * ROWS_J_LEN + NU + NJ + v, OFF_J + r, OFF_PHI + v, ph.sigma * acc);  // - sigma dphi div s
-      emit<MODE>(S, rk, val, E_PHI + v * ROWS_PHI_LEN + r, OFF_PHI + v, OFF_J + r, acc);                   // - div dj phi_t
-    }
-  }
-}
-
-// cells[i] (or i when cells == nullptr) for i < ncells; SCATTER_COLOUR needs
-// a colour class: no two listed cells share a dof.  SCATTER_EBUF writes cell c's
-// entries to val + c * NENT (val is then the element buffer).
+// Jacobian of one cell per workgroup and turn, on FP64 MFMA tiles (16x16x4) in
+// reference space: every factor that is the same for all cells (reference
+// values and gradients) sits in LDS tables loaded once per workgroup, and a
+// cell brings 57 weights per quadrature point.  With a, b Q2 nodes, r, s RT1
+// dofs of the axes d, d' (one nonzero reference component each):
+//   uu(c,d) = delta_cd S + N^{cd} + zeta_u D_c^T M^-1 D_d
+//     S   = sum_q [d_0 a, d_1 a, d_2 a, a] . mq [d_l b]                    (K = 27 x 4)
+//     N   = sum_q wN_cd a b                                              (K = 27)
+//   up / pu = -D, D = sum_q d_l a (W J^-1_lc) psi_k                        (K = 27 x 3)
+//   X_c[a][r] = sum_q wx_cd a r -> uj = -gamma X, ju = +sigma X^T          (K = 27)
+//   jj  = sum_q wd_dd' r s + wv div r div s                              (K = 2 x 27)
+//   jphi / phij = sum_q ws q1 div r                                      (K = 27)
+// The first version mapped the 27 + 36 basis functions to physical space at
+// every point: half of a cell's 124 K cycles went into that staging and jj took
+// K = 27 x 4.  JACFIG
 template <int MODE>
 __global__ __launch_bounds__(WG, 2) void k_cell_jacobian(int ncells, const int32_t *__restrict__ cells,
-                                                         const double *__restrict__ xyz,
-                                                         const int32_t *__restrict__ dofs, const int8_t *__restrict__ sign,
-                                                         const double *__restrict__ dir, const double *__restrict__ x,
-                                                         const RefTables *__restrict__ T,
-                                                         const int64_t *__restrict__ rowptr,
-                                                         const uint16_t *__restrict__ rank, double *__restrict__ val,
-                                                         MhdPhys ph) {
-  __shared__ CellLDS S;
-  for (int i = blockIdx.x; i < ncells; i += gridDim.x) {
-    const int c = cells ? cells[i] : i;
-    stage_cell(S, c, xyz, dofs, sign, dir, x, T, rowptr, ph, ph.zeta_u != 0.0);
-    if (threadIdx.x < 3) S.B[threadIdx.x] = ph.B[threadIdx.x];
+                                                      const double *__restrict__ xyz,
+                                                      const int32_t *__restrict__ dofs,
+                                                      const int8_t *__restrict__ sign,
+                                                      const double *__restrict__ dir, const double *__restrict__ x,
+                                                      const double *__restrict__ minv,
+                                                      const RefTables *__restrict__ T,
+                                                      const int64_t *__restrict__ rowptr,
+                                                      const uint16_t *__restrict__ rank, double *__restrict__ val,
+                                                      MhdPhys ph) {
+  __shared__ JacTab R;
+  __shared__ JacCell S;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const d4_t zero = {0.0, 0.0, 0.0, 0.0};
+  for (int e = tid; e < (NQ + 1) * 108; e += WG) {
+    const int q = e / 108, l = e / 27 % 4, a = e % 27;
+    R.t4[q][l][a] = q == NQ ? 0.0 : (l < 3 ? T->dq2[q][a][l] : T->q2[q][a]);
+  }
+  for (int e = tid; e < (NQ + 1) * NJ; e += WG) {
+    const int q = e / NJ, d = e % NJ / 12, r = rt_local(d, e % 12);
+    R.rv[q][e % NJ] = q == NQ ? 0.0 : T->rt[q][r][d];
+    R.rd[q][e % NJ] = q == NQ ? 0.0 : T->rtdiv[q][r];
+  }
+  for (int e = tid; e < (NQ + 1) * 8; e += WG) R.q1[e / 8][e % 8] = e < NQ * 8 ? T->q1[e / 8][e % 8] : 0.0;
+  for (int e = tid; e < (NQ + 1) * 4; e += WG) R.p1[e / 4][e % 4] = e < NQ * 4 ? T->p1[e / 4][e % 4] : 0.0;
+  if (tid < 16) R.slack[tid] = 0.0;
+  if (tid < 12) S.mq[NQ][tid] = S.sg[NJ + tid] = 0.0;
+  if (tid < 9) S.wN[NQ][tid] = S.wx[NQ][tid] = S.wj[NQ][tid] = 0.0;
+  if (tid < 6) S.wd[NQ][tid] = 0.0;
+  if (tid == 0) S.wv[NQ] = S.ws[NQ] = 0.0;
+  for (int cell = blockIdx.x; cell < ncells; cell += gridDim.x) {
+    const int c = cells ? cells[cell] : cell;
+    const uint16_t *rk = rank + (int64_t)c * NENT;
+    double *out = MODE == SCATTER_EBUF ? val + (int64_t)c * NENT : val;
+    // ---- the cell's data (the previous cell's tiles are done)
+    if (tid < NU) {
+      const int32_t g = dofs[(int64_t)c * NDOF + tid];
+      S.x[tid] = g >= 0 ? x[g] : dir[-(int64_t)g - 1];
+    } else if (tid < 128 && tid >= 96) {
+      if (tid < 120) S.xyz[tid - 96] = xyz[(int64_t)c * 24 + tid - 96];
+    } else if (tid >= 128 && tid < 128 + NJ) {
+      const int i = tid - 128;
+      S.sg[i] = sign && i % 12 < 8 ? (double)sign[(int64_t)c * 6 + (rt_local(i / 12, i % 12) >> 2)] : 1.0;
+    } else if (tid >= 192 && tid < 208) {
+      S.minv[tid - 192] = minv[(int64_t)c * 16 + tid - 192];
+    }
+    if (MODE != SCATTER_EBUF && tid < NDOF) {
+      const int32_t g = dofs[(int64_t)c * NDOF + tid];
+      S.g[tid] = g;
+      S.rp[tid] = g >= 0 ? rowptr[g] : -1;
+    }
     __syncthreads();
-    cell_jacobian_tiles<MODE>(S, ph, rank + (int64_t)c * NENT, MODE == SCATTER_EBUF ? val + (int64_t)c * NENT : val);
+    // ---- weights at the points: wave 0, one lane per point
+    if (wave == 0) {
+      const int q = lane < NQ ? lane : NQ - 1;
+      const int d[3] = {q % 3, (q / 3) % 3, q / 9};
+      double fw[3][4], V[3], dv, J[9], Ji[9];
+      if (ph.convection) fields_forward<false>(S.x, nullptr, S.fl, 9, d, lane < NQ, fw, V, dv);
+      tri_jacobian(S.xyz, gauss_x(d[0]), gauss_x(d[1]), gauss_x(d[2]), J);
+      const double det = inv3(J, Ji);
+      const double W = gauss_w(d[0]) * gauss_w(d[1]) * gauss_w(d[2]) * fabs(det), id = 1.0 / det;
+      if (lane < NQ) {
+        const double wb = W * ph.beta, wi = W * id, wii = wi * id;
+#pragma unroll
+        for (int l = 0; l < 3; ++l)
+#pragma unroll
+          for (int m = 0; m < 3; ++m) {
+            S.mq[q][3 * l + m] = wb * (Ji[3 * l] * Ji[3 * m] + Ji[3 * l + 1] * Ji[3 * m + 1] + Ji[3 * l + 2] * Ji[3 * m + 2]);
+            S.wj[q][3 * l + m] = W * Ji[3 * l + m];
+          }
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+          S.mq[q][9 + m] = ph.convection ? W * ph.alpha * (fw[0][0] * Ji[3 * m] + fw[1][0] * Ji[3 * m + 1] + fw[2][0] * Ji[3 * m + 2])
+                                         : 0.0;
+        if (ph.convection == 2)
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)  // d u_k / d x_i
+              S.wN[q][3 * k + i] = W * ph.alpha * (Ji[i] * fw[k][1] + Ji[3 + i] * fw[k][2] + Ji[6 + i] * fw[k][3]);
+        int e = 0;
+#pragma unroll
+        for (int l = 0; l < 3; ++l)
+#pragma unroll
+          for (int m = l; m < 3; ++m) S.wd[q][e++] = wii * (J[l] * J[m] + J[3 + l] * J[3 + m] + J[6 + l] * J[6 + m]);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+          S.wx[q][l] = wi * (J[3 + l] * ph.B[2] - J[6 + l] * ph.B[1]);
+          S.wx[q][3 + l] = wi * (J[6 + l] * ph.B[0] - J[l] * ph.B[2]);
+          S.wx[q][6 + l] = wi * (J[l] * ph.B[1] - J[3 + l] * ph.B[0]);
+        }
+        S.wv[q] = wii * ph.zeta_j;
+        S.ws[q] = wi;
+      }
+    }
+    __syncthreads();
+    // ---- S tile of the wave; the waves of the first column tile also form D
+    const int ti = wave >> 1, tj = wave & 1;
+    const int a = 16 * ti + li, b = 16 * tj + li;
+    d4_t Sacc = zero, Dacc = zero;
+    {
+      const int cc = min(li >> 2, 2), kk = li & 3;
+#pragma unroll 3
+      for (int q = 0; q < NQ; ++q) {
+        const double A = (&R.t4[q][lk][0])[a];
+        const double *m = &S.mq[q][3 * lk];
+        const double *t = &R.t4[q][0][0] + b;
+        Sacc = mfma16(A, m[0] * t[0] + m[1] * t[27] + m[2] * t[54], Sacc);
+        if (tj == 0) Dacc = mfma16(A, lk < 3 ? S.wj[q][3 * lk + cc] * R.p1[q][kk] : 0.0, Dacc);
+      }
+    }
+    if (tj == 0 && li < 12) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * ti + lk + 4 * r;
+        if (row < 27) S.D[li & 3][(li >> 2) * 27 + row] = Dacc[r];
+      }
+    }
+    __syncthreads();
+    for (int e = tid; e < 4 * NU; e += WG) {
+      const int k = e / NU, row = e % NU;
+      const double dk = S.D[k][row];
+      if (ph.zeta_u != 0.0)
+        S.MD[k][row] = ph.zeta_u * (S.minv[4 * k] * S.D[0][row] + S.minv[4 * k + 1] * S.D[1][row] +
+                                    S.minv[4 * k + 2] * S.D[2][row] + S.minv[4 * k + 3] * S.D[3][row]);
+      emit<MODE>(S, rk, out, row * ROWS_U_LEN + OFF_P + k, row, OFF_P + k, -dk);  // - dp div v
+      emit<MODE>(S, rk, out, E_P + k * ROWS_P_LEN + row, OFF_P + k, row, -dk);    // - div du q
+    }
+    // ---- 18 cross, 9 jj and 3 jphi jobs of 14 MFMAs each
+    for (int job = wave; job < 30; job += WG / 64) {
+      if (job < 18) {
+        const int at = job / 9, d = job / 3 % 3, cc = job % 3;
+        const double sgr = S.sg[12 * d + li];
+        d4_t acc = zero, accT = zero;
+#pragma unroll
+        for (int st = 0; st < 7; ++st) {
+          const int q = 4 * st + lk;
+          const double A = (&R.t4[q][3][0])[16 * at + li];
+          const double Bv = S.wx[q][3 * cc + d] * sgr * (&R.rv[q][12 * d])[li];
+          acc = mfma16(A, Bv, acc);
+          accT = mfma16(Bv, A, accT);  // A and B share the lane layout: swapped, they give X^T
+        }
+        const int a0 = cc * 27 + 16 * at, na = at ? 11 : 16;
+        store_tile<MODE>(S, acc, -ph.gamma, na, 12, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
+          lr = a0 + i;
+          lc = OFF_J + rt_local(d, j);
+          e = lr * ROWS_U_LEN + lc;
+        });
+        store_tile<MODE>(S, accT, ph.sigma, 12, na, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
+          const int r = rt_local(d, i);
+          lr = OFF_J + r;
+          lc = a0 + j;
+          e = E_J + r * ROWS_J_LEN + lc;
+        });
+      } else if (job < 27) {
+        const int d = (job - 18) / 3, d2 = (job - 18) % 3;
+        const int lo = min(d, d2), hi = max(d, d2), wk = lo == 0 ? hi : lo + hi + 1;  // place of (lo, hi) in wd
+        const double sr = S.sg[12 * d + li], ss = S.sg[12 * d2 + li];
+        d4_t acc = zero, acc2 = zero;
+#pragma unroll
+        for (int st = 0; st < 7; ++st) {
+          const int q = 4 * st + lk;
+          acc = mfma16(sr * (&R.rv[q][12 * d])[li], S.wd[q][wk] * ss * (&R.rv[q][12 * d2])[li], acc);
+          acc2 = mfma16(sr * (&R.rd[q][12 * d])[li], S.wv[q] * ss * (&R.rd[q][12 * d2])[li], acc2);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] += acc2[r];
+        store_tile<MODE>(S, acc, 1.0, 12, 12, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
+          const int r = rt_local(d, i), s2 = rt_local(d2, j);
+          lr = OFF_J + r;
+          lc = OFF_J + s2;
+          e = E_J + r * ROWS_J_LEN + NU + s2;
+        });
+      } else {
+        const int d = job - 27;
+        const double sr = S.sg[12 * d + li];
+        d4_t acc = zero, accT = zero;
+#pragma unroll
+        for (int st = 0; st < 7; ++st) {
+          const int q = 4 * st + lk;
+          const double A = sr * (&R.rd[q][12 * d])[li], Bv = S.ws[q] * (&R.q1[q][0])[li & 7];
+          acc = mfma16(A, Bv, acc);
+          accT = mfma16(Bv, A, accT);
+        }
+        store_tile<MODE>(S, acc, -ph.sigma, 12, 8, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
+          const int r = rt_local(d, i);
+          lr = OFF_J + r;
+          lc = OFF_PHI + j;
+          e = E_J + r * ROWS_J_LEN + NU + NJ + j;  // - sigma dphi div s
+        });
+        store_tile<MODE>(S, accT, -1.0, 8, 12, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
+          const int r = rt_local(d, j);
+          lr = OFF_PHI + i;
+          lc = OFF_J + r;
+          e = E_PHI + i * ROWS_PHI_LEN + r;  // - div dj phi_t
+        });
+      }
+    }
+    __syncthreads();
+    // ---- the nine (c, d) blocks of the wave's uu tile
+    double qa[7], qb[7];
+#pragma unroll
+    for (int st = 0; st < 7; ++st) {
+      qa[st] = (&R.t4[4 * st + lk][3][0])[a];
+      qb[st] = (&R.t4[4 * st + lk][3][0])[b];
+    }
+    const int na = ti ? 11 : 16, nb = tj ? 11 : 16;
+#pragma unroll 1
+    for (int cd = 0; cd < 9; ++cd) {
+      const int cc = cd / 3, dd = cd % 3;
+      d4_t acc = cc == dd ? Sacc : zero;
+      if (ph.convection == 2) {
+        double wq[7];
+#pragma unroll
+        for (int st = 0; st < 7; ++st) wq[st] = S.wN[4 * st + lk][cd] * qb[st];
+#pragma unroll
+        for (int st = 0; st < 7; ++st) acc = mfma16(qa[st], wq[st], acc);
+      }
+      if (ph.zeta_u != 0.0)
+        acc = mfma16(a < 27 ? S.D[lk][cc * 27 + a] : 0.0, b < 27 ? S.MD[lk][dd * 27 + b] : 0.0, acc);
+      const int r0 = cc * 27 + 16 * ti, c0 = dd * 27 + 16 * tj;
+      store_tile<MODE>(S, acc, 1.0, na, nb, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
+        lr = r0 + i;
+        lc = c0 + j;
+        e = lr * ROWS_U_LEN + lc;
+      });
+    }
     __syncthreads();
   }
 }
 
 // Per-cell integrals of the state (post-processing, src/Applications/hunt.jl:247-260):
 // out[c] = (int u.u, int grad u : grad u, int j.j, int (div j)^2, int p, |K|).  The 3x3x3
-// Gauss rule integrates these polynomial quantities exactly on affine cells.
-__global__ __launch_bounds__(WG, 2) void k_cell_integrals(int ncells, const double *__restrict__ xyz,
-                                                         const int32_t *__restrict__ dofs,
-                                                         const int8_t *__restrict__ sign,
-                                                         const double *__restrict__ dir,
-                                                         const double *__restrict__ x,
-                                                         const RefTables *__restrict__ T, double *__restrict__ out,
-                                                         MhdPhys ph) {
-  __shared__ CellLDS S;
-  for (int c = blockIdx.x; c < ncells; c += gridDim.x) {
-    stage_cell(S, c, xyz, dofs, sign, dir, x, T, nullptr, ph, false);
-    const int k = threadIdx.x;
-    if (k < 6) {
-      double acc = 0.0;
-      for (int q = 0; q < NQ; ++q) {
-        double v;
-        if (k == 0) v = S.u[q][0] * S.u[q][0] + S.u[q][1] * S.u[q][1] + S.u[q][2] * S.u[q][2];
-        else if (k == 1) {
-          v = 0.0;
-          for (int i = 0; i < 9; ++i) v += S.gu[q][i] * S.gu[q][i];
-        } else if (k == 2) v = S.jv[q][0] * S.jv[q][0] + S.jv[q][1] * S.jv[q][1] + S.jv[q][2] * S.jv[q][2];
-        else if (k == 3) v = S.divj[q] * S.divj[q];
-        else if (k == 4) v = S.p[q];
-        else v = 1.0;
-        acc += S.W[q] * v;
-      }
-      out[(int64_t)c * 6 + k] = acc;
+// Gauss rule integrates these polynomial quantities exactly on affine cells.  Half a
+// wave per cell, one lane per point (see mhd_cellop.hip).
+__global__ __launch_bounds__(64) void k_cell_integrals(int ncells, const double *__restrict__ xyz,
+                                                       const int32_t *__restrict__ dofs,
+                                                       const int8_t *__restrict__ sign,
+                                                       const double *__restrict__ dir, const double *__restrict__ x,
+                                                       double *__restrict__ out) {
+  __shared__ double xs[2][NDOF + 1], X[2][24], fl[2][NQ * 14];
+  const int half = threadIdx.x >> 5, hl = threadIdx.x & 31;
+  const int c = blockIdx.x * 2 + half;
+  if (c < ncells) {
+    for (int l = hl; l < NDOF; l += 32) {
+      const int32_t g = dofs[(int64_t)c * NDOF + l];
+      double v = g >= 0 ? x[g] : dir[-(int64_t)g - 1];
+      if (l >= OFF_J && l < OFF_J + 24 && sign) v *= (double)sign[(int64_t)c * 6 + ((l - OFF_J) >> 2)];
+      xs[half][l] = v;
     }
-    __syncthreads();
+    if (hl < 24) X[half][hl] = xyz[(int64_t)c * 24 + hl];
+  }
+  __syncthreads();
+  const int q = hl < NQ ? hl : NQ - 1;
+  const int d[3] = {q % 3, (q / 3) % 3, q / 9};
+  double fw[3][4], V[3], dv, J[9], Ji[9];
+  fields_forward<true>(xs[half], xs[half] + OFF_J, fl[half], 14, d, hl < NQ, fw, V, dv);
+  const double px = gauss_x(d[0]), py = gauss_x(d[1]), pz = gauss_x(d[2]);
+  tri_jacobian(X[half], px, py, pz, J);
+  const double det = inv3(J, Ji), id = 1.0 / det;
+  const double W = hl < NQ && c < ncells ? gauss_w(d[0]) * gauss_w(d[1]) * gauss_w(d[2]) * fabs(det) : 0.0;
+  double v[6] = {0.0, 0.0, 0.0, dv * id * dv * id, 0.0, 1.0};
+  for (int k = 0; k < 3; ++k) {
+    v[0] += fw[k][0] * fw[k][0];
+    for (int i = 0; i < 3; ++i) {
+      const double g = Ji[i] * fw[k][1] + Ji[3 + i] * fw[k][2] + Ji[6 + i] * fw[k][3];
+      v[1] += g * g;
+    }
+    const double jk = (J[3 * k] * V[0] + J[3 * k + 1] * V[1] + J[3 * k + 2] * V[2]) * id;
+    v[2] += jk * jk;
+  }
+  const double *xp = xs[half] + OFF_P;
+  v[4] = xp[0] * (1.0 - px - py - pz) + xp[1] * px + xp[2] * py + xp[3] * pz;
+  for (int k = 0; k < 6; ++k) {
+    double s = W != 0.0 ? W * v[k] : 0.0;
+    for (int off = 16; off > 0; off >>= 1) s += __shfl_xor(s, off, 32);
+    if (hl == 0 && c < ncells) out[(int64_t)c * 6 + k] = s;
   }
 }
 
@@ -1155,6 +985,11 @@ __global__ __launch_bounds__(64) void k_skel_jacobian(int64_t n, const int64_t *
 
 }  // namespace
 
+// Workgroups of the cell kernel: it loads 43 KB of tables, so a workgroup takes
+// several cells.  Two fit a CU (256 CUs); four times that many keep the last
+// round short (tables are then under a tenth of a workgroup's 16 cells).
+static unsigned jacobian_blocks(int ncells) { return (unsigned)std::min(ncells, 2048); }
+
 int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_t s) {
   // a cell holding one dof twice (a periodic direction one cell thick) needs
   // the atomic scatter: its own entries may coincide
@@ -1162,9 +997,9 @@ int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_
   if (mode == 2 && sizeof(double) * (size_t)RA_WAVES * c->max_row > 65536) mode = 1;  // row too long for LDS
   if (mode == 2 && c->ncells > 0) {
     if (!c->d_ebuf) MHD_HIP(hipMalloc(&c->d_ebuf, sizeof(double) * (size_t)c->ncells * NENT));
-    hipLaunchKernelGGL((k_cell_jacobian<SCATTER_EBUF>), dim3(c->ncells), dim3(WG), 0, s, c->ncells,
-                       (const int32_t *)nullptr, c->d_xyz, c->d_dofs, c->d_sign, c->d_dir, d_x, c->d_ref, c->d_rowptr,
-                       c->d_rank, c->d_ebuf, c->phys);
+    hipLaunchKernelGGL((k_cell_jacobian<SCATTER_EBUF>), dim3(jacobian_blocks(c->ncells)), dim3(WG), 0, s, c->ncells,
+                       (const int32_t *)nullptr, c->d_xyz, c->d_dofs, c->d_sign, c->d_dir, d_x, c->d_minv, c->d_ref,
+                       c->d_rowptr, c->d_rank, c->d_ebuf, c->phys);
     MHD_HIP(hipGetLastError());
     if (c->n > 0) {
       const int64_t blocks = std::min<int64_t>((c->n + RA_WAVES - 1) / RA_WAVES, 1 << 20);
@@ -1178,17 +1013,17 @@ int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_
   }
   if (mode == 2 || c->ncells == 0) {
   } else if (mode == 0 || c->color_ptr.size() < 2) {
-    hipLaunchKernelGGL((k_cell_jacobian<SCATTER_ATOMIC>), dim3(c->ncells), dim3(WG), 0, s, c->ncells,
-                       (const int32_t *)nullptr, c->d_xyz, c->d_dofs, c->d_sign, c->d_dir, d_x, c->d_ref, c->d_rowptr,
-                       c->d_rank, d_val, c->phys);
+    hipLaunchKernelGGL((k_cell_jacobian<SCATTER_ATOMIC>), dim3(jacobian_blocks(c->ncells)), dim3(WG), 0, s, c->ncells,
+                       (const int32_t *)nullptr, c->d_xyz, c->d_dofs, c->d_sign, c->d_dir, d_x, c->d_minv, c->d_ref,
+                       c->d_rowptr, c->d_rank, d_val, c->phys);
     MHD_HIP(hipGetLastError());
   } else {
     for (size_t k = 0; k + 1 < c->color_ptr.size(); ++k) {
       const int n = c->color_ptr[k + 1] - c->color_ptr[k];
       if (n == 0) continue;
-      hipLaunchKernelGGL((k_cell_jacobian<SCATTER_COLOUR>), dim3(n), dim3(WG), 0, s, n,
-                         c->d_color_cells + c->color_ptr[k], c->d_xyz, c->d_dofs, c->d_sign, c->d_dir, d_x, c->d_ref,
-                         c->d_rowptr, c->d_rank, d_val, c->phys);
+      hipLaunchKernelGGL((k_cell_jacobian<SCATTER_COLOUR>), dim3(jacobian_blocks(n)), dim3(WG), 0, s, n,
+                         c->d_color_cells + c->color_ptr[k], c->d_xyz, c->d_dofs, c->d_sign, c->d_dir, d_x, c->d_minv,
+                         c->d_ref, c->d_rowptr, c->d_rank, d_val, c->phys);
       MHD_HIP(hipGetLastError());
     }
   }
@@ -1364,8 +1199,8 @@ int mhd_launch_transpose_values(mhd_ctx *c, const double *d_val, double *d_val_t
 }
 
 int mhd_launch_cell_integrals(mhd_ctx *c, const double *d_x, double *d_out, hipStream_t s) {
-  hipLaunchKernelGGL(k_cell_integrals, dim3(c->ncells), dim3(WG), 0, s, c->ncells, c->d_xyz, c->d_dofs, c->d_sign,
-                     c->d_dir, d_x, c->d_ref, d_out, c->phys);
+  hipLaunchKernelGGL(k_cell_integrals, dim3((unsigned)((c->ncells + 1) / 2)), dim3(64), 0, s, c->ncells, c->d_xyz,
+                     c->d_dofs, c->d_sign, c->d_dir, d_x, d_out);
   MHD_HIP(hipGetLastError());
   return 0;
 }
