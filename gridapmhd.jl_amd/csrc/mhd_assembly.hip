@@ -143,7 +143,13 @@ __device__ inline void store_tile(const JacCell &S, const d4_t &acc, double scal
 //   jphi / phij = sum_q ws q1 div r                                      (K = 27)
 // The first version mapped the 27 + 36 basis functions to physical space at
 // every point: half of a cell's 124 K cycles went into that staging and jj took
-// K = 27 x 4.  JACFIG
+// K = 27 x 4.  At 64 x 64 x 8 the kernel went from 3.4 to 1.93 ms (22 TFLOP/s of
+// matrix instructions, the matrix unit 45 % busy), at 8 x 8 x 3 from 52 to 34 us,
+// one cell's serial chain.  It is bound by latency at two waves a SIMD (225
+// VGPRs): two accumulator chains in flight in the uu job instead of three cost
+// 6 %.  Writing the rows of one cell's own dofs straight into the CSR values
+// was tried: 1.93 -> 2.74 ms with a look-up for every row (2.34 for the p, phi
+// and interior j rows alone), more than the sums save (2.20 -> 1.65, 1.76 ms).
 template <int MODE>
 __global__ __launch_bounds__(WG, 2) void k_cell_jacobian(int ncells, const int32_t *__restrict__ cells,
                                                       const double *__restrict__ xyz,
@@ -175,22 +181,31 @@ __global__ __launch_bounds__(WG, 2) void k_cell_jacobian(int ncells, const int32
   if (tid < 9) S.wN[NQ][tid] = S.wx[NQ][tid] = S.wj[NQ][tid] = 0.0;
   if (tid < 6) S.wd[NQ][tid] = 0.0;
   if (tid == 0) S.wv[NQ] = S.ws[NQ] = 0.0;
+  // this thread's share of a cell's data
+  auto fetch = [&](int cell) {
+    const int c = cells ? cells[cell] : cell;
+    if (tid < NU) {
+      const int32_t g = dofs[(int64_t)c * NDOF + tid];
+      return g >= 0 ? x[g] : dir[-(int64_t)g - 1];
+    }
+    if (tid >= 96 && tid < 120) return xyz[(int64_t)c * 24 + tid - 96];
+    if (tid >= 128 && tid < 128 + NJ) {
+      const int i = tid - 128;
+      return sign && i % 12 < 8 ? (double)sign[(int64_t)c * 6 + (rt_local(i / 12, i % 12) >> 2)] : 1.0;
+    }
+    if (tid >= 192 && tid < 208) return minv[(int64_t)c * 16 + tid - 192];
+    return 0.0;
+  };
+  double pre = blockIdx.x < ncells ? fetch(blockIdx.x) : 0.0;
   for (int cell = blockIdx.x; cell < ncells; cell += gridDim.x) {
     const int c = cells ? cells[cell] : cell;
     const uint16_t *rk = rank + (int64_t)c * NENT;
     double *out = MODE == SCATTER_EBUF ? val + (int64_t)c * NENT : val;
-    // ---- the cell's data (the previous cell's tiles are done)
-    if (tid < NU) {
-      const int32_t g = dofs[(int64_t)c * NDOF + tid];
-      S.x[tid] = g >= 0 ? x[g] : dir[-(int64_t)g - 1];
-    } else if (tid < 128 && tid >= 96) {
-      if (tid < 120) S.xyz[tid - 96] = xyz[(int64_t)c * 24 + tid - 96];
-    } else if (tid >= 128 && tid < 128 + NJ) {
-      const int i = tid - 128;
-      S.sg[i] = sign && i % 12 < 8 ? (double)sign[(int64_t)c * 6 + (rt_local(i / 12, i % 12) >> 2)] : 1.0;
-    } else if (tid >= 192 && tid < 208) {
-      S.minv[tid - 192] = minv[(int64_t)c * 16 + tid - 192];
-    }
+    // ---- the cell's data, loaded during the previous cell (whose tiles are done)
+    if (tid < NU) S.x[tid] = pre;
+    else if (tid >= 96 && tid < 120) S.xyz[tid - 96] = pre;
+    else if (tid >= 128 && tid < 128 + NJ) S.sg[tid - 128] = pre;
+    else if (tid >= 192 && tid < 208) S.minv[tid - 192] = pre;
     if (MODE != SCATTER_EBUF && tid < NDOF) {
       const int32_t g = dofs[(int64_t)c * NDOF + tid];
       S.g[tid] = g;
@@ -241,6 +256,7 @@ __global__ __launch_bounds__(WG, 2) void k_cell_jacobian(int ncells, const int32
       }
     }
     __syncthreads();
+    if (cell + (int)gridDim.x < ncells) pre = fetch(cell + gridDim.x);
     // ---- S tile of the wave; the waves of the first column tile also form D
     const int ti = wave >> 1, tj = wave & 1;
     const int a = 16 * ti + li, b = 16 * tj + li;
@@ -353,24 +369,31 @@ __global__ __launch_bounds__(WG, 2) void k_cell_jacobian(int ncells, const int32
     }
     const int na = ti ? 11 : 16, nb = tj ? 11 : 16;
 #pragma unroll 1
-    for (int cd = 0; cd < 9; ++cd) {
-      const int cc = cd / 3, dd = cd % 3;
-      d4_t acc = cc == dd ? Sacc : zero;
-      if (ph.convection == 2) {
-        double wq[7];
+    for (int cc = 0; cc < 3; ++cc) {  // three independent MFMA chains
+      d4_t acc[3];
 #pragma unroll
-        for (int st = 0; st < 7; ++st) wq[st] = S.wN[4 * st + lk][cd] * qb[st];
+      for (int dd = 0; dd < 3; ++dd) acc[dd] = cc == dd ? Sacc : zero;
+      if (ph.convection == 2)
 #pragma unroll
-        for (int st = 0; st < 7; ++st) acc = mfma16(qa[st], wq[st], acc);
+        for (int st = 0; st < 7; ++st) {
+          const double *w = &S.wN[4 * st + lk][3 * cc];
+#pragma unroll
+          for (int dd = 0; dd < 3; ++dd) acc[dd] = mfma16(qa[st], w[dd] * qb[st], acc[dd]);
+        }
+      if (ph.zeta_u != 0.0) {
+        const double A = a < 27 ? S.D[lk][cc * 27 + a] : 0.0;
+#pragma unroll
+        for (int dd = 0; dd < 3; ++dd) acc[dd] = mfma16(A, b < 27 ? S.MD[lk][dd * 27 + b] : 0.0, acc[dd]);
       }
-      if (ph.zeta_u != 0.0)
-        acc = mfma16(a < 27 ? S.D[lk][cc * 27 + a] : 0.0, b < 27 ? S.MD[lk][dd * 27 + b] : 0.0, acc);
-      const int r0 = cc * 27 + 16 * ti, c0 = dd * 27 + 16 * tj;
-      store_tile<MODE>(S, acc, 1.0, na, nb, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
-        lr = r0 + i;
-        lc = c0 + j;
-        e = lr * ROWS_U_LEN + lc;
-      });
+#pragma unroll
+      for (int dd = 0; dd < 3; ++dd) {
+        const int r0 = cc * 27 + 16 * ti, c0 = dd * 27 + 16 * tj;
+        store_tile<MODE>(S, acc[dd], 1.0, na, nb, rk, out, [&](int i, int j, int &e, int &lr, int &lc) {
+          lr = r0 + i;
+          lc = c0 + j;
+          e = lr * ROWS_U_LEN + lc;
+        });
+      }
     }
     __syncthreads();
   }
