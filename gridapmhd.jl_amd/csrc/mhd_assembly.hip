@@ -681,7 +681,8 @@ __device__ inline void row_segment(int a, int &start, int &len) {
 // ranks of one segment are distinct and its lanes never collide in LDS.
 // All holders of a dof hold it as the same field, so the segments of a row
 // share one length (<= 125 = 2 x 64 lanes); up to RA_BATCH segments are loaded
-// into registers together before they are added in order.
+// into registers together before they are added in order.  In a context with a
+// skeleton term (sptr not null) the row's skeleton entries are added last.
 constexpr int RA_WAVES = 4;
 constexpr int RA_BATCH = 8;
 __global__ __launch_bounds__(64 * RA_WAVES) void k_row_assemble(int64_t n, const int64_t *__restrict__ rowptr,
@@ -689,6 +690,9 @@ __global__ __launch_bounds__(64 * RA_WAVES) void k_row_assemble(int64_t n, const
                                                                 const int32_t *__restrict__ centry,
                                                                 const double *__restrict__ ebuf,
                                                                 const uint16_t *__restrict__ rank,
+                                                                const int64_t *__restrict__ sptr,
+                                                                const uint16_t *__restrict__ srank,
+                                                                const double *__restrict__ sval,
                                                                 double *__restrict__ val, int maxrow) {
   extern __shared__ double ra_lds[];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -728,6 +732,11 @@ __global__ __launch_bounds__(64 * RA_WAVES) void k_row_assemble(int64_t n, const
         if (k1[u] != RANK_NONE) buf[k1[u]] += v1[u];
         __builtin_amdgcn_wave_barrier();
       }
+    }
+    if (sptr) {
+      const int64_t s1 = sptr[row + 1];
+      for (int64_t p = sptr[row] + lane; p < s1; p += 64) buf[srank[p]] += sval[p];
+      __builtin_amdgcn_wave_barrier();
     }
     for (int t = lane; t < len; t += 64) val[b + t] = buf[t];
     __builtin_amdgcn_wave_barrier();
@@ -938,71 +947,87 @@ __global__ void k_skel_res_gather(int64_t n, const int32_t *__restrict__ srow, c
   }
 }
 
-// Rank of every slot dof of an entry's face (same component) in the entry's
-// CSR row, found once at creation by binary search (RANK_NONE for non-free
-// slots).  One wave per row.
-__global__ __launch_bounds__(64) void k_skel_rank(int64_t n, const int64_t *__restrict__ rowptr,
+// Skeleton part of the matrix, constant for a context: every row's entries
+// (rank in the CSR row, sum of K_f[slot][b] over the row's skeleton entries in
+// increasing face order) are summed once at creation, and the Jacobian adds
+// them to the assembled rows.  Summing them from the face matrices in every
+// assembly read 420 MB at 21 x 17 x 5 (each K_f three times, a rank for each
+// entry) in chains of dependent loads: 212 us, against 85 MB for the sums, which
+// lengthen the row assembly from 157 to 186 us.
+// One wave per row; the slot dofs of one entry are distinct, so lanes never
+// collide.  The first pass (srank null) counts a row's entries into cnt, the
+// second writes them at sptr.  flag and buf share the LDS: max_row doubles.
+__device__ inline int skel_rank(const int32_t *colind, int64_t rb, int len, int32_t g) {
+  int lo = 0, hi = len;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (colind[rb + mid] < g) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo < len && colind[rb + lo] == g ? lo : -1;
+}
+
+__global__ __launch_bounds__(64) void k_skel_rows(int64_t n, const int64_t *__restrict__ rowptr,
                                                   const int32_t *__restrict__ colind, const int32_t *__restrict__ srow,
                                                   const int32_t *__restrict__ sentry,
-                                                  const int32_t *__restrict__ sdofs, uint16_t *__restrict__ rank) {
+                                                  const int32_t *__restrict__ sdofs, const double *__restrict__ K,
+                                                  int32_t *__restrict__ cnt, const int64_t *__restrict__ sptr,
+                                                  uint16_t *srank, double *__restrict__ sval) {
+  extern __shared__ double sk_lds[];
+  uint8_t *flag = reinterpret_cast<uint8_t *>(sk_lds);
   const int lane = threadIdx.x;
   for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
     const int p0 = srow[i], p1 = srow[i + 1];
-    if (p0 == p1) continue;
+    if (p0 == p1) {
+      if (!srank && lane == 0) cnt[i] = 0;
+      continue;
+    }
     const int64_t rb = rowptr[i];
     const int len = (int)(rowptr[i + 1] - rb);
-    for (int p = p0; p < p1; ++p) {
-      if (lane >= SKEL_SLOTS) continue;
-      const int32_t e = sentry[p];
-      const int f = e / SKEL_DOFS, comp = (e % SKEL_DOFS) / SKEL_SLOTS;
-      const int32_t g = sdofs[(int64_t)f * SKEL_DOFS + comp * SKEL_SLOTS + lane];
-      uint16_t rk = RANK_NONE;
-      if (g >= 0) {
-        int lo = 0, hi = len;
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (colind[rb + mid] < g) lo = mid + 1;
-          else hi = mid;
-        }
-        if (lo < len && colind[rb + lo] == g) rk = (uint16_t)lo;
+    auto each = [&](auto &&visit) {
+      for (int p = p0; p < p1; ++p) {
+        const int32_t e = sentry[p];
+        const int f = e / SKEL_DOFS, comp = (e % SKEL_DOFS) / SKEL_SLOTS, a = e % SKEL_SLOTS;
+        const int32_t g = lane < SKEL_SLOTS ? sdofs[(int64_t)f * SKEL_DOFS + comp * SKEL_SLOTS + lane] : -1;
+        const int rk = g >= 0 ? skel_rank(colind, rb, len, g) : -1;
+        if (rk >= 0) visit(rk, ((int64_t)f * SKEL_SLOTS + a) * SKEL_SLOTS + lane);
+        __syncthreads();
       }
-      rank[(int64_t)p * SKEL_SLOTS + lane] = rk;
+    };
+    for (int t = lane; t < len; t += 64) flag[t] = 0;
+    __syncthreads();
+    each([&](int rk, int64_t) { flag[rk] = 1; });
+    int m = 0;
+    for (int t0 = 0; t0 < len; t0 += 64) {
+      const bool on = t0 + lane < len && flag[t0 + lane];
+      const uint64_t mask = __ballot(on);
+      if (srank && on) srank[sptr[i] + m + __popcll(mask & ((1ull << lane) - 1))] = (uint16_t)(t0 + lane);
+      m += __popcll(mask);
     }
+    __syncthreads();
+    if (!srank) {
+      if (lane == 0) cnt[i] = m;
+      continue;
+    }
+    for (int t = lane; t < len; t += 64) sk_lds[t] = 0.0;
+    __syncthreads();
+    each([&](int rk, int64_t k) { sk_lds[rk] += K[k]; });
+    __threadfence_block();
+    for (int t = lane; t < m; t += 64) sval[sptr[i] + t] = sk_lds[srank[sptr[i] + t]];
+    __syncthreads();
   }
 }
 
-// Skeleton rows of the Jacobian, added to the assembled CSR values: one
-// 64-lane wave per row; the row is accumulated in LDS (lane b adds K_f[slot][b]
-// at the rank of slot b's dof, from the rank table -- the slot dofs of one
-// entry are distinct, so lanes never collide), entries in increasing face
-// order, then added to the row once.
-__global__ __launch_bounds__(64) void k_skel_jacobian(int64_t n, const int64_t *__restrict__ rowptr,
-                                                      const int32_t *__restrict__ srow,
-                                                      const int32_t *__restrict__ sentry,
-                                                      const uint16_t *__restrict__ rank,
-                                                      const double *__restrict__ K, double *__restrict__ val) {
-  extern __shared__ double sk_lds[];
-  const int lane = threadIdx.x;
-  for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
-    const int p0 = srow[i], p1 = srow[i + 1];
-    if (p0 == p1) continue;
-    const int64_t rb = rowptr[i];
-    const int len = (int)(rowptr[i + 1] - rb);
-    for (int t = lane; t < len; t += 64) sk_lds[t] = 0.0;
-    __builtin_amdgcn_wave_barrier();
-    for (int p = p0; p < p1; ++p) {
-      if (lane < SKEL_SLOTS) {
-        const uint16_t rk = rank[(int64_t)p * SKEL_SLOTS + lane];
-        if (rk != RANK_NONE) {
-          const int32_t e = sentry[p];
-          const int f = e / SKEL_DOFS, a = (e % SKEL_DOFS) % SKEL_SLOTS;
-          sk_lds[rk] += K[((int64_t)f * SKEL_SLOTS + a) * SKEL_SLOTS + lane];
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-    for (int t = lane; t < len; t += 64) val[rb + t] += sk_lds[t];
-    __builtin_amdgcn_wave_barrier();
+// The skeleton rows added to CSR values that other kernels wrote (k_row_assemble
+// adds them itself): one wave per row.
+__global__ __launch_bounds__(256) void k_skel_add(int64_t n, const int64_t *__restrict__ rowptr,
+                                                  const int64_t *__restrict__ sptr,
+                                                  const uint16_t *__restrict__ srank,
+                                                  const double *__restrict__ sval, double *__restrict__ val) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t i = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); i < n; i += (int64_t)gridDim.x * 4) {
+    const int64_t p1 = sptr[i + 1], rb = rowptr[i];
+    for (int64_t p = sptr[i] + lane; p < p1; p += 64) val[rb + srank[p]] += sval[p];
   }
 }
 
@@ -1014,6 +1039,10 @@ __global__ __launch_bounds__(64) void k_skel_jacobian(int64_t n, const int64_t *
 static unsigned jacobian_blocks(int ncells) { return (unsigned)std::min(ncells, 2048); }
 
 int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_t s) {
+  if (c->nskel > 0 && c->max_row > SKEL_MAX_ROW) {
+    c->err = "skeleton Jacobian: a CSR row longer than 8192 entries";
+    return -1;
+  }
   // a cell holding one dof twice (a periodic direction one cell thick) needs
   // the atomic scatter: its own entries may coincide
   int mode = c->dup_dofs ? 0 : c->assembly_mode;
@@ -1028,7 +1057,8 @@ int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_
       const int64_t blocks = std::min<int64_t>((c->n + RA_WAVES - 1) / RA_WAVES, 1 << 20);
       const size_t lds = sizeof(double) * (size_t)RA_WAVES * c->max_row;
       hipLaunchKernelGGL(k_row_assemble, dim3((unsigned)blocks), dim3(64 * RA_WAVES), lds, s, c->n, c->d_rowptr,
-                         c->d_crow, c->d_centry, c->d_ebuf, c->d_rank, d_val, c->max_row);
+                         c->d_crow, c->d_centry, c->d_ebuf, c->d_rank, c->d_skel_ptr, c->d_skel_rank, c->d_skel_val,
+                         d_val, c->max_row);
       MHD_HIP(hipGetLastError());
     }
   } else {
@@ -1056,7 +1086,13 @@ int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_
                        c->d_sign, c->d_fcell, c->d_flf, c->d_fK, c->d_rowptr, c->d_rank, d_val);
     MHD_HIP(hipGetLastError());
   }
-  return mhd_launch_skeleton_jacobian(c, d_val, s);
+  if (mode != 2 && c->nskel > 0 && c->n > 0) {
+    const int64_t blocks = std::min<int64_t>((c->n + 3) / 4, 1 << 20);
+    hipLaunchKernelGGL(k_skel_add, dim3((unsigned)blocks), dim3(256), 0, s, c->n, c->d_rowptr, c->d_skel_ptr,
+                       c->d_skel_rank, c->d_skel_val, d_val);
+    MHD_HIP(hipGetLastError());
+  }
+  return 0;
 }
 
 int mhd_assemble_own(mhd_ctx *c, hipStream_t s) {
@@ -1079,16 +1115,37 @@ int mhd_build_skeleton(mhd_ctx *c, const int32_t *d_fcell, const int8_t *d_flf, 
   if (c->nskel <= 0) return 0;
   MHD_HIP(hipMalloc(&c->d_skel_K, sizeof(double) * (size_t)c->nskel * SKEL_SLOTS * SKEL_SLOTS));
   MHD_HIP(hipMalloc(&c->d_skel_res, sizeof(double) * (size_t)c->nskel * SKEL_DOFS));
-  MHD_HIP(hipMalloc(&c->d_skel_rank, sizeof(uint16_t) * (size_t)std::max<int64_t>(c->nsentry, 1) * SKEL_SLOTS));
   const int blocks = std::min(c->nskel, 1 << 20);
   hipLaunchKernelGGL(k_skel_matrix, dim3(blocks), dim3(64), 0, c->stream, c->nskel, c->d_xyz, d_fcell, d_flf,
                      d_fperm, d_mslot, d_mu, c->d_fref, c->d_skel_K);
   MHD_HIP(hipGetLastError());
-  if (c->n > 0) {
-    hipLaunchKernelGGL(k_skel_rank, dim3((unsigned)std::min<int64_t>(c->n, 1 << 20)), dim3(64), 0, c->stream, c->n,
-                       c->d_rowptr, c->d_colind, c->d_srow, c->d_sentry, c->d_skel_dofs, c->d_skel_rank);
-    MHD_HIP(hipGetLastError());
-  }
+  if (c->n <= 0 || c->max_row > SKEL_MAX_ROW) return 0;  // the Jacobian refuses longer rows
+  int32_t *d_cnt = nullptr;
+  MHD_HIP(hipMalloc(&d_cnt, sizeof(int32_t) * (size_t)c->n));
+  std::vector<int32_t> cnt((size_t)c->n);
+  std::vector<int64_t> ptr((size_t)c->n + 1, 0);
+  const dim3 grid((unsigned)std::min<int64_t>(c->n, 1 << 20));
+  const size_t lds = sizeof(double) * (size_t)c->max_row;
+  hipLaunchKernelGGL(k_skel_rows, grid, dim3(64), lds, c->stream, c->n, c->d_rowptr, c->d_colind, c->d_srow,
+                     c->d_sentry, c->d_skel_dofs, c->d_skel_K, d_cnt, (const int64_t *)nullptr, (uint16_t *)nullptr,
+                     (double *)nullptr);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(cnt.data(), d_cnt, sizeof(int32_t) * (size_t)c->n, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  (void)hipFree(d_cnt);
+  MHD_HIP(e);
+  for (int64_t i = 0; i < c->n; ++i) ptr[i + 1] = ptr[i] + cnt[i];
+  const size_t m = (size_t)std::max<int64_t>(ptr[c->n], 1);
+  MHD_HIP(hipMalloc(&c->d_skel_ptr, sizeof(int64_t) * ptr.size()));
+  MHD_HIP(hipMalloc(&c->d_skel_rank, sizeof(uint16_t) * m));
+  MHD_HIP(hipMalloc(&c->d_skel_val, sizeof(double) * m));
+  MHD_HIP(hipMemcpyAsync(c->d_skel_ptr, ptr.data(), sizeof(int64_t) * ptr.size(), hipMemcpyHostToDevice, c->stream));
+  hipLaunchKernelGGL(k_skel_rows, grid, dim3(64), lds, c->stream, c->n, c->d_rowptr, c->d_colind, c->d_srow,
+                     c->d_sentry, c->d_skel_dofs, c->d_skel_K, (int32_t *)nullptr, c->d_skel_ptr, c->d_skel_rank,
+                     c->d_skel_val);
+  MHD_HIP(hipGetLastError());
+  MHD_HIP(hipStreamSynchronize(c->stream));
   return 0;
 }
 
@@ -1099,20 +1156,6 @@ int mhd_launch_skeleton_residual(mhd_ctx *c, const double *d_x, double *d_r, hip
   const int64_t blocks = std::min<int64_t>((c->n + 255) / 256, 65536);
   hipLaunchKernelGGL(k_skel_res_gather, dim3((unsigned)blocks), dim3(256), 0, s, c->n, c->d_srow, c->d_sentry,
                      c->d_skel_res, d_r);
-  MHD_HIP(hipGetLastError());
-  return 0;
-}
-
-int mhd_launch_skeleton_jacobian(mhd_ctx *c, double *d_val, hipStream_t s) {
-  if (c->nskel <= 0 || c->n <= 0) return 0;
-  const size_t lds = sizeof(double) * (size_t)c->max_row;
-  if (lds > 65536) {
-    c->err = "skeleton Jacobian: a CSR row longer than 8192 entries";
-    return -1;
-  }
-  const int64_t blocks = std::min<int64_t>(c->n, 1 << 20);
-  hipLaunchKernelGGL(k_skel_jacobian, dim3((unsigned)blocks), dim3(64), lds, s, c->n, c->d_rowptr, c->d_srow,
-                     c->d_sentry, c->d_skel_rank, c->d_skel_K, d_val);
   MHD_HIP(hipGetLastError());
   return 0;
 }

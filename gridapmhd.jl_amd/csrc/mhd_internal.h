@@ -52,6 +52,7 @@ struct FaceTables {
 // cell (slots 0..26) and those of the second cell not shared with the first
 // (slot 27 + local node); SKEL_NONE marks the unused slots.
 constexpr int SKEL_SLOTS = 54;
+constexpr int SKEL_MAX_ROW = 8192;  // longest CSR row of a stabilised Jacobian (64 KiB of LDS)
 constexpr int SKEL_DOFS = 3 * SKEL_SLOTS;   // [component][slot]
 constexpr int32_t SKEL_NONE = INT32_MIN;
 
@@ -143,8 +144,10 @@ struct mhd_ctx {
   double *d_skel_K = nullptr;         // [nskel][54][54] face matrices of one velocity component
   int32_t *d_srow = nullptr;          // [n + 1] skeleton entries of each row
   int32_t *d_sentry = nullptr;        // face * SKEL_DOFS + component * 54 + slot, increasing face order per row
-  int64_t nsentry = 0;                // entries over all rows
-  uint16_t *d_skel_rank = nullptr;    // [nsentry][54] rank of each slot dof of the entry's face in the entry's row
+  // the skeleton part of the matrix: entries of row i at [skel_ptr[i], skel_ptr[i + 1])
+  int64_t *d_skel_ptr = nullptr;      // [n + 1]
+  uint16_t *d_skel_rank = nullptr;    // rank of each entry in its CSR row
+  double *d_skel_val = nullptr;
   double *d_skel_res = nullptr;       // [nskel][SKEL_DOFS] the face products K_f x_c of the last residual
   // solver workspace (allocated lazily)
   struct Solver *solver = nullptr;
@@ -228,7 +231,6 @@ int mhd_launch_residual_noalloc(mhd_ctx *c, const double *d_x, double *d_r, hipS
 int mhd_build_skeleton(mhd_ctx *c, const int32_t *d_fcell, const int8_t *d_flf, const int8_t *d_fperm,
                        const uint8_t *d_mslot, const double *d_mu);
 int mhd_launch_skeleton_residual(mhd_ctx *c, const double *d_x, double *d_r, hipStream_t s);
-int mhd_launch_skeleton_jacobian(mhd_ctx *c, double *d_val, hipStream_t s);
 
 #define MHD_HIP(call)                                                                 \
   do {                                                                                \
