@@ -673,18 +673,63 @@ __device__ inline void row_segment(int a, int &start, int &len) {
   }
 }
 
-// Row assembly from the element buffer: one 64-lane wave per CSR row.  The row
-// is accumulated in LDS -- every (cell, local row) holding the row's dof adds
-// its contiguous element-buffer segment at the entries' ranks, in increasing
-// cell order -- and then written once, coalesced.  Every entry of the row is
-// written, so val needs no clearing.  A cell holds a dof at most once, so the
-// ranks of one segment are distinct and its lanes never collide in LDS.
-// All holders of a dof hold it as the same field, so the segments of a row
-// share one length (<= 125 = 2 x 64 lanes); up to RA_BATCH segments are loaded
-// into registers together before they are added in order.  In a context with a
-// skeleton term (sptr not null) the row's skeleton entries are added last.
+// Row assembly from the element buffer: one 64-lane wave per CSR row at a time.
+// The row is accumulated in LDS -- every (cell, local row) holding the row's dof
+// adds its contiguous element-buffer segment at the entries' ranks, in
+// increasing cell order -- and then written once, coalesced.  Every entry of
+// the row is written, so val needs no clearing.  A cell holds a dof at most
+// once, so the ranks of one segment are distinct and its lanes never collide in
+// LDS.  All holders of a dof hold it as the same field, so the segments of a
+// row share one length (<= 125 = 2 x 64 lanes).  In a context with a skeleton
+// term (sptr not null) the row's skeleton entries are added last.
+//
+// It streams 10 bytes for an element entry and 8 for a CSR entry.  Four of five
+// rows have one or two holders, too little to keep in flight for a wave that
+// ends each row before it loads the next, so a wave runs through rows with the
+// next row's first RA_BATCH segments already loading, and a row of one holder,
+// which has no sums, goes to its place without the LDS: 2.19 -> 2.09 ms at
+// 64 x 64 x 8 (8.2 GB, 3.9 TB/s; 4.3 with the parts of cache lines beside the
+// segments, against 4.9 of a copy), 186 -> 148 us at 21 x 17 x 5 with the
+// skeleton term.  One round of workgroups (7 fit a CU by their LDS).
 constexpr int RA_WAVES = 4;
-constexpr int RA_BATCH = 8;
+constexpr int RA_BATCH = 4;
+constexpr int RA_BLOCKS = 256 * 8;
+struct RowMeta {
+  int64_t b;
+  int len, p0, p1;
+};
+struct RowSegs {
+  double v0[RA_BATCH], v1[RA_BATCH];
+  int k0[RA_BATCH], k1[RA_BATCH];
+};
+__device__ inline RowMeta row_meta(int64_t row, int64_t n, const int64_t *__restrict__ rowptr,
+                                   const int32_t *__restrict__ crow) {
+  if (row >= n) return RowMeta{0, 0, 0, 0};
+  return RowMeta{rowptr[row], (int)(rowptr[row + 1] - rowptr[row]), crow[row], crow[row + 1]};
+}
+__device__ inline void row_load(RowSegs &S, int pb, int p1, int lane, const int32_t *__restrict__ centry,
+                                const double *__restrict__ ebuf, const uint16_t *__restrict__ rank) {
+#pragma unroll
+  for (int u = 0; u < RA_BATCH; ++u) {
+    S.k0[u] = S.k1[u] = RANK_NONE;
+    S.v0[u] = S.v1[u] = 0.0;
+    if (pb + u < p1) {
+      const int32_t ce = centry[pb + u];
+      const int cell = ce / NDOF, a = ce - cell * NDOF;
+      int start, slen;
+      row_segment(a, start, slen);
+      const int64_t base = (int64_t)cell * NENT + start;
+      if (lane < slen) {
+        S.k0[u] = rank[base + lane];
+        S.v0[u] = ebuf[base + lane];
+      }
+      if (lane + 64 < slen) {
+        S.k1[u] = rank[base + lane + 64];
+        S.v1[u] = ebuf[base + lane + 64];
+      }
+    }
+  }
+}
 __global__ __launch_bounds__(64 * RA_WAVES) void k_row_assemble(int64_t n, const int64_t *__restrict__ rowptr,
                                                                 const int32_t *__restrict__ crow,
                                                                 const int32_t *__restrict__ centry,
@@ -695,51 +740,52 @@ __global__ __launch_bounds__(64 * RA_WAVES) void k_row_assemble(int64_t n, const
                                                                 const double *__restrict__ sval,
                                                                 double *__restrict__ val, int maxrow) {
   extern __shared__ double ra_lds[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   double *buf = ra_lds + (size_t)wave * maxrow;
-  for (int64_t row = (int64_t)blockIdx.x * RA_WAVES + wave; row < n; row += (int64_t)gridDim.x * RA_WAVES) {
-    const int64_t b = rowptr[row];
-    const int len = (int)(rowptr[row + 1] - b);
-    const int p0 = crow[row], p1 = crow[row + 1];
-    for (int t = lane; t < len; t += 64) buf[t] = 0.0;
+  auto finish = [&](int64_t row, const RowMeta &m, RowSegs &S) {
+    if (row >= n) return;
+    if (m.p1 - m.p0 == 1 && !sptr) {
+      if (S.k0[0] != RANK_NONE) val[m.b + S.k0[0]] = S.v0[0];
+      if (S.k1[0] != RANK_NONE) val[m.b + S.k1[0]] = S.v1[0];
+      return;
+    }
+    for (int t = lane; t < m.len; t += 64) buf[t] = 0.0;
     __builtin_amdgcn_wave_barrier();
-    for (int pb = p0; pb < p1; pb += RA_BATCH) {
-      double v0[RA_BATCH], v1[RA_BATCH];
-      uint16_t k0[RA_BATCH], k1[RA_BATCH];
+    for (int pb = m.p0;;) {
 #pragma unroll
       for (int u = 0; u < RA_BATCH; ++u) {
-        k0[u] = k1[u] = RANK_NONE;
-        v0[u] = v1[u] = 0.0;
-        if (pb + u < p1) {
-          const int32_t ce = centry[pb + u];
-          const int cell = ce / NDOF, a = ce - cell * NDOF;
-          int start, slen;
-          row_segment(a, start, slen);
-          const int64_t base = (int64_t)cell * NENT + start;
-          if (lane < slen) {
-            k0[u] = rank[base + lane];
-            v0[u] = ebuf[base + lane];
-          }
-          if (lane + 64 < slen) {
-            k1[u] = rank[base + lane + 64];
-            v1[u] = ebuf[base + lane + 64];
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < RA_BATCH; ++u) {
-        if (k0[u] != RANK_NONE) buf[k0[u]] += v0[u];
-        if (k1[u] != RANK_NONE) buf[k1[u]] += v1[u];
+        if (pb + u >= m.p1) break;
+        if (S.k0[u] != RANK_NONE) buf[S.k0[u]] += S.v0[u];
+        if (S.k1[u] != RANK_NONE) buf[S.k1[u]] += S.v1[u];
         __builtin_amdgcn_wave_barrier();
       }
+      pb += RA_BATCH;
+      if (pb >= m.p1) break;
+      row_load(S, pb, m.p1, lane, centry, ebuf, rank);
     }
     if (sptr) {
       const int64_t s1 = sptr[row + 1];
       for (int64_t p = sptr[row] + lane; p < s1; p += 64) buf[srank[p]] += sval[p];
       __builtin_amdgcn_wave_barrier();
     }
-    for (int t = lane; t < len; t += 64) val[b + t] = buf[t];
+    for (int t = lane; t < m.len; t += 64) val[m.b + t] = buf[t];
     __builtin_amdgcn_wave_barrier();
+  };
+  const int64_t step = (int64_t)gridDim.x * RA_WAVES;
+  int64_t row = (int64_t)blockIdx.x * RA_WAVES + wave;
+  RowSegs A, B;
+  RowMeta ma = row_meta(row, n, rowptr, crow), mb = row_meta(row + step, n, rowptr, crow);
+  row_load(A, ma.p0, ma.p1, lane, centry, ebuf, rank);
+  while (row < n) {
+    row_load(B, mb.p0, mb.p1, lane, centry, ebuf, rank);
+    RowMeta next = row_meta(row + 2 * step, n, rowptr, crow);
+    finish(row, ma, A);
+    ma = next;
+    row_load(A, ma.p0, ma.p1, lane, centry, ebuf, rank);
+    next = row_meta(row + 3 * step, n, rowptr, crow);
+    finish(row + step, mb, B);
+    mb = next;
+    row += 2 * step;
   }
 }
 
@@ -953,7 +999,7 @@ __global__ void k_skel_res_gather(int64_t n, const int32_t *__restrict__ srow, c
 // them to the assembled rows.  Summing them from the face matrices in every
 // assembly read 420 MB at 21 x 17 x 5 (each K_f three times, a rank for each
 // entry) in chains of dependent loads: 212 us, against 85 MB for the sums, which
-// lengthen the row assembly from 157 to 186 us.
+// cost the row assembly 29 us.
 // One wave per row; the slot dofs of one entry are distinct, so lanes never
 // collide.  The first pass (srank null) counts a row's entries into cnt, the
 // second writes them at sptr.  flag and buf share the LDS: max_row doubles.
@@ -1054,7 +1100,7 @@ int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_
                        c->d_rowptr, c->d_rank, c->d_ebuf, c->phys);
     MHD_HIP(hipGetLastError());
     if (c->n > 0) {
-      const int64_t blocks = std::min<int64_t>((c->n + RA_WAVES - 1) / RA_WAVES, 1 << 20);
+      const int64_t blocks = std::min<int64_t>((c->n + RA_WAVES - 1) / RA_WAVES, RA_BLOCKS);
       const size_t lds = sizeof(double) * (size_t)RA_WAVES * c->max_row;
       hipLaunchKernelGGL(k_row_assemble, dim3((unsigned)blocks), dim3(64 * RA_WAVES), lds, s, c->n, c->d_rowptr,
                          c->d_crow, c->d_centry, c->d_ebuf, c->d_rank, c->d_skel_ptr, c->d_skel_rank, c->d_skel_val,
