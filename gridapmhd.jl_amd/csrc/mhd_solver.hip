@@ -293,10 +293,16 @@ __global__ void k_set_diag(int64_t n, double v, double *__restrict__ D) {
 // each block column K of width BGJ_B, P = A_KK^-1 (one workgroup, pivoting
 // inside its 32 x 32 diagonal blocks), then the rank-BGJ_B update
 //   A <- A - A[:,K] P A[K,:],  A[K,:] <- P A[K,:],  A[:,K] <- -A[:,K] P,  A_KK <- P
-// on FP64 GEMMs (2 n^3 flops in all, like an LU plus triangular solves, but in
-// n / BGJ_B wide GEMM steps instead of one panel kernel per column).  Pivoting
-// is inside the diagonal blocks only; the result is checked by a residual and
-// redone with the row-pivoted LU if it fails.
+// (2 n^3 flops in all, like an LU plus triangular solves).  Pivoting is inside
+// the diagonal blocks only; the result is checked by a residual and redone with
+// the row-pivoted LU if it fails.
+// Two launches a block column: k_gj_panel writes C = -A[:,K] and R = P A[K,:]
+// with R[:,K] = P, so that k_gj_update is A += C R with zero for A[:,K] and R
+// for A[K,:].  The next diagonal block needs only its own part of the update,
+// so the first workgroup of k_gj_update forms and inverts it while the others
+// update: the chain of pivots (73 us a block) hides behind the update.  A block
+// column of a 4144-block takes 95 + 20 us; with library products, the copies
+// between them and the inverse in its turn it took 181 (8.0 -> 5.1 ms in all).
 constexpr int BGJ_B = 96;
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
@@ -314,13 +320,13 @@ __device__ inline double read_lane(double v, int lane) {
   return __hiloint2double(hi, lo);
 }
 
-// One wave inverts the 32 x 32 block A (LDS) into P: Gauss-Jordan with the
+// One wave inverts the 32 x 32 block A (LDS) in place: Gauss-Jordan with the
 // block in registers (lane = row + 32 half, 16 columns each), no workgroup
 // barrier.  A diagonal pivot is taken unless an unused row holds an entry ten
 // times larger, then the largest.
 constexpr int SB = 32;
-__device__ inline void wave_inverse(const double *__restrict__ A, int lda, double (*P)[SB + 1], double *prow, int *pk,
-                                    int lane, int32_t *__restrict__ flag) {
+__device__ inline void wave_inverse(double *A, int lda, double *prow, int *pk, int lane,
+                                    int32_t *__restrict__ flag) {
   const int r = lane & 31, h = lane >> 5;
   double a[16];
 #pragma unroll
@@ -369,73 +375,254 @@ __device__ inline void wave_inverse(const double *__restrict__ A, int lda, doubl
   }
   // A^-1[k][pk[c]] = S[pk[k]][c]
 #pragma unroll
-  for (int j = 0; j < 16; ++j) P[kof][pk[16 * h + j]] = a[j];
+  for (int j = 0; j < 16; ++j) A[kof * lda + pk[16 * h + j]] = a[j];
 }
 
-// One 1024-thread workgroup inverts the kb x kb (kb <= BGJ_B = 96) block in
-// LDS by block Gauss-Jordan with 32 x 32 diagonal blocks (wave_inverse) and
-// FP64 MFMA tiles for their updates.  The chain of pivots is what bounds it:
-// a step of one wave in registers costs a sixth of a step of the whole
-// workgroup with its four barriers (a 96-block took 200 us, now 60).
-__global__ __launch_bounds__(1024) void k_block_inv(int64_t ld, int kb, const double *__restrict__ Mkk,
-                                                    double *__restrict__ Pout, int32_t *__restrict__ flag) {
-  static_assert(BGJ_B == 96, "three 32-blocks; 16 waves cover the 4 x 4 tiles outside one of them");
-  __shared__ double A[BGJ_B][BGJ_B + 1];
-  __shared__ double T[SB][BGJ_B + 1];
-  __shared__ double P[SB][SB + 1];
-  __shared__ double prow[SB];
-  __shared__ int pk[SB];
+// One workgroup inverts a kb x kb (kb <= BGJ_B = 96) block in LDS by block
+// Gauss-Jordan with 32 x 32 diagonal blocks (wave_inverse) and FP64 MFMA tiles
+// for their updates.  The chain of pivots is what bounds it: a step of one wave
+// in registers costs a sixth of a step of the whole workgroup with its four
+// barriers (a 96-block took 200 us, now 60).  The block is src (leading
+// dimension ld); P [96 x 96] is padded by the identity.
+constexpr int GJ_T = 512;
+struct GJBlock {
+  double A[BGJ_B][BGJ_B + 1];
+  double prow[SB];
+  int pk[SB];
+};
+__device__ __forceinline__ void invert_block(GJBlock &S, const double *__restrict__ src, int64_t ld, int kb,
+                                             double *__restrict__ Pout, int32_t *__restrict__ flag) {
+  static_assert(BGJ_B == 96 && SB == 32 && GJ_T == 512, "4 x 4 tiles outside a 32-block, two for each of 8 waves");
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
-  for (int e = tid; e < BGJ_B * BGJ_B; e += 1024) {
-    const int i = e % BGJ_B, j = e / BGJ_B;
-    A[i][j] = i < kb && j < kb ? Mkk[i + (int64_t)j * ld] : (i == j ? 1.0 : 0.0);
+#pragma unroll
+  for (int u = 0; u < BGJ_B * BGJ_B / GJ_T; ++u) {
+    const int e = tid + u * GJ_T, i = e % BGJ_B, j = e / BGJ_B;
+    S.A[i][j] = i < kb && j < kb ? src[i + (int64_t)j * ld] : (i == j ? 1.0 : 0.0);
   }
   __syncthreads();
   for (int s0 = 0; s0 < kb; s0 += SB) {
-    if (wave == 0) wave_inverse(&A[s0][s0], BGJ_B + 1, P, prow, pk, lane, flag);
+    if (wave == 0) wave_inverse(&S.A[s0][s0], BGJ_B + 1, S.prow, S.pk, lane, flag);
     __syncthreads();
     // tile t = 0..3 of the 16-wide tiles outside the block
     auto outside = [&](int t) { return 16 * t + (16 * t >= s0 ? SB : 0); };
-    if (wave < 8) {  // T = P A[s][:]
-      const int i0 = 16 * (wave & 1), j0 = outside(wave >> 1);
+    {  // A[s][:] <- P A[s][:]
+      const int i0 = s0 + 16 * (wave & 1), j0 = outside(wave >> 1);
       d4_t acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int k = 0; k < SB; k += 4)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(P[i0 + li][k + lk], A[s0 + k + lk][j0 + li], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(S.A[i0 + li][s0 + k + lk], S.A[s0 + k + lk][j0 + li], acc, 0, 0, 0);
+      __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 4; ++q) T[i0 + lk + 4 * q][j0 + li] = acc[q];
+      for (int q = 0; q < 4; ++q) S.A[i0 + lk + 4 * q][j0 + li] = acc[q];
     }
     __syncthreads();
-    {  // A[i][j] -= A[i][s] T[:][j] outside the block
-      const int i0 = outside(wave & 3), j0 = outside(wave >> 2);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {  // A[i][j] -= A[i][s] A[s][j] outside the block
+      const int i0 = outside(wave & 3), j0 = outside((wave >> 2) + 2 * h);
       d4_t acc;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = A[i0 + lk + 4 * q][j0 + li];
+      for (int q = 0; q < 4; ++q) acc[q] = S.A[i0 + lk + 4 * q][j0 + li];
 #pragma unroll
       for (int k = 0; k < SB; k += 4)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-A[i0 + li][s0 + k + lk], T[k + lk][j0 + li], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-S.A[i0 + li][s0 + k + lk], S.A[s0 + k + lk][j0 + li], acc, 0, 0,
+                                                   0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) A[i0 + lk + 4 * q][j0 + li] = acc[q];
+      for (int q = 0; q < 4; ++q) S.A[i0 + lk + 4 * q][j0 + li] = acc[q];
     }
-    d4_t col = {0.0, 0.0, 0.0, 0.0};  // -A[i][s] P, written once every wave has read A[i][s]
-    const int ci = outside(wave & 3), cj = 16 * ((wave >> 2) & 1);
-    if (wave < 8) {
+    // A[i][s] <- -A[i][s] P, written once every wave has read A[i][s]
+    d4_t col = {0.0, 0.0, 0.0, 0.0};
+    const int ci = outside(wave & 3), cj = s0 + 16 * (wave >> 2);
 #pragma unroll
-      for (int k = 0; k < SB; k += 4)
-        col = __builtin_amdgcn_mfma_f64_16x16x4f64(-A[ci + li][s0 + k + lk], P[k + lk][cj + li], col, 0, 0, 0);
-    }
+    for (int k = 0; k < SB; k += 4)
+      col = __builtin_amdgcn_mfma_f64_16x16x4f64(-S.A[ci + li][s0 + k + lk], S.A[s0 + k + lk][cj + li], col, 0, 0, 0);
     __syncthreads();
-    if (wave < 8) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) A[ci + lk + 4 * q][s0 + cj + li] = col[q];
-    }
-    for (int e = tid; e < SB * BGJ_B; e += 1024) {
-      const int i = e / BGJ_B, j = e % BGJ_B;
-      A[s0 + i][j] = j >= s0 && j < s0 + SB ? P[i][j - s0] : T[i][j];
-    }
+    for (int q = 0; q < 4; ++q) S.A[ci + lk + 4 * q][cj + li] = col[q];
     __syncthreads();
   }
-  for (int e = tid; e < kb * kb; e += 1024) Pout[e] = A[e % kb][e / kb];
+  for (int e = tid; e < BGJ_B * BGJ_B; e += GJ_T) Pout[e] = S.A[e % BGJ_B][e / BGJ_B];
+}
+
+__global__ __launch_bounds__(GJ_T) void k_block_inv(int64_t m, int kb, const double *__restrict__ M,
+                                                    double *__restrict__ P, int32_t *__restrict__ flag) {
+  __shared__ GJBlock S;
+  invert_block(S, M, m, kb, P, flag);
+}
+
+// C = -M[:,K], R = P M[K,:] with R[:,K] = P (both [k][m], zero for k >= kb); 32
+// columns (and rows of C) per workgroup.  The workgroups of the next block's
+// columns also form that block after the update, D (kd x kd in [96 x 96]).
+constexpr int GJ_PC = 32;
+__global__ __launch_bounds__(GJ_T) void k_gj_panel(int64_t m, int64_t k0, int kb, int kd, const double *__restrict__ M,
+                                                  const double *__restrict__ P, double *__restrict__ C,
+                                                  double *__restrict__ R, double *__restrict__ D) {
+  __shared__ double S[GJ_PC][BGJ_B + 1], Q[BGJ_B][BGJ_B + 1];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int64_t j0 = (int64_t)blockIdx.x * GJ_PC;
+  const int64_t k1 = k0 + BGJ_B;
+#pragma unroll
+  for (int u = 0; u < BGJ_B * BGJ_B / GJ_T; ++u) {
+    const int e = tid + u * GJ_T;
+    Q[e / BGJ_B][e % BGJ_B] = P[e];
+  }
+#pragma unroll
+  for (int u = 0; u < GJ_PC * BGJ_B / GJ_T; ++u) {
+    const int e = tid + u * GJ_T, k = e % BGJ_B, j = e / BGJ_B;
+    S[j][k] = k < kb && j0 + j < m ? M[k0 + k + (j0 + j) * m] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < GJ_PC * BGJ_B / GJ_T; ++u) {
+    const int e = tid + u * GJ_T, k = e / GJ_PC;
+    const int64_t i = j0 + e % GJ_PC;
+    if (i < m) C[k * m + i] = k < kb ? -M[i + (k0 + k) * m] : 0.0;
+  }
+  double ck[BGJ_B * BGJ_B / GJ_T];
+  const bool next = j0 >= k1 && j0 < k1 + kd;
+  if (next) {
+#pragma unroll
+    for (int u = 0; u < BGJ_B * BGJ_B / GJ_T; ++u) {
+      const int e = tid + u * GJ_T, i = e % BGJ_B, k = e / BGJ_B;
+      ck[u] = i < kd && k < kb ? -M[k1 + i + (k0 + k) * m] : 0.0;
+    }
+  }
+  __syncthreads();
+  d4_t rt[2] = {};
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {  // 6 x 2 tiles
+    const int t = wave + q * (GJ_T / 64), i0 = 16 * (t >> 1), c0 = 16 * (t & 1);
+    if (t >= 12) break;
+    d4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+    for (int k = 0; k < BGJ_B; k += 4)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Q[k + lk][i0 + li], S[c0 + li][k + lk], acc, 0, 0, 0);
+    rt[q] = acc;
+    const int64_t j = j0 + c0 + li;
+    if (j >= m) continue;
+    const bool in = j >= k0 && j < k0 + kb;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = i0 + lk + 4 * r;
+      R[k * m + j] = in ? Q[j - k0][k] : acc[r];
+    }
+  }
+  if (!next) return;
+  static_assert(BGJ_B % GJ_PC == 0, "a workgroup's columns lie inside or outside the next block");
+  __syncthreads();
+  // D = M[K1, j] + C[K1, :] R[:, j]: C's rows take P's place, R's columns M's
+#pragma unroll
+  for (int u = 0; u < BGJ_B * BGJ_B / GJ_T; ++u) Q[(tid + u * GJ_T) / BGJ_B][(tid + u * GJ_T) % BGJ_B] = ck[u];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int t = wave + q * (GJ_T / 64);
+    if (t < 12) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[16 * (t & 1) + li][16 * (t >> 1) + lk + 4 * r] = rt[q][r];
+    }
+  }
+  __syncthreads();
+  for (int t = wave; t < 12; t += GJ_T / 64) {
+    const int i0 = 16 * (t >> 1), c0 = 16 * (t & 1);
+    const int64_t j = j0 + c0 + li;
+    d4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + lk + 4 * r;
+      if (i < kd && j < m) acc[r] = M[k1 + i + j * m];
+    }
+#pragma unroll 8
+    for (int k = 0; k < BGJ_B; k += 4)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Q[k + lk][i0 + li], S[c0 + li][k + lk], acc, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) D[i0 + lk + 4 * r + BGJ_B * (j - k1)] = acc[r];
+  }
+}
+
+// M += C R outside [K,:], M[:,K] counted as zero and M[K,:] = R; one 48 x 48 tile
+// per wave, straight from L2 (9 matrix instructions, 576 cycles, for 6 loads of
+// 512 bytes); 4 x 2 waves of a workgroup share its rows and columns in L1.  At
+// 4144 it takes 86 us, 95 with the inverse: 47 to move M in and out (275 MB, as
+// measured with one k step) and the products, 43 at the matrix unit's rate,
+// which overlap little (starting half of the waves with the products changed
+// nothing).  Workgroup 0 inverts the next block (kd > 0).
+constexpr int GJ_W = 48;
+__global__ __launch_bounds__(GJ_T, 4) void k_gj_update(int64_t m, int64_t k0, int kb, int kd,
+                                                       const double *__restrict__ C, const double *__restrict__ R,
+                                                       const double *__restrict__ D, double *__restrict__ P,
+                                                       int32_t *__restrict__ flag, double *__restrict__ M) {
+  __shared__ GJBlock S;
+  static_assert(BGJ_B % GJ_W == 0, "a wave's tile lies inside or outside K");
+  if (blockIdx.x == 0) {
+    __builtin_amdgcn_s_setprio(3);
+    if (kd > 0) invert_block(S, D, BGJ_B, kd, P, flag);
+    return;
+  }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const unsigned ni = (unsigned)((m + 4 * GJ_W - 1) / (4 * GJ_W)), b = blockIdx.x - 1;
+  const int64_t i0 = ((int64_t)(b % ni) * 4 + (wave & 3)) * GJ_W, j0 = ((int64_t)(b / ni) * 2 + (wave >> 2)) * GJ_W;
+  if (i0 >= m || j0 >= m) return;
+  if (i0 >= k0 && i0 < k0 + BGJ_B) {
+    for (int e = lane; e < GJ_W * GJ_W; e += 64) {
+      const int64_t i = i0 + e % GJ_W, j = j0 + e / GJ_W;
+      if (i < m && j < m) M[i + j * m] = R[(i - k0) * m + j];
+    }
+    return;
+  }
+  // the tile transposed: D row (l / 16 + 4 r) is a column of M, its 16 lanes rows
+  const bool skip = j0 >= k0 && j0 < k0 + BGJ_B;
+  int64_t ii[3], jj[3];
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    ii[t] = min(i0 + 16 * t + li, m - 1);
+    jj[t] = min(j0 + 16 * t + li, m - 1);
+  }
+  d4_t acc[3][3];
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        acc[t][u][r] = skip ? 0.0 : M[ii[u] + min(j0 + 16 * t + lk + 4 * r, m - 1) * m];
+  // operands one step ahead; the barriers keep the compiler from moving the
+  // loads down to their use
+  const double *Ck = C + lk * m, *Rk = R + lk * m;
+  double a[2][3], c[2][3];
+  auto load = [&](int h) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      a[h][t] = Rk[jj[t]];
+      c[h][t] = Ck[ii[t]];
+    }
+    Ck += 4 * m;
+    Rk += 4 * m;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](int h) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[h][t], c[h][u], acc[t][u], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  load(0);
+  for (int k = 0; k < kb; k += 8) {  // C and R are zero in [kb, BGJ_B)
+    load(1);
+    multiply(0);
+    if (k + 8 < kb) load(0);
+    multiply(1);
+  }
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t i = i0 + 16 * u + li, j = j0 + 16 * t + lk + 4 * r;
+        if (i < m && j < m) M[i + j * m] = acc[t][u][r];
+      }
+  }
 }
 
 // b_i = deterministic values in [-1/2, 1/2) + 1 (the check's right-hand side)
@@ -1939,13 +2126,6 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
   if ((rc = dmalloc(c, &S->d_pstatus, (size_t)S->npatch))) return rc;
   if ((rc = dmalloc(c, &S->d_rt, (size_t)S->n1))) return rc;
   if ((rc = dmalloc(c, &S->d_cflag, 1))) return rc;
-  if (rocblas_create_handle(&S->rb) != rocblas_status_success) {
-    c->err = "rocblas_create_handle failed";
-    return -2;
-  }
-  rocblas_set_stream(S->rb, c->stream);
-  // the same bits in every run: no atomics inside rocBLAS / rocSOLVER routines
-  rocblas_set_atomics_mode(S->rb, rocblas_atomics_not_allowed);
   // Krylov workspace
   S->m = krylov_dim(o->restart);
   S->kin = std::max(0, std::min(o->inner_iters, 120));
@@ -2573,8 +2753,7 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     // row-major (the layout of the row-dot product).  The row-major copy of the
     // block S is the column-major S^T; block Gauss-Jordan inverts it in place
     // into (S^T)^-1, whose column-major storage is S^-1 row-major.
-    const Solver *SC = cc->solver;
-    rocblas_handle rb = SC->rb;  // bound to cs, the stream of every level
+    Solver *SC = cc->solver;
     if (!L->d_Ainv) {
       std::vector<int32_t> bidx, bmap(L->n1c, -1), ones(cc->ncells, 1);
       std::vector<uint8_t> elim(L->n1c);
@@ -2585,7 +2764,7 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
           bidx.push_back((int32_t)i);
         }
       const int64_t m = L->nb = (int64_t)bidx.size();
-      const int64_t nw = 2 * m * BGJ_B + (int64_t)BGJ_B * BGJ_B + 3 * m + 2;
+      const int64_t nw = 2 * m * BGJ_B + 2 * (int64_t)BGJ_B * BGJ_B + 3 * m + 2;
       MHD_HIP(hipMalloc(&L->d_bidx, sizeof(int32_t) * (size_t)std::max<int64_t>(m, 1)));
       MHD_HIP(hipMalloc(&L->d_bmap, sizeof(int32_t) * (size_t)L->n1c));
       MHD_HIP(hipMalloc(&L->d_ones, sizeof(int32_t) * (size_t)cc->ncells));
@@ -2616,31 +2795,20 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     MHD_HIP(hipMemcpyAsync(L->d_Ainv, L->d_LU, sizeof(double) * (size_t)(m * m), hipMemcpyDeviceToDevice, cs));
     MHD_HIP(hipMemsetAsync(L->d_gjflag, 0, sizeof(int32_t), cs));
     double *M = L->d_Ainv, *C = L->d_gjw, *R = C + m * BGJ_B, *P = R + m * BGJ_B;
-    double *vb = P + (int64_t)BGJ_B * BGJ_B, *vy = vb + m, *vz = vy + m, *chk = vz + m;
-    const double one = 1.0, zero = 0.0, mone = -1.0;
-    const rocblas_operation N = rocblas_operation_none;
-    bool blas_ok = true;
-    for (int64_t k0 = 0; k0 < m && blas_ok; k0 += BGJ_B) {
+    double *D = P + (int64_t)BGJ_B * BGJ_B;
+    double *vb = D + (int64_t)BGJ_B * BGJ_B, *vy = vb + m, *vz = vy + m, *chk = vz + m;
+    if (m > 0)
+      hipLaunchKernelGGL(k_block_inv, dim3(1), dim3(GJ_T), 0, cs, m, (int)std::min<int64_t>(BGJ_B, m), M, P,
+                         L->d_gjflag);
+    const unsigned panels = (unsigned)((m + GJ_PC - 1) / GJ_PC);
+    const unsigned tiles = (unsigned)(((m + 4 * GJ_W - 1) / (4 * GJ_W)) * ((m + 2 * GJ_W - 1) / (2 * GJ_W)));
+    for (int64_t k0 = 0; k0 < m; k0 += BGJ_B) {
       const int kb = (int)std::min<int64_t>(BGJ_B, m - k0);
-      const rocblas_int rm = (rocblas_int)m, rkb = kb;
-      hipLaunchKernelGGL(k_block_inv, dim3(1), dim3(1024), 0, cs, m, kb, M + k0 + k0 * m, P, L->d_gjflag);
-      MHD_HIP(hipGetLastError());
-      MHD_HIP(hipMemcpyAsync(C, M + k0 * m, sizeof(double) * (size_t)(m * kb), hipMemcpyDeviceToDevice, cs));
-      blas_ok = rocblas_dgemm(rb, N, N, rkb, rm, rkb, &one, P, rkb, M + k0, rm, &zero, R, rkb) ==
-                    rocblas_status_success &&
-                rocblas_dgemm(rb, N, N, rm, rm, rkb, &mone, C, rm, R, rkb, &one, M, rm) == rocblas_status_success;
-      if (!blas_ok) break;
-      MHD_HIP(hipMemcpy2DAsync(M + k0, sizeof(double) * m, R, sizeof(double) * kb, sizeof(double) * kb, m,
-                               hipMemcpyDeviceToDevice, cs));
-      blas_ok = rocblas_dgemm(rb, N, N, rm, rkb, rkb, &mone, C, rm, P, rkb, &zero, M + k0 * m, rm) ==
-                rocblas_status_success;
-      MHD_HIP(hipMemcpy2DAsync(M + k0 + k0 * m, sizeof(double) * m, P, sizeof(double) * kb, sizeof(double) * kb, kb,
-                               hipMemcpyDeviceToDevice, cs));
+      const int kd = (int)std::max<int64_t>(0, std::min<int64_t>(BGJ_B, m - k0 - BGJ_B));
+      hipLaunchKernelGGL(k_gj_panel, dim3(panels), dim3(GJ_T), 0, cs, m, k0, kb, kd, M, P, C, R, D);
+      hipLaunchKernelGGL(k_gj_update, dim3(tiles + 1), dim3(GJ_T), 0, cs, m, k0, kb, kd, C, R, D, P, L->d_gjflag, M);
     }
-    if (!blas_ok) {
-      c->err = "rocblas_dgemm of the coarsest block Gauss-Jordan failed";
-      return -2;
-    }
+    MHD_HIP(hipGetLastError());
     // check: z = A (A^-1 b) against b for a fixed b
     hipLaunchKernelGGL(k_check_rhs, dim3(nblocks(m)), dim3(TB), 0, cs, m, vb);
     hipLaunchKernelGGL((k_dense_rowdot<double>), dim3((unsigned)m), dim3(TB), 0, cs, m, M, vb,
@@ -2663,6 +2831,17 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
       MHD_HIP(hipMemsetAsync(M, 0, sizeof(double) * (size_t)(m * m), cs));
       hipLaunchKernelGGL(k_set_diag, dim3(nblocks(m)), dim3(TB), 0, cs, m, 1.0, M);
       MHD_HIP(hipGetLastError());
+      if (!SC->rb) {
+        if (rocblas_create_handle(&SC->rb) != rocblas_status_success) {
+          SC->rb = nullptr;
+          c->err = "rocblas_create_handle failed";
+          return -2;
+        }
+        rocblas_set_stream(SC->rb, cs);
+        // the same bits in every run: no atomics inside rocSOLVER routines
+        rocblas_set_atomics_mode(SC->rb, rocblas_atomics_not_allowed);
+      }
+      rocblas_handle rb = SC->rb;
       if (rocsolver_dgetrf(rb, (rocblas_int)m, (rocblas_int)m, L->d_LU, (rocblas_int)m, L->d_piv, L->d_info) !=
               rocblas_status_success ||
           rocsolver_dgetrs(rb, rocblas_operation_none, (rocblas_int)m, (rocblas_int)m, L->d_LU, (rocblas_int)m,
