@@ -1064,8 +1064,10 @@ __global__ __launch_bounds__(256) void k_cond_rhs(int64_t n1, const int32_t *__r
 // wave per cell: it gathers yb of its dofs into LDS (the cell that is the first
 // holder of a dof writes it), then takes the E rows l = s, s + 5, ... on lanes
 // i + 12 s, coalesced.  One launch and no yb vector; the product sums are read
-// 2.7 times (75 MB at 32,768 cells), E once: 92 us there, 11 us on 200 cells,
-// where two launches (sums, then interiors) took 26 + 72 and 6 + 11 us.
+// 2.7 times (75 MB at 32,768 cells), E once: 94 us there, 9 us on 200 cells,
+// where two launches (sums, then interiors) took 26 + 72 and 6 + 11 us.  Small
+// levels are one chain of dependent loads: a dof at a time took 11 us, all
+// eight products of two dofs 8, but 110 on the large one (registers).
 constexpr int CG_CELLS = 4;
 template <class T, class TE>
 __global__ __launch_bounds__(64 * CG_CELLS) void k_cond_gather(
@@ -1087,21 +1089,57 @@ __global__ __launch_bounds__(64 * CG_CELLS) void k_cond_gather(
   if (c < ncells) {
     const int32_t *cd = dofs + (int64_t)c * NDOF;
     const int nl = f0 < 0 ? NB + NI : NB;
-    for (int k = lane; k < nl; k += 64) {
-      const int l = k < NU ? (k % 3) * 27 + k / 3 : k;  // node by node: neighbouring lanes read neighbouring sums
-      const int a = bdof_local(l);
-      const int32_t id = cd[a];
-      double s = 0.0;
-      if (id >= 0 && id < n1) {
-        const int32_t b = dptr[id], e = dptr[id + 1];
-        for (int32_t q = b; q < e; q += 4) {  // four products in flight
+    for (int k0 = lane; k0 < nl; k0 += 128) {
+      // two dofs a lane and four products of each (only the cell's central node
+      // lies in more stars) requested together: one chain of dependent loads
+      int32_t id[2], b[2], n[2], h[2], at[2][4];
+      double pv[2][4];
+      int loc[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int k = min(k0 + 64 * u, nl - 1);
+        const int l = k < NU ? (k % 3) * 27 + k / 3 : k;  // node by node: neighbouring lanes read neighbouring sums
+        loc[u] = l;
+        const int32_t g = cd[bdof_local(l)];
+        id[u] = k0 + 64 * u < nl && g >= 0 && g < n1 ? g : -1;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        b[u] = n[u] = 0;
+        h[u] = -1;
+        if (id[u] >= 0) {
+          b[u] = dptr[id[u]];
+          n[u] = dptr[id[u] + 1] - b[u];
+          h[u] = crow[id[u]];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q < n[u]) at[u][q] = dent[b[u] + q];
+        if (h[u] >= 0) h[u] = centry[h[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) pv[u][q] = q < n[u] ? part[at[u][q]] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (k0 + 64 * u >= nl) continue;
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += pv[u][q];
+        for (int32_t q = b[u] + 4, e = b[u] + n[u]; q < e; q += 4) {
           const double p0 = part[dent[q]], p1 = q + 1 < e ? part[dent[q + 1]] : 0.0;
           const double p2 = q + 2 < e ? part[dent[q + 2]] : 0.0, p3 = q + 3 < e ? part[dent[q + 3]] : 0.0;
           s = (((s + p0) + p1) + p2) + p3;
         }
-        if (centry[crow[id]] == c * NDOF + a) y[id] = accumulate ? (T)((double)y[id] + w * s) : (T)(w * s);
+        const int32_t g = id[u];
+        if (g >= 0 && h[u] == c * NDOF + bdof_local(loc[u]))
+          y[g] = accumulate ? (T)((double)y[g] + w * s) : (T)(w * s);
+        if (loc[u] < NB) yb[wave][loc[u]] = s;
       }
-      if (l < NB) yb[wave][l] = s;
     }
   }
   __syncthreads();
