@@ -1146,7 +1146,8 @@ int mhd_assemble_own(mhd_ctx *c, hipStream_t s) {
   int rc = mhd_launch_jacobian(c, c->d_x, c->d_val, s);
   if (!rc && c->nskel == 0) rc = mhd_cellop_state(c, c->d_x, s);
   if (rc) return rc;
-  if (!c->d_sbuf && c->nskel == 0 && c->own_stream &&  // not on coarse levels, which make no products for callers
+  // not on coarse levels, which make no products for callers
+  if (!c->d_sbuf && c->nskel == 0 && c->nnz >= APPLY_NNZ && c->own_stream &&
       hipMalloc(&c->d_sbuf, sizeof(double) * (size_t)c->ncells * NDOF) != hipSuccess) {
     c->d_sbuf = nullptr;
     (void)hipGetLastError();
@@ -1355,8 +1356,8 @@ int mhd_build_tperm(mhd_ctx *c) {
   return 0;
 }
 
-// y = A x with the Jacobian in d_val.  Without a skeleton term the form is
-// applied cell by cell (48 x 40 x 8: 439 us streamed, 63 us applied).
+// y = A x with the Jacobian in d_val.  Without a skeleton term, and from
+// APPLY_NNZ nonzeros on, the form is applied cell by cell.
 // That needs a buffer of element results, so it belongs to the first stream
 // that calls; calls on any other stream, which may overlap it, stream the
 // matrix as before, and so does a context whose buffer could not be allocated.

@@ -73,3 +73,35 @@ def test_spmv_is_the_assembled_jacobian(nc, convection, stab, orc_mod):
     finally:
         ctx.close()
         hip().hipStreamDestroy(other)
+
+
+@pytest.mark.parametrize("nc", [(12, 10, 4), (12, 12, 4), (13, 11, 5)])
+def test_spmv_routes_agree_around_their_line(nc):
+    """Below 5M nonzeros both streams stream the matrix (the same bits), from
+    there on the first stream applies the form: sums of at most 700 products in
+    another order, on rows of entries of one size."""
+    import ctypes
+    import gridapmhd_amd as g
+    from devmem import DeviceArray, hip
+    from gridapmhd_amd import adjoint
+    sp, phys = adjoint.inlet_duct(nc, 20.0, 5.0, 0.05, convection="newton", jitter=0.15)
+    rng = np.random.default_rng(9)
+    x, v = 0.3 * rng.standard_normal(sp.ndofs), rng.standard_normal(sp.ndofs)
+    other = ctypes.c_void_p()
+    ctx = g._lib.context_from_spaces(sp, phys)
+    try:
+        assert hip().hipStreamCreate(ctypes.byref(other)) == 0
+        dx, dv, dy = DeviceArray.from_numpy(x), DeviceArray.from_numpy(v), DeviceArray.from_numpy(np.zeros(sp.ndofs))
+        ctx.jacobian_d(dx.ptr)
+        hip().hipDeviceSynchronize()
+        y = {}
+        for stream in (0, other.value):
+            dy.copy_from(np.full(sp.ndofs, np.nan))
+            ctx.spmv_d(dv.ptr, dy.ptr, stream)
+            y[stream] = dy.numpy().copy()
+        err = np.linalg.norm(y[0] - y[other.value]) / np.linalg.norm(y[0])
+        print(f"[spmv routes] {nc}: nnz {ctx.nnz}, {err:.2e}", flush=True)
+        assert (err == 0.0) == (ctx.nnz < 5000000) and err < 1e-13
+    finally:
+        ctx.close()
+        hip().hipStreamDestroy(other)
