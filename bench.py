@@ -42,11 +42,11 @@ FP64_PEAK_TFS = 78.6
 # rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (KiB per dispatch) over
 # `bench.py --kernels-only`, each scaled by what the counter reads for a 1 GiB
 # device-to-device copy (FETCH_SIZE x 2, WRITE_SIZE x 1).  The smoother
-# entries cover one application: k_patch_apply + k_patch_gather.
-C2_TRAFFIC = {"smoother_f32": 6.907e9, "smoother_f64": 1.4046e10, "spmv_f64": 5.991e9, "jacobian": 1.3641e10}
+# entries cover one application: k_cond_rhs + k_patch_apply + k_cond_gather.
+C2_TRAFFIC = {"smoother_f32": 3.095e9, "smoother_f64": 5.616e9, "spmv_f64": 5.990e9, "jacobian": 1.3515e10}
 # k_cell_jacobian at 64 x 64 x 8: SQ_INSTS_VALU_MFMA_MOPS_F64 x 512 flops and
 # SQ_VALU_MFMA_BUSY_CYCLES / (GRBM_GUI_ACTIVE per XCD x 1024 SIMDs), same runs.
-C2_JACOBIAN_MFMA = {"executed_flops": 5.979e10, "mfma_busy_frac": 0.231, "cell_kernel_ms": 3.341}
+C2_JACOBIAN_MFMA = {"executed_flops": 5.838e10, "mfma_busy_frac": 0.453, "cell_kernel_ms": 1.734}
 
 
 def log(msg):
@@ -443,16 +443,19 @@ def main():
     ctx.jacobian_d(x.data_ptr(), 0, sh)          # into the context: the Jacobian the set-up factors
     torch.cuda.synchronize()
     n1 = sp.nfree["u"] + sp.nfree["j"]
-    t_sm = {}
+    t_sm, sm_bytes = {}, {}
+    esize = {0: 8, 1: 4, 2: 2, 3: 2}
     for prec, dt in ((0, torch.float64), (args.mixed, torch.float32)):
         ctx.precond_setup(opts(prec, 1e-8, 1e-9, 10))
         rr = torch.rand(n1, dtype=dt, device=dev)
         yy = torch.zeros(n1, dtype=dt, device=dev)
+        ctx.op_counts(reset=True)
         ctx.smoother_apply_d(rr.data_ptr(), yy.data_ptr(), sh)
+        # bytes of one application: condensed patch inverses and cell couplings
+        sm_bytes[prec] = esize[prec] * sum(v for k, v in ctx.op_counts(reset=True).items()
+                                           if k.startswith("patch_entries"))
         t_sm[prec] = time_events(lambda: ctx.smoother_apply_d(rr.data_ptr(), yy.data_ptr(), sh), 10, stream)
-    npatch, pdim, pent, npiv = ctx.smoother_info(pivoted=True)
-    esize = {0: 8, 1: 4, 2: 2, 3: 2}
-    sm_bytes = {p: pent * esize[p] for p in t_sm}
+    npatch, pdim, _, npiv = ctx.smoother_info(pivoted=True)
     log(f"smoother apply FP64 {t_sm[0] * 1e3:.3f} ms ({sm_bytes[0] / t_sm[0] / 1e9:.0f} GB/s), "
         f"mixed {t_sm[args.mixed] * 1e3:.3f} ms ({sm_bytes[args.mixed] / t_sm[args.mixed] / 1e9:.0f} GB/s), "
         f"npatch={npatch} dim={pdim} partial-pivoting patches={npiv}")
@@ -519,11 +522,11 @@ def main():
         "asm_residual_ms": round(t_res * 1e3, 4),
         "residual_cells_per_s": round(ncells / t_res, 1),
         # the dominant kernel of the mixed Newton step: the fine-level smoother
-        "roofline": roof(f"k_patch_apply<{'float' if args.mixed == 1 else 'bf16'}> + k_patch_gather: one "
-                         f"vertex-star Schwarz application, fine level ({npatch} patches; bytes = the patch "
-                         f"inverses)", sm_bytes[args.mixed], t_sm[args.mixed],
+        "roofline": roof(f"k_cond_rhs + k_patch_apply<{'float' if args.mixed == 1 else 'bf16'}> + k_cond_gather: "
+                         f"one vertex-star Schwarz application, fine level ({npatch} patches; bytes = the condensed "
+                         f"patch inverses and the cells' couplings)", sm_bytes[args.mixed], t_sm[args.mixed],
                          "smoother_f32" if args.mixed == 1 else None),
-        "roofline_kernels": [roof("k_patch_apply<double> + k_patch_gather, fine level", sm_bytes[0], t_sm[0],
+        "roofline_kernels": [roof("k_cond_rhs + k_patch_apply<double> + k_cond_gather, fine level", sm_bytes[0], t_sm[0],
                                   "smoother_f64"),
                              roof("k_spmv fp64 CSR", spmv_bytes, t_spmv, "spmv_f64"),
                              jac_roof],
