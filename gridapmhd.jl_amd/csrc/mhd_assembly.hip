@@ -952,7 +952,8 @@ __global__ __launch_bounds__(64) void k_skel_matrix(int nf, const double *__rest
 // same products in the same order), so the loads are coalesced.
 // k_skel_res_gather: one thread per row adds the face products of the row's
 // (face, component, slot) entries, whose index is the product's own index, in
-// increasing face order: the sums do not depend on the launch.
+// increasing face order: the sums do not depend on the launch.  Up to 36 faces
+// a row, one load after another 24 us at 21 x 17 x 5, eight at a time 16.
 __global__ __launch_bounds__(64) void k_skel_face_product(int nf, const int32_t *__restrict__ sdofs,
                                                           const double *__restrict__ K, const double *__restrict__ x,
                                                           const double *__restrict__ dir, double *__restrict__ fres) {
@@ -988,7 +989,18 @@ __global__ void k_skel_res_gather(int64_t n, const int32_t *__restrict__ srow, c
     const int p0 = srow[i], p1 = srow[i + 1];
     if (p0 == p1) continue;
     double acc = 0.0;
-    for (int p = p0; p < p1; ++p) acc += fres[sentry[p]];
+    int p = p0;
+    for (; p + 8 <= p1; p += 8) {  // eight products in flight, added in order
+      int32_t e[8];
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) e[u] = sentry[p + u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = fres[e[u]];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += v[u];
+    }
+    for (; p < p1; ++p) acc += fres[sentry[p]];
     r[i] += acc;
   }
 }

@@ -187,7 +187,7 @@ struct CoarseLink {
   double *d_Ainv = nullptr;        // [nb][nb]
   double *d_LU = nullptr;          // [nb][nb] the condensed block, then its LU factors (set-up scratch)
   int32_t *d_piv = nullptr, *d_info = nullptr;
-  double *d_gjw = nullptr;         // block Gauss-Jordan workspace (column and row panels, pivot block, check)
+  double *d_gjw = nullptr;         // block Gauss-Jordan workspace (panels, pivot block, next block, check)
   int32_t *d_gjflag = nullptr;     // set when a diagonal block of the block Gauss-Jordan has a zero pivot
   int dense_fallbacks = 0;         // coarsest inversions redone with the pivoted LU
   double omega = 0.175;            // damping of the Schwarz smoother inside the V-cycle
