@@ -134,7 +134,7 @@ struct mhd_ctx {
   int64_t nhold = 0;                  // crow[n]
   int32_t max_row = 0;                // longest CSR row
   double *d_ebuf = nullptr;           // [ncells][NENT] element buffer (allocated on first use)
-  double *d_rbuf = nullptr;           // [ncells][NDOF] element results (allocated on first use)
+  double *d_rbuf = nullptr;           // [ncells][NDOF] element results of the residual (allocated on first use)
   // cell-wise application of the form (mhd_cellop.hip)
   int32_t *d_gslot = nullptr;         // [crow[n]] element-result slots of every dof's holders
   double *d_minv = nullptr;           // [ncells][16] inverse dP1 mass matrices

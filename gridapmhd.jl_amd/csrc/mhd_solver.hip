@@ -1873,8 +1873,11 @@ struct Solver {
   double pent = 0.0, pcube = 0.0;
   double ops[MHD_NOPS] = {};
   // products without the matrix (mhd_cellop_apply); with a skeleton term they
-  // stream it instead, through the row groups below
+  // stream it instead, through the row groups below.  Their element results have
+  // a buffer of their own: the context's belongs to mhd_residual_d, which may be
+  // pending on a caller's stream.
   bool matfree = true;
+  double *d_prod = nullptr;           // [ncells][NDOF]
   // row groups sharing a column list (k_spmv_grp): all rows, and the first
   // ngroups11 groups cover the [u,j] rows exactly
   int64_t ngroups = 0, ngroups11 = 0;
@@ -2391,7 +2394,7 @@ int a11_product(mhd_ctx *c, const T *x, const T *v, T *y, int prec) {
   if (S->matfree) {
     count(c, prec == 0 ? OP_SPMV64 : OP_SPMV32, (double)S->nnz11);
     return mhd_cellop_apply<T>(c, MHD_OP_UJ, S->transposed, op_scale(c), x, MODE == 3 ? v : (const T *)nullptr, y,
-                               c->d_rbuf, c->stream);
+                               S->d_prod, c->stream);
   }
   constexpr int LPG = 16;
   const int grid = (int)((S->ngroups11 * LPG + 255) / 256);
@@ -2412,7 +2415,7 @@ int full_product(mhd_ctx *c, const double *x, double *y) {
   if (S->matfree) {
     count(c, OP_SPMV64, (double)c->nnz);
     return mhd_cellop_apply<double>(c, MHD_OP_FULL, S->transposed, op_scale(c), x, (const double *)nullptr, y,
-                                    c->d_rbuf, c->stream);
+                                    S->d_prod, c->stream);
   }
   constexpr int LPG = 16;
   const int grid = (int)((S->ngroups * LPG + 255) / 256);
@@ -2584,7 +2587,7 @@ int precond(mhd_ctx *c, const double *v, double *z, int prec) {
   double *rhs1 = prec == 0 ? (double *)S->r1 : S->t1;
   count(c, OP_SPMV64, (double)S->nnz1x);
   if (S->matfree) {
-    if ((rc = mhd_cellop_apply<double>(c, MHD_OP_PPHI, S->transposed, op_scale(c), z, v, rhs1, c->d_rbuf,
+    if ((rc = mhd_cellop_apply<double>(c, MHD_OP_PPHI, S->transposed, op_scale(c), z, v, rhs1, S->d_prod,
                                        c->stream))) return rc;
   } else {
     constexpr int LPR = 16;
@@ -2751,7 +2754,7 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     S->alpha_phi = aphi;
   }
   if (S->matfree) {
-    if (!c->d_rbuf) MHD_HIP(hipMalloc(&c->d_rbuf, sizeof(double) * (size_t)c->ncells * NDOF));
+    if (!S->d_prod && (rc = dmalloc(c, &S->d_prod, (size_t)c->ncells * NDOF))) return rc;
   } else if (prec >= 1)
     hipLaunchKernelGGL((k_convert<double, float>), dim3(nblocks(c->nnz)), dim3(TB), 0, c->stream, c->nnz, c->d_val,
                        S->d_val32);
@@ -2988,7 +2991,7 @@ void mhd_solver_free(mhd_ctx *c) {
                   S->d_pA32, S->d_pA16, S->d_pAh, S->d_pscale, S->d_pperm, S->d_pstatus, S->d_pscratch, S->d_val32, S->V, S->Z, S->w, S->b, S->dx, S->t1,
                   S->V1, S->Z1, S->w1, S->x1, S->r1, S->d_part, S->d_dots, S->d_y, S->d_dptr, S->d_dent,
                   S->d_ppart, S->d_grow, S->d_gcp, S->d_gcol, S->d_pcptr, S->d_pcell, S->d_ifirst, S->d_npat, S->d_elim,
-                  S->d_cE64, S->d_cB64, S->d_cF64, S->d_cG64, S->d_cE32, S->d_cF32, S->d_cG32, S->d_cflag, S->d_rt};
+                  S->d_cE64, S->d_cB64, S->d_cF64, S->d_cG64, S->d_cE32, S->d_cF32, S->d_cG32, S->d_cflag, S->d_rt, S->d_prod};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (S->h_dots) (void)hipHostFree(S->h_dots);

@@ -174,7 +174,12 @@ int mhd_cell_integrals(mhd_ctx *ctx, const double *x_free, double *out);
  * is structurally symmetric, so CSR(A) and CSC(A) share index arrays and the
  * CSC values are CSR(A^T).  mhd_jacobian_d with d_nzval_csr = NULL assembles
  * into the context's own storage (and keeps d_x as its state): the Jacobian
- * that mhd_precond_setup and mhd_spmv_d use. */
+ * that mhd_precond_setup and mhd_spmv_d use.
+ * Residuals of one context share a buffer of element results, and so do its
+ * Jacobians: calls of one kind that overlap on different streams race, and a
+ * pending mhd_residual_d races with mhd_newton_solve (its own residuals) and
+ * mhd_residual, a pending mhd_jacobian_d with every solve and mhd_jacobian.  A
+ * pending mhd_residual_d beside mhd_linear_solve or mhd_adjoint_solve is safe. */
 int mhd_residual_d(mhd_ctx *ctx, const double *d_x, double *d_r, void *stream);
 int mhd_jacobian_d(mhd_ctx *ctx, const double *d_x, double *d_nzval_csr, void *stream);
 int mhd_csr_arrays(mhd_ctx *ctx, const int64_t **d_rowptr, const int32_t **d_colind);
