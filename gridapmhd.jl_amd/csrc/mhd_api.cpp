@@ -311,7 +311,7 @@ int mhd_create_stabilized(mhd_ctx **out, const mhd_mesh *mesh, const mhd_spaces 
   MHD_HIP(hipMalloc(&c->d_val, sizeof(double) * std::max<int64_t>(c->nnz, 1)));
   MHD_HIP(hipMalloc(&c->d_x, sizeof(double) * std::max<int64_t>(n, 1)));
   MHD_HIP(hipMalloc(&c->d_r, sizeof(double) * std::max<int64_t>(n, 1)));
-  if ((rc = mhd_build_face_matrices(c)) || (rc = mhd_cellop_build(c))) return rc;
+  if ((rc = mhd_build_face_matrices(c)) || (rc = mhd_cellop_build(c, nskel == 0))) return rc;
   if (nskel > 0) {
     // skeleton entries of every row, in increasing face order
     std::vector<int32_t> srow(n + 1, 0);

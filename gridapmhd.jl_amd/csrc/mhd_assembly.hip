@@ -1158,12 +1158,6 @@ int mhd_assemble_own(mhd_ctx *c, hipStream_t s) {
   int rc = mhd_launch_jacobian(c, c->d_x, c->d_val, s);
   if (!rc && c->nskel == 0) rc = mhd_cellop_state(c, c->d_x, s);
   if (rc) return rc;
-  // not on coarse levels, which make no products for callers
-  if (!c->d_sbuf && c->nskel == 0 && c->nnz >= APPLY_NNZ && c->own_stream &&
-      hipMalloc(&c->d_sbuf, sizeof(double) * (size_t)c->ncells * NDOF) != hipSuccess) {
-    c->d_sbuf = nullptr;
-    (void)hipGetLastError();
-  }
   c->jac_phys = c->phys;
   c->jac_valid = true;
   return 0;
@@ -1374,7 +1368,7 @@ int mhd_build_tperm(mhd_ctx *c) {
 // that calls; calls on any other stream, which may overlap it, stream the
 // matrix as before, and so does a context whose buffer could not be allocated.
 int mhd_launch_spmv(mhd_ctx *c, const double *d_x, double *d_y, hipStream_t s) {
-  if (c->jac_valid && c->nskel == 0 && c->d_sbuf) {
+  if (c->jac_valid && c->d_sbuf && c->own_stream) {  // coarse levels make no products for callers
     if (!c->sbuf_bound) {
       c->sbuf_bound = true;
       c->sbuf_stream = s;

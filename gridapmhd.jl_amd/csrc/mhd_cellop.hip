@@ -486,9 +486,19 @@ int launch_op(mhd_ctx *c, const T *x, const T *v, T *y, int64_t rows, double *bu
 
 }  // namespace
 
-int mhd_cellop_build(mhd_ctx *c) {
+// Everything that the products need is allocated with the context: an assembly
+// into it may be the first one and under capture, where nothing can be.
+int mhd_cellop_build(mhd_ctx *c, bool products) {
   MHD_HIP(hipMalloc(&c->d_gslot, sizeof(int32_t) * (size_t)std::max<int64_t>(c->nhold, 1)));
   MHD_HIP(hipMalloc(&c->d_minv, sizeof(double) * (size_t)c->ncells * 16));
+  if (products) {
+    MHD_HIP(hipMalloc(&c->d_state, sizeof(double) * (size_t)c->ncells * 12 * NQ));
+    if (c->nnz >= APPLY_NNZ &&
+        hipMalloc(&c->d_sbuf, sizeof(double) * (size_t)c->ncells * NDOF) != hipSuccess) {
+      c->d_sbuf = nullptr;  // mhd_spmv_d streams the matrix
+      (void)hipGetLastError();
+    }
+  }
   if (c->nhold > 0)
     hipLaunchKernelGGL(k_gslot, dim3((unsigned)((c->nhold + 255) / 256)), dim3(256), 0, c->stream, c->nhold,
                        c->d_centry, c->d_gslot);
@@ -504,7 +514,6 @@ int mhd_cellop_residual(mhd_ctx *c, const double *d_x, double *d_r, double *buf,
 }
 
 int mhd_cellop_state(mhd_ctx *c, const double *d_x, hipStream_t s) {
-  if (!c->d_state) MHD_HIP(hipMalloc(&c->d_state, sizeof(double) * (size_t)c->ncells * 12 * NQ));
   if (c->phys.convection == 0) return 0;
   hipLaunchKernelGGL(k_cell_state, dim3((unsigned)((c->ncells + 1) / 2)), dim3(64), 0, s, c->ncells, c->d_xyz,
                      c->d_dofs, c->d_dir, d_x, c->d_state);

@@ -217,7 +217,7 @@ int mhd_assemble_own(mhd_ctx *c, hipStream_t s);
 // the (u,j) rows' p and phi columns (MHD_OP_PPHI); `trans`: of D^-1 A^T D with
 // D = scale on the j and phi dofs.  No skeleton term.  buf: [ncells][NDOF].
 enum { MHD_OP_FULL = 1, MHD_OP_UJ = 2, MHD_OP_PPHI = 3 };
-int mhd_cellop_build(mhd_ctx *c);
+int mhd_cellop_build(mhd_ctx *c, bool products);
 int mhd_cellop_residual(mhd_ctx *c, const double *d_x, double *d_r, double *buf, int mode, hipStream_t s);
 int mhd_cellop_state(mhd_ctx *c, const double *d_x, hipStream_t s);
 template <class T>
