@@ -1153,8 +1153,19 @@ int mhd_launch_jacobian(mhd_ctx *c, const double *d_x, double *d_val, hipStream_
   return 0;
 }
 
+// Whether s records its work into a graph (an error counts as yes: the stream
+// of a capture elsewhere that cannot be asked).
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 int mhd_assemble_own(mhd_ctx *c, hipStream_t s) {
   c->jac_valid = false;
+  // a replay changes d_val and the state later, with the parameters of now
+  if (c->d_sbuf && capturing(s)) c->jac_replayed = true;
   int rc = mhd_launch_jacobian(c, c->d_x, c->d_val, s);
   if (!rc && c->nskel == 0) rc = mhd_cellop_state(c, c->d_x, s);
   if (rc) return rc;
@@ -1367,8 +1378,13 @@ int mhd_build_tperm(mhd_ctx *c) {
 // That needs a buffer of element results, so it belongs to the first stream
 // that calls; calls on any other stream, which may overlap it, stream the
 // matrix as before, and so does a context whose buffer could not be allocated.
+// The matrix is streamed as well where the host does not know when the product
+// runs or what it is a product with: a captured call (its graph may run beside
+// other calls, and after another assembly), the per-thread stream (one handle
+// for many streams), and every call once an assembly was captured.
 int mhd_launch_spmv(mhd_ctx *c, const double *d_x, double *d_y, hipStream_t s) {
-  if (c->jac_valid && c->d_sbuf && c->own_stream) {  // coarse levels make no products for callers
+  if (c->jac_valid && c->d_sbuf && c->own_stream &&  // coarse levels make no products for callers
+      !c->jac_replayed && s != hipStreamPerThread && !capturing(s)) {
     if (!c->sbuf_bound) {
       c->sbuf_bound = true;
       c->sbuf_stream = s;

@@ -142,6 +142,7 @@ struct mhd_ctx {
   double *d_sbuf = nullptr;           // [ncells][NDOF] element results of mhd_spmv_d
   hipStream_t sbuf_stream = nullptr;  // the one stream whose mhd_spmv_d calls use it
   bool sbuf_bound = false;
+  bool jac_replayed = false;          // an assembly into d_val was captured: replays change it unseen
   int32_t *d_cfptr = nullptr, *d_cface = nullptr;  // thin-wall faces of every cell
   double *d_fK = nullptr;             // [nfaces][4][36] thin-wall face matrices (without orientation signs)
   double *d_fc = nullptr;             // [nfaces][4] their constant parts (-jw)

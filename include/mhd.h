@@ -199,8 +199,9 @@ int mhd_residual_d_noalloc(mhd_ctx *ctx, const double *d_x, double *d_r, void *s
 /* y = A x with the Jacobian last assembled into the context (device pointers),
  * at the parameters and state of that assembly.  From 5 million nonzeros on
  * the first stream that calls gets the product without the matrix (through a
- * buffer of the context); calls on other streams, which may overlap it, and
- * smaller contexts stream the assembled matrix. */
+ * buffer of the context); calls on other streams, which may overlap it,
+ * captured calls, calls after a captured assembly and smaller contexts stream
+ * the assembled matrix. */
 int mhd_spmv_d(mhd_ctx *ctx, const double *d_x, double *d_y, void *stream);
 
 /* Newton + FGMRES + Badia2024 block preconditioner.  Replaces
