@@ -863,15 +863,16 @@ __global__ __launch_bounds__(CND_T) void k_condense(int ncells, const int32_t *_
 // around the vertex, cell by cell in a fixed order.  Two dofs of a patch couple
 // only through cells that hold both, and those are around the vertex, so the
 // entries are taken cell by cell through the rank map, without a search (10 K
-// entries per patch, where scanning the CSR rows visits 32 K columns).  SKEL:
-// the skeleton term couples dofs across cells; the rows are scanned then, each
-// by a wave whose lanes binary-search the columns among the sorted ids.  One
+// entries per patch, where scanning the CSR rows visits 32 K columns).  SCAN:
+// the skeleton term, or an unusual numbering, couples dofs across cells; the
+// rows are scanned then, each by a wave whose lanes binary-search the columns
+// among the sorted ids.  One
 // 1024-thread workgroup per patch.  LDSM: the matrix is built in LDS (129 x 129
 // FP64, 133 of the CU's 160 KB) and written once, coalesced; larger patches are
 // built in place in A.  5.1 ms for 33,800 patches; with the rows scanned and the
 // cells taken one after another, each waiting for its loads, 7.5 ms (the full
 // 225 x 225 matrices, scattered into cleared memory, 18 ms).
-template <bool LDSM, bool SKEL>
+template <bool LDSM, bool SCAN>
 __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__restrict__ psize,
                                                       const int32_t *__restrict__ pidx,
                                                       const int32_t *__restrict__ pcptr,
@@ -912,7 +913,7 @@ __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__r
     }
     return lo < sz && sid[lo] == id ? lo : -1;
   };
-  if (SKEL) {
+  if (SCAN) {
     const int wave = t >> 6, lane = t & 63;
     for (int a = wave; a < sz; a += 16) {
       const int32_t row = sid[a];
@@ -951,7 +952,7 @@ __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__r
   };
   // entries of A, all cells at once (an entry of two cells is written twice,
   // with the same value)
-  if (!SKEL)
+  if (!SCAN)
     for (int qb = q0; qb < q1; qb += CB) {
       locate(qb);
       const int k = t >> 7, mk = m[k];
@@ -968,7 +969,7 @@ __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__r
     }
   // minus A_bi E, cell after cell; the next cell's couplings are loaded meanwhile
   for (int qb = q0; qb < q1; qb += CB) {
-    if (SKEL || q1 - q0 > CB) locate(qb);
+    if (SCAN || q1 - q0 > CB) locate(qb);
     else __syncthreads();  // the entries are in place, the lists still hold
     const int nk = min(CB, q1 - qb);
     constexpr int PF = (NB * NI + 1023) / 1024;
@@ -1872,10 +1873,11 @@ struct Solver {
   int64_t nnz11 = 0, nnz1x = 0;
   double pent = 0.0, pcube = 0.0;
   double ops[MHD_NOPS] = {};
-  // products without the matrix (mhd_cellop_apply); with a skeleton term they
-  // stream it instead, through the row groups below.  Their element results have
-  // a buffer of their own: the context's belongs to mhd_residual_d, which may be
-  // pending on a caller's stream.
+  // products without the matrix (mhd_cellop_apply); with a skeleton term, or
+  // with u or j dofs numbered outside of the [u,j] block, they stream it
+  // instead, through the row groups below.  Their element results have a buffer
+  // of their own: the context's belongs to mhd_residual_d, which may be pending
+  // on a caller's stream.
   bool matfree = true;
   double *d_prod = nullptr;           // [ncells][NDOF]
   // row groups sharing a column list (k_spmv_grp): all rows, and the first
@@ -2005,7 +2007,8 @@ void build_patches(mhd_ctx *c, std::vector<std::vector<int32_t>> &all, std::vect
 }
 
 // Cells whose interior current dofs can be eliminated: 12 consecutive free
-// [u,j] dofs that no other cell and no other place of the cell lists.
+// [u,j] dofs that no other cell and no other place of the cell lists, and no u
+// or j dof of the cell numbered outside of the [u,j] block.
 void build_condensation(const mhd_ctx *c, std::vector<int32_t> &ifirst, std::vector<uint8_t> &elim) {
   const int64_t n1 = (int64_t)c->nfree[0] + c->nfree[2];
   std::vector<uint8_t> held(std::max<int64_t>(n1, 1), 0);  // places listing the dof, 2 = more than one
@@ -2014,9 +2017,10 @@ void build_condensation(const mhd_ctx *c, std::vector<int32_t> &ifirst, std::vec
   ifirst.assign(c->ncells, -1);
   elim.assign(std::max<int64_t>(n1, 1), 0);
   for (int32_t cc = 0; cc < c->ncells; ++cc) {
-    const int32_t *cd = &c->h_dofs[(size_t)cc * NDOF + OFF_J + 24];
+    const int32_t *uj = &c->h_dofs[(size_t)cc * NDOF], *cd = uj + OFF_J + 24;
     bool ok = cd[0] >= 0 && (int64_t)cd[0] + NI <= n1;
     for (int k = 0; k < NI && ok; ++k) ok = cd[k] == cd[0] + k && held[cd[k]] == 1;
+    for (int l = 0; l < NB && ok; ++l) ok = uj[l < NU ? l : l + (OFF_J - NU)] < n1;
     if (!ok) continue;
     ifirst[cc] = cd[0];
     for (int k = 0; k < NI; ++k) elim[cd[k]] = 1;
@@ -2039,6 +2043,7 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
   S->n1 = (int64_t)c->nfree[0] + c->nfree[2];
   S->np = c->nfree[1];
   S->nphi = c->nfree[3];
+  S->matfree = c->nskel == 0;
   // p / phi dofs: consecutive per cell
   std::vector<int32_t> pf(c->ncells), ff(c->ncells);
   for (int32_t cc = 0; cc < c->ncells; ++cc) {
@@ -2055,6 +2060,8 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
         c->err = "phi dofs of a cell must be consecutive and inside the phi block";
         return -1;
       }
+    for (int l = 0; l < NU + NJ; ++l)
+      if (cd[l < NU ? l : l + NP] >= S->n1) S->matfree = false;  // A11 is a block of the matrix, not of the form
   }
   int rc;
   if ((rc = dmalloc(c, &S->d_pfirst, c->ncells))) return rc;
@@ -2071,7 +2078,6 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
     S->nnz11 += k;
     S->nnz1x += (e - b) - k;
   }
-  S->matfree = c->nskel == 0;
   if (!S->matfree) {
     // runs of consecutive rows with one column list (at most GMAX rows; no run
     // crosses the end of the [u,j] rows)
@@ -2664,13 +2670,13 @@ int invert_patches_to(mhd_ctx *c, OutT *inv, float *scale) {
   for (int p0 = 0; p0 < S->npatch; p0 += S->pchunk) {
     const int np = std::min(S->pchunk, S->npatch - p0);
     double *mat = S->d_pscratch;
-    const bool small = S->PS <= GJSmall::NMAX, skel = c->nskel > 0;
+    const bool small = S->PS <= GJSmall::NMAX, scan = !S->matfree;
     auto build = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(np), dim3(1024), 0, c->stream, S->PS, S->d_psize + p0,
                          S->d_pidx + (int64_t)p0 * S->PS, S->d_pcptr + p0, S->d_pcell, c->d_rowptr, c->d_colind,
                          c->d_rank, c->d_val, c->d_dofs, S->d_ifirst, dups, S->d_cE64, S->d_cB64, mat);
     };
-    if (skel) small ? build(k_patch_build<true, true>) : build(k_patch_build<false, true>);
+    if (scan) small ? build(k_patch_build<true, true>) : build(k_patch_build<false, true>);
     else small ? build(k_patch_build<true, false>) : build(k_patch_build<false, false>);
     int16_t *pp = S->d_pperm + (int64_t)p0 * 2 * S->PS;
     int32_t *st = S->d_pstatus + p0;

@@ -1,0 +1,59 @@
+"""Dof and vertex tables that no mesher here makes but the interface takes."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import cases
+
+pytestmark = pytest.mark.gpu
+
+
+def _u_dof_in_the_p_block(sp):
+    """One velocity dof of the first cell numbered as a pressure dof of the last:
+    outside of the [u,j] block, in a cell that does not hold it already."""
+    cd = sp.cell_dofs.copy()
+    k = [l for l in range(27) if cd[0, l] >= 0 and np.count_nonzero(cd == cd[0, l]) > 1][0]
+    cd[0, k] = cd[-1, 82]
+    return dataclasses.replace(sp, cell_dofs=cd)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kind", ["linear", "adjoint"])
+@pytest.mark.parametrize("level", ["fine", "coarse"])
+def test_velocity_dof_outside_of_its_block(level, kind, precision, orc_mod):
+    """The residual that a solve reports is that of the oracle's system (the fine
+    table altered: the preconditioner is a poor one, ten steps); on the coarsest
+    level such a table leaves the solve converging."""
+    import gridapmhd_amd as g
+    from gridapmhd_amd import adjoint, fespaces, multigrid
+    sp, phys = adjoint.inlet_duct((4, 4, 3), 10.0, 5.0, 0.05, convection="picard")
+    rng = np.random.default_rng(5)
+    bc = sp.bc_spec
+    spc = fespaces.setup_fe_spaces(multigrid.coarsen_mesh(sp.mesh), bc["u_tags"], bc["j_tags"], bc["thin_walls"],
+                                   style=sp.style)
+    P, R = multigrid.prolongation(sp, spc)
+    if level == "fine":
+        sp = _u_dof_in_the_p_block(sp)
+    else:
+        spc = _u_dof_in_the_p_block(spc)
+    x, rhs = 0.1 * rng.standard_normal(sp.ndofs), rng.standard_normal(sp.ndofs)
+    A = orc_mod.Oracle(cases.problem_dict(sp, phys)).jacobian(x).tocsr()
+    ctx = g._lib.context_from_spaces(sp, phys)
+    try:
+        ctx.attach_coarse(g._lib.context_from_spaces(spc, phys), P, R, 0, 0.175, "full")
+        o = ctx.default_opts(precision=precision, ls_rtol=1e-10, max_krylov=400 if level == "coarse" else 10, restart=400)
+        s, info, rc = (ctx.linear_solve if kind == "linear" else ctx.adjoint_solve)(x, rhs, o)
+        r = (A if kind == "linear" else A.T.tocsr()) @ s - rhs
+        if kind == "adjoint":  # measured with the j and phi rows over gamma / sigma
+            fs = sp.field_slices()
+            for f in ("j", "phi"):
+                r[fs[f]] /= phys["gamma"] / phys["sigma"]
+        print(f"[tables] u dof in the p block, {level}, {kind}, precision={precision}: rc={rc}, "
+              f"{info.krylov_iters} iterations, residual {np.linalg.norm(r):.6e}, reported {info.residual:.6e}", flush=True)
+        if level == "coarse":
+            assert rc == 0 and np.linalg.norm(r) < 1e-9 * np.linalg.norm(rhs)
+        else:
+            assert abs(np.linalg.norm(r) - info.residual) < 1e-9 * np.linalg.norm(rhs)
+    finally:
+        ctx.close()
