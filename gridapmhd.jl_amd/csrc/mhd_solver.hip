@@ -864,9 +864,9 @@ __global__ __launch_bounds__(CND_T) void k_condense(int ncells, const int32_t *_
 // only through cells that hold both, and those are around the vertex, so the
 // entries are taken cell by cell through the rank map, without a search (10 K
 // entries per patch, where scanning the CSR rows visits 32 K columns).  SCAN:
-// the skeleton term, or an unusual numbering, couples dofs across cells; the
-// rows are scanned then, each by a wave whose lanes binary-search the columns
-// among the sorted ids.  One
+// the skeleton term, or an unusual dof or vertex table, couples dofs of a patch
+// beyond those cells; the rows are scanned then, each by a wave whose lanes
+// binary-search the columns among the sorted ids.  One
 // 1024-thread workgroup per patch.  LDSM: the matrix is built in LDS (129 x 129
 // FP64, 133 of the CU's 160 KB) and written once, coalesced; larger patches are
 // built in place in A.  5.1 ms for 33,800 patches; with the rows scanned and the
@@ -1879,6 +1879,7 @@ struct Solver {
   // of their own: the context's belongs to mhd_residual_d, which may be pending
   // on a caller's stream.
   bool matfree = true;
+  bool scan = false;                  // patch entries from the rows, not cell by cell
   double *d_prod = nullptr;           // [ncells][NDOF]
   // row groups sharing a column list (k_spmv_grp): all rows, and the first
   // ngroups11 groups cover the [u,j] rows exactly
@@ -2006,22 +2007,75 @@ void build_patches(mhd_ctx *c, std::vector<std::vector<int32_t>> &all, std::vect
   }
 }
 
+// The vertices of a cell (bit lv) whose stars hold the local [u,j] dof l.
+uint8_t star_vertices(int l) {
+  uint8_t m = 0;
+  for (int lv = 0; lv < 8; ++lv) {
+    const int at[3] = {lv & 1, (lv >> 1) & 1, lv >> 2};
+    bool in = true;
+    if (l < NU) {
+      const int a = l % 27, x[3] = {a % 3, (a / 3) % 3, a / 9};
+      for (int d = 0; d < 3; ++d) in = in && std::abs(x[d] - 2 * at[d]) <= 1;
+    } else if (l < NB) {
+      const int f = (l - NU) >> 2;
+      in = at[2 - f / 2] == (f & 1);
+    }
+    if (in) m |= (uint8_t)(1 << lv);
+  }
+  return m;
+}
+
 // Cells whose interior current dofs can be eliminated: 12 consecutive free
-// [u,j] dofs that no other cell and no other place of the cell lists, and no u
-// or j dof of the cell numbered outside of the [u,j] block.
-void build_condensation(const mhd_ctx *c, std::vector<int32_t> &ifirst, std::vector<uint8_t> &elim) {
+// [u,j] dofs that no other cell and no other place of the cell lists, no u or j
+// dof of the cell numbered outside of the [u,j] block, and every star that
+// holds a dof of the cell holds the whole cell.  That fails where two cells
+// share dofs of an entity but not its vertices (a periodic direction glued in
+// the dof table only): a dof then lies in more stars (`stars`) than its entity
+// has vertices in the cell.  regular: false if any cell fails the last test.
+void build_condensation(const mhd_ctx *c, const std::vector<std::vector<int32_t>> &stars, std::vector<int32_t> &ifirst,
+                        std::vector<uint8_t> &elim, bool &regular) {
   const int64_t n1 = (int64_t)c->nfree[0] + c->nfree[2];
   std::vector<uint8_t> held(std::max<int64_t>(n1, 1), 0);  // places listing the dof, 2 = more than one
   for (int32_t g : c->h_dofs)
     if (g >= 0 && g < n1) held[g] = (uint8_t)std::min(2, held[g] + 1);
+  std::vector<int32_t> nstars(std::max<int64_t>(n1, 1), 0);
+  for (const auto &L : stars)
+    for (int32_t g : L) ++nstars[g];
+  uint8_t mask[NB];
+  int local[NB], size[NB];
+  for (int l = 0; l < NB; ++l) {
+    local[l] = l < NU ? l : l + (OFF_J - NU);
+    mask[l] = star_vertices(l);
+    size[l] = __builtin_popcount(mask[l]);
+  }
   ifirst.assign(c->ncells, -1);
   elim.assign(std::max<int64_t>(n1, 1), 0);
+  regular = true;
   for (int32_t cc = 0; cc < c->ncells; ++cc) {
-    const int32_t *uj = &c->h_dofs[(size_t)cc * NDOF], *cd = uj + OFF_J + 24;
-    bool ok = cd[0] >= 0 && (int64_t)cd[0] + NI <= n1;
+    const int32_t *uj = &c->h_dofs[(size_t)cc * NDOF], *cd = uj + OFF_J + 24, *v = &c->h_verts[(size_t)cc * 8];
+    bool ok = cd[0] >= 0 && (int64_t)cd[0] + NI <= n1, whole = true;
     for (int k = 0; k < NI && ok; ++k) ok = cd[k] == cd[0] + k && held[cd[k]] == 1;
-    for (int l = 0; l < NB && ok; ++l) ok = uj[l < NU ? l : l + (OFF_J - NU)] < n1;
-    if (!ok) continue;
+    uint8_t first = 0xff;  // local vertices that are not a repetition of an earlier one
+    for (int a = 1; a < 8; ++a)
+      for (int b = 0; b < a; ++b)
+        if (v[a] == v[b]) first &= (uint8_t)~(1 << a);
+    for (int l = 0; l < NB; ++l) {
+      const int32_t g = uj[local[l]];
+      if (g >= n1) ok = false;
+      if (g < 0 || g >= n1) continue;
+      int n = size[l];
+      if (first != 0xff) {
+        n = 0;
+        for (int a = 0; a < 8; ++a) {
+          bool seen = !(mask[l] >> a & 1);
+          for (int b = 0; b < a && !seen; ++b) seen = (mask[l] >> b & 1) && v[a] == v[b];
+          n += !seen;
+        }
+      }
+      whole = whole && nstars[g] == n;
+    }
+    regular = regular && whole;
+    if (!ok || !whole) continue;
     ifirst[cc] = cd[0];
     for (int k = 0; k < NI; ++k) elim[cd[k]] = 1;
   }
@@ -2117,7 +2171,9 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
     std::vector<int32_t> ifirst, npat(c->ncells, 0);
     std::vector<uint8_t> elim;
     build_patches(c, stars, around);
-    build_condensation(c, ifirst, elim);
+    bool regular;
+    build_condensation(c, stars, ifirst, elim, regular);
+    S->scan = !S->matfree || !regular;
     S->npatch = (int)stars.size();
     for (const auto &L : stars) {
       S->PS_all = std::max<int>(S->PS_all, (int)L.size());
@@ -2670,7 +2726,7 @@ int invert_patches_to(mhd_ctx *c, OutT *inv, float *scale) {
   for (int p0 = 0; p0 < S->npatch; p0 += S->pchunk) {
     const int np = std::min(S->pchunk, S->npatch - p0);
     double *mat = S->d_pscratch;
-    const bool small = S->PS <= GJSmall::NMAX, scan = !S->matfree;
+    const bool small = S->PS <= GJSmall::NMAX, scan = S->scan;
     auto build = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(np), dim3(1024), 0, c->stream, S->PS, S->d_psize + p0,
                          S->d_pidx + (int64_t)p0 * S->PS, S->d_pcptr + p0, S->d_pcell, c->d_rowptr, c->d_colind,

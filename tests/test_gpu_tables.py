@@ -57,3 +57,44 @@ def test_velocity_dof_outside_of_its_block(level, kind, precision, orc_mod):
             assert abs(np.linalg.norm(r) - info.residual) < 1e-9 * np.linalg.norm(rhs)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nz", [1, 2, 3])
+def test_smoother_of_a_period_in_the_dof_table_only(nz, precision, orc_mod):
+    """The two ends of a duct identified in the dof table but not in the vertex
+    table: the patches of the end vertices hold dofs of cells that are not
+    around them.  Against the full patches of the oracle's Jacobian."""
+    import gridapmhd_amd as g
+    from devmem import DeviceArray
+    from test_gpu_condensation import _glued
+    from test_gpu_solver import _vertex_patches
+    sp = _glued((3, 2, nz))
+    n = (nz + 1) * 12
+    verts = np.unique(sp.mesh.cell_xyz().reshape(-1, 3).round(9), axis=0, return_inverse=True)[1]
+    sp = dataclasses.replace(sp, cell_verts=verts.reshape(-1, 8).astype(sp.cell_verts.dtype))
+    assert sp.cell_verts.max() + 1 == n
+    phys = cases.cfd_physics(30.0, 10.0, zeta_u=1.0, zeta_j=1.0)
+    rng = np.random.default_rng(9)
+    x = 0.3 * rng.standard_normal(sp.ndofs)
+    n1 = sp.nfree["u"] + sp.nfree["j"]
+    A = orc_mod.Oracle(cases.problem_dict(sp, phys)).jacobian(x).tocsr()[:n1, :n1]
+    r = rng.standard_normal(n1)
+    ref = np.zeros(n1)
+    patches = _vertex_patches(sp)
+    for ids in patches:
+        ref[ids] += np.linalg.solve(A[ids][:, ids].toarray(), r[ids])
+    ctx = g._lib.context_from_spaces(sp, phys)
+    try:
+        ctx.jacobian(x)
+        ctx.precond_setup(ctx.default_opts(precision=precision))
+        dt = np.float64 if precision == 0 else np.float32
+        rr, yy = DeviceArray.from_numpy(r, dt), DeviceArray.from_numpy(np.zeros(n1), dt)
+        ctx.smoother_apply_d(rr.ptr, yy.ptr)
+        err = np.linalg.norm(yy.numpy() - ref) / np.linalg.norm(ref)
+        print(f"[tables] period of {nz} cells in the dof table only, precision={precision}: {len(patches)} patches, "
+              f"rel err {err:.2e}", flush=True)
+        # the bounds of the smoother test on full patches
+        assert err < (1e-12 if precision == 0 else 1e-5)
+    finally:
+        ctx.close()
