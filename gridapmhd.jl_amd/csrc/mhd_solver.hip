@@ -1293,7 +1293,8 @@ __global__ __launch_bounds__(256) void k_cond_inner(int ncells, const int32_t *_
 // flags the patch.  The rows are first scaled by powers of two to a diagonal in
 // [1, 2) (exactly; the columns of the inverse take the scale back), so that the
 // penalty rows of thin-wall faces do not fail the test against rows of another
-// magnitude.  Flagged patches are inverted again by k_patch_gj, with
+// magnitude; a row whose diagonal is too small for that is scaled by its
+// largest entry (gj_row_scale) and fails.  Flagged patches are inverted again by k_patch_gj, with
 // partial pivoting (the unused row of largest |a_ik|, lowest row on ties).
 // Rows are not swapped there: A^-1[k][j] = S[p_k][q_j] with q = p^-1, and the
 // smoother applies it without un-permuting: z = S x' with x'_c = x_{p_c}, and
@@ -1310,7 +1311,7 @@ __device__ inline __half from_dbl<__half>(double v) { return __float2half((float
 template <class G>
 struct GJShared {
   double colbuf[G::NMAX], rowbuf[G::NMAX], Rl[G::NMAX], Cl[G::NL];
-  double rs[G::NMAX];  // powers of two: row r of the matrix times rs[r] has a diagonal in [1, 2)
+  double rs[G::NMAX];  // powers of two: the scale of row r (gj_row_scale)
   int used[G::NMAX];
   int16_t pk[G::NMAX];
   int p, bad;
@@ -1318,26 +1319,62 @@ struct GJShared {
   double wmax[G::T / 64];
 };
 
+// Scale of a row with diagonal |d| and largest |entry| m: d into [1, 2), or, if
+// d is smaller than 2^-8 m, that.  A row scaled by a vanishing diagonal would
+// pass the threshold test with entries of any size and carry them into the
+// others.  (The u rows' Lorentz entries are up to 800 times the diagonal at
+// Ha = 500, where both lines accept the same patches.)
+__device__ inline double gj_row_scale(double d, double m) {
+  const double v = fmax(d, ldexp(m, -8));
+  return v > 0.0 && v < INFINITY ? ldexp(1.0, -max(-1000, min(1000, ilogb(v)))) : 1.0;
+}
+
 template <class G>
 __device__ __forceinline__ void gj_load(double (&S)[G::RI][G::RJ], GJShared<G> &L, const double *__restrict__ Ap, int PS,
                                         int t, int tr, int tc) {
+  double d = 0.0;
   if (t < G::NMAX) {
-    const double d = t < PS ? fabs(Ap[(int64_t)t * PS + t]) : 1.0;
-    L.rs[t] = d > 0.0 && d < INFINITY ? ldexp(1.0, -ilogb(d)) : 1.0;
+    d = t < PS ? fabs(Ap[(int64_t)t * PS + t]) : 1.0;
+    L.rs[t] = 0.0;
+    L.used[t] = 0;
   }
-  __syncthreads();
 #pragma unroll
   for (int i = 0; i < G::RI; ++i)
 #pragma unroll
     for (int j = 0; j < G::RJ; ++j) {
       const int r = tr + G::TR * i, c = tc + G::TC * j;
-      S[i][j] = (r < PS && c < PS) ? Ap[(int64_t)c * PS + r] * L.rs[r] : (r == c ? 1.0 : 0.0);
+      S[i][j] = (r < PS && c < PS) ? Ap[(int64_t)c * PS + r] : (r == c ? 1.0 : 0.0);
     }
-  if (t < G::NMAX) {
-    L.Rl[t] = (t < PS && G::NL < PS) ? Ap[(int64_t)t * PS + G::NL] * L.rs[G::NL] : (t == G::NL ? 1.0 : 0.0);
-    L.used[t] = 0;
+  const double rl = t < PS && G::NL < PS ? Ap[(int64_t)t * PS + G::NL] : (t == G::NL ? 1.0 : 0.0);
+  const double cl = t < PS && t < G::NL && G::NL < PS ? Ap[(int64_t)G::NL * PS + t] : 0.0;
+  __syncthreads();
+  // largest |entry| of every row, as the bits of non-negative doubles, which
+  // order as integers
+  auto row_max = [&](int r, double m) {
+    atomicMax(reinterpret_cast<unsigned long long *>(&L.rs[r]), (unsigned long long)__double_as_longlong(m));
+  };
+#pragma unroll
+  for (int i = 0; i < G::RI; ++i) {
+    double m = 0.0;
+#pragma unroll
+    for (int j = 0; j < G::RJ; ++j) m = fmax(m, fabs(S[i][j]));
+    m = fmax(m, __shfl_xor(m, 16, 64));
+    m = fmax(m, __shfl_xor(m, 32, 64));
+    if ((t & 63) < G::TR) row_max(tr + G::TR * i, m);
   }
-  if (t < G::NL) L.Cl[t] = (t < PS && G::NL < PS) ? Ap[(int64_t)G::NL * PS + t] * L.rs[t] : 0.0;
+  double m = fabs(rl);
+  for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+  if ((t & 63) == 0) row_max(G::NL, m);
+  if (t < G::NL) row_max(t, fabs(cl));
+  __syncthreads();
+  if (t < G::NMAX) L.rs[t] = gj_row_scale(d, L.rs[t]);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < G::RI; ++i)
+#pragma unroll
+    for (int j = 0; j < G::RJ; ++j) S[i][j] *= L.rs[tr + G::TR * i];
+  if (t < G::NMAX) L.Rl[t] = rl * L.rs[G::NL];
+  if (t < G::NL) L.Cl[t] = cl * L.rs[t];
   if (t == 0) L.bad = 0;
 }
 

@@ -269,10 +269,12 @@ int mhd_precond_setup(mhd_ctx *ctx, const mhd_solver_opts *opts);
 int mhd_smoother_apply_d(mhd_ctx *ctx, const void *d_r, void *d_y, void *stream);
 /* The vertex-patch inversions of mhd_precond_setup (batched Gauss-Jordan on
  * the patch matrices with the cells' interior current dofs eliminated and the
- * rows scaled by powers of two to a diagonal in [1, 2)) pivot on the diagonal
- * while |a_kk| >= tau max_{i>k} |a_ik| and invert a patch whose diagonal pivot
- * fails that test again with partial pivoting (the largest |a_ik|).  tau in [0, 1]: 1 = every patch with partial pivoting,
- * 0 = diagonal pivots unless one is zero.  Default 0.03; applies to the
+ * rows scaled by powers of two to a diagonal in [1, 2), or to a largest entry
+ * in [256, 512) where the diagonal is less than 1 / 256 of it) pivot on the
+ * diagonal while |a_kk| >= tau max_{i>k} |a_ik| and invert a patch whose diagonal
+ * pivot fails that test again with partial pivoting (the largest |a_ik|).  tau
+ * in [0, 1]: 1 = every patch with partial pivoting, 0 = diagonal pivots unless
+ * one is zero.  Default 0.03; applies to the
  * attached coarse levels too.  No counterpart in the reference (its patch
  * solves are library LU factorisations). */
 int mhd_set_pivot_threshold(mhd_ctx *ctx, double tau);
