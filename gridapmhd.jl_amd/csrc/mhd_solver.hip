@@ -1917,6 +1917,7 @@ struct Solver {
   // on a caller's stream.
   bool matfree = true;
   bool scan = false;                  // patch entries from the rows, not cell by cell
+  bool unheld = false;                // some [u,j] dof is in no cell
   double *d_prod = nullptr;           // [ncells][NDOF]
   // row groups sharing a column list (k_spmv_grp): all rows, and the first
   // ngroups11 groups cover the [u,j] rows exactly
@@ -2211,6 +2212,10 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
     bool regular;
     build_condensation(c, stars, ifirst, elim, regular);
     S->scan = !S->matfree || !regular;
+    std::vector<uint8_t> in_cell(std::max<int64_t>(S->n1, 1), 0);
+    for (int32_t g : c->h_dofs)
+      if (g >= 0 && g < S->n1) in_cell[g] = 1;
+    S->unheld = std::count(in_cell.begin(), in_cell.begin() + S->n1, (uint8_t)0) > 0;
     S->npatch = (int)stars.size();
     for (const auto &L : stars) {
       S->PS_all = std::max<int>(S->PS_all, (int)L.size());
@@ -2462,6 +2467,8 @@ int patch_as_on(mhd_ctx *c, const T *r, T *y, int prec, double w, bool accumulat
     G = S->d_cG32;
   }
   if (S->npatch == 0) return 0;
+  if (S->unheld && !accumulate)  // k_cond_gather goes through the cells
+    hipLaunchKernelGGL((k_fill<T>), dim3(nblocks(S->n1)), dim3(TB), 0, st, S->n1, (T)0, y);
   hipLaunchKernelGGL((k_cond_rhs<T, TE>), dim3((unsigned)((4 * S->n1 + 255) / 256)), dim3(256), 0, st, S->n1,
                      c->d_crow, c->d_centry, S->d_elim, S->d_ifirst, F, r, S->d_rt, (const int32_t *)nullptr);
   if (prec == 0) patch_products(S, S->d_pA, (const float *)nullptr, st);

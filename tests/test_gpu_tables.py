@@ -98,3 +98,34 @@ def test_smoother_of_a_period_in_the_dof_table_only(nz, precision, orc_mod):
         assert err < (1e-12 if precision == 0 else 1e-5)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_dofs_in_no_cell_stay_zero(precision):
+    """Three current dofs that no cell lists (empty rows): a solve leaves them zero
+    and the others as they are without them."""
+    import gridapmhd_amd as g
+    from devmem import DeviceArray
+    from gridapmhd_amd import adjoint
+    sp, phys = adjoint.inlet_duct((3, 3, 2), 10.0, 5.0, 0.05, convection="picard")
+    n1, extra = sp.nfree["u"] + sp.nfree["j"], 3
+    more = dataclasses.replace(sp, cell_dofs=np.where(sp.cell_dofs >= n1, sp.cell_dofs + extra, sp.cell_dofs).astype(np.int32),
+                               nfree=dict(sp.nfree, j=sp.nfree["j"] + extra))
+    rng = np.random.default_rng(5)
+    x, rhs = 0.1 * rng.standard_normal(sp.ndofs), rng.standard_normal(sp.ndofs)
+    pad = lambda v: np.concatenate([v[:n1], np.zeros(extra), v[n1:]])
+    sol = []
+    for s, a, b in ((sp, x, rhs), (more, pad(x), pad(rhs))):
+        for _ in range(8):                                     # freed memory that holds other values than zero
+            DeviceArray.from_numpy(np.full(1 << 20, 1e30))
+        ctx = g._lib.context_from_spaces(s, phys)
+        try:
+            out, info, rc = ctx.linear_solve(a, b, ctx.default_opts(precision=precision, ls_rtol=1e-10, max_krylov=400,
+                                                                    restart=400))
+            assert rc == 0
+            sol.append(out)
+        finally:
+            ctx.close()
+    err = np.linalg.norm(np.delete(sol[1], range(n1, n1 + extra)) - sol[0]) / np.linalg.norm(sol[0])
+    print(f"[tables] dofs in no cell, precision={precision}: {sol[1][n1:n1 + extra]}, others {err:.2e}", flush=True)
+    assert np.all(sol[1][n1:n1 + extra] == 0.0) and err < 1e-7  # 1e-10 times the condition number's part
