@@ -181,6 +181,7 @@ struct CoarseLink {
   // coarsest level solved exactly: explicit inverse (row-major) of its [u,j]
   // block with the cells' interior current dofs condensed out
   int64_t nb = 0;                  // dofs that are not eliminated
+  bool condensed = true;           // whether the arrays are those of a level that eliminates dofs
   int32_t *d_bidx = nullptr, *d_bmap = nullptr;  // [nb] their ids, [n1c] the inverse (-1)
   int32_t *d_ones = nullptr;       // [ncells of the level]
   double *d_cF = nullptr, *d_cG = nullptr;       // A_bi D^-1, D^-1 of every cell

@@ -1918,6 +1918,7 @@ struct Solver {
   bool matfree = true;
   bool scan = false;                  // patch entries from the rows, not cell by cell
   bool unheld = false;                // some [u,j] dof is in no cell
+  bool condense = true;               // cells' interior current dofs eliminated where they can be
   double *d_prod = nullptr;           // [ncells][NDOF]
   // row groups sharing a column list (k_spmv_grp): all rows, and the first
   // ngroups11 groups cover the [u,j] rows exactly
@@ -2071,7 +2072,7 @@ uint8_t star_vertices(int l) {
 // the dof table only): a dof then lies in more stars (`stars`) than its entity
 // has vertices in the cell.  regular: false if any cell fails the last test.
 void build_condensation(const mhd_ctx *c, const std::vector<std::vector<int32_t>> &stars, std::vector<int32_t> &ifirst,
-                        std::vector<uint8_t> &elim, bool &regular) {
+                        std::vector<uint8_t> &elim, bool &regular, bool condense) {
   const int64_t n1 = (int64_t)c->nfree[0] + c->nfree[2];
   std::vector<uint8_t> held(std::max<int64_t>(n1, 1), 0);  // places listing the dof, 2 = more than one
   for (int32_t g : c->h_dofs)
@@ -2113,14 +2114,21 @@ void build_condensation(const mhd_ctx *c, const std::vector<std::vector<int32_t>
       whole = whole && nstars[g] == n;
     }
     regular = regular && whole;
-    if (!ok || !whole) continue;
+    if (!condense || !ok || !whole) continue;
     ifirst[cc] = cd[0];
     for (int k = 0; k < NI; ++k) elim[cd[k]] = 1;
   }
 }
 
-int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
-  if (c->solver) return 0;
+// The interior block of a cell is the RT1 mass plus zeta_j div-div: for a
+// negative zeta_j it may be singular where no patch is, so nothing is eliminated.
+bool may_condense(const mhd_ctx *c) {
+  return !(c->phys.zeta_j < 0.0 || (c->jac_valid && c->jac_phys.zeta_j < 0.0));
+}
+
+int solver_init(mhd_ctx *c, const mhd_solver_opts *o, bool condense) {
+  if (c->solver && c->solver->condense == condense) return 0;
+  if (c->solver) mhd_solver_free(c);
   if (c->block_style != 1) {
     c->err = "mhd_newton_solve needs the Badia2024 block numbering (spaces.block_style = 1)";
     return -1;
@@ -2131,6 +2139,7 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
   }
   Solver *S = new Solver();
   c->solver = S;
+  S->condense = condense;
   S->n = c->n;
   S->n1 = (int64_t)c->nfree[0] + c->nfree[2];
   S->np = c->nfree[1];
@@ -2210,7 +2219,7 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
     std::vector<uint8_t> elim;
     build_patches(c, stars, around);
     bool regular;
-    build_condensation(c, stars, ifirst, elim, regular);
+    build_condensation(c, stars, ifirst, elim, regular, S->condense);
     S->scan = !S->matfree || !regular;
     std::vector<uint8_t> in_cell(std::max<int64_t>(S->n1, 1), 0);
     for (int32_t g : c->h_dofs)
@@ -2303,7 +2312,7 @@ int solver_init(mhd_ctx *c, const mhd_solver_opts *o) {
     oc.restart = 2;  // coarse levels only run the inner solve
     oc.inner_iters = cc->coarse ? 0 : c->coarse->coarse_iters;
     if (cc->solver && (cc->solver->kin != std::max(0, std::min(oc.inner_iters, 120)))) mhd_solver_free(cc);
-    if ((rc = solver_init(cc, &oc))) {
+    if ((rc = solver_init(cc, &oc, condense))) {
       c->err = "coarse level: " + cc->err;
       return rc;
     }
@@ -2716,8 +2725,6 @@ int precond(mhd_ctx *c, const double *v, double *z, int prec) {
   return 0;
 }
 
-int solver_init(mhd_ctx *c, const mhd_solver_opts *o);
-
 int coarse_alloc(mhd_ctx *c, int prec) {
   CoarseLink *L = c->coarse;
   const int tp = prec == 0 ? 0 : 1;
@@ -2839,6 +2846,16 @@ int invert_patches(mhd_ctx *c, int prec) {
   return 0;
 }
 
+// the arrays of the exact coarsest solve
+void dense_free(CoarseLink *L) {
+  auto drop = [](auto *&p) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+  };
+  drop(L->d_bidx), drop(L->d_bmap), drop(L->d_ones), drop(L->d_piv), drop(L->d_info), drop(L->d_gjflag);
+  drop(L->d_cF), drop(L->d_cG), drop(L->d_rb), drop(L->d_yb), drop(L->d_Ainv), drop(L->d_LU), drop(L->d_gjw);
+}
+
 // Per-Jacobian set-up of one level: Schur scalings, FP32 copy and patch
 // factorisation, then the coarser levels: the u state is injected from
 // `d_state` and the [u,j] block re-assembled with the same kernels
@@ -2904,7 +2921,9 @@ int precond_setup(mhd_ctx *c, int prec, const double *d_state) {
     // block S is the column-major S^T; block Gauss-Jordan inverts it in place
     // into (S^T)^-1, whose column-major storage is S^-1 row-major.
     Solver *SC = cc->solver;
-    if (!L->d_Ainv) {
+    if (!L->d_Ainv || L->condensed != SC->condense) {
+      dense_free(L);
+      L->condensed = SC->condense;
       std::vector<int32_t> bidx, bmap(L->n1c, -1), ones(cc->ncells, 1);
       std::vector<uint8_t> elim(L->n1c);
       MHD_HIP(hipMemcpy(elim.data(), SC->d_elim, (size_t)L->n1c, hipMemcpyDeviceToHost));
@@ -3110,10 +3129,10 @@ void mhd_coarse_free(mhd_ctx *c) {
   if (!c || !c->coarse) return;
   CoarseLink *L = c->coarse;
   void *ptrs[] = {L->d_Prow, L->d_Trow, L->d_Pcol, L->d_Tcol, L->d_Pval, L->d_Tval, L->d_Pval32, L->d_Tval32,
-                  L->d_Rrow, L->d_Rcol, L->d_Rval, L->rr, L->rc, L->ec, L->d_Ainv, L->d_LU, L->d_piv, L->d_info, L->d_ab,
-                  L->d_gjw, L->d_gjflag, L->d_bidx, L->d_bmap, L->d_ones, L->d_cF, L->d_cG, L->d_rb, L->d_yb};
+                  L->d_Rrow, L->d_Rcol, L->d_Rval, L->rr, L->rc, L->ec, L->d_ab};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
+  dense_free(L);
   if (L->ctx) mhd_destroy(L->ctx);
   delete L;
   c->coarse = nullptr;
@@ -3258,7 +3277,7 @@ int mhd_precond_setup(mhd_ctx *c, const mhd_solver_opts *o) {
   if (c->solver && (c->solver->m != krylov_dim(o->restart) ||
                     c->solver->kin != std::max(0, std::min(o->inner_iters, 120))))
     mhd_solver_free(c);
-  if ((rc = solver_init(c, o))) return rc;
+  if ((rc = solver_init(c, o, may_condense(c)))) return rc;
   if ((rc = precond_setup(c, o->precision, c->d_x))) return rc;
   MHD_HIP(hipStreamSynchronize(c->stream));
   return 0;
@@ -3338,7 +3357,7 @@ int linear_solve(mhd_ctx *c, const double *x_state, const double *rhs, double *l
   // every level of an attached V-cycle hierarchy works on its transposed
   // Jacobian for the duration (the transfers P, P^T are unchanged)
   if (c->solver) mhd_solver_free(c);
-  rc = solver_init(c, o);
+  rc = solver_init(c, o, may_condense(c));
   if (rc) return rc;
   Solver *S = c->solver;
   const int64_t n = c->n;
@@ -3424,11 +3443,11 @@ int mhd_newton_solve(mhd_ctx *c, double *x_host, const mhd_solver_opts *o, mhd_s
   MHD_HIP(hipSetDevice(c->device));
   int rc;
   double t0 = now();
-  if ((rc = solver_init(c, o))) return rc;
+  if ((rc = solver_init(c, o, may_condense(c)))) return rc;
   Solver *S = c->solver;
   if (S->m != krylov_dim(o->restart) || S->kin != std::max(0, std::min(o->inner_iters, 120))) {
     mhd_solver_free(c);
-    if ((rc = solver_init(c, o))) return rc;
+    if ((rc = solver_init(c, o, may_condense(c)))) return rc;
     S = c->solver;
   }
   info->t_setup += now() - t0;
