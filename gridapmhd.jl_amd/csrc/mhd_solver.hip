@@ -2126,9 +2126,19 @@ bool may_condense(const mhd_ctx *c) {
   return !(c->phys.zeta_j < 0.0 || (c->jac_valid && c->jac_phys.zeta_j < 0.0));
 }
 
+int solver_build(mhd_ctx *c, const mhd_solver_opts *o, bool condense);
+
+// The solver of a context, built if it has none for this choice.  A solver that
+// was refused half-way is not kept: the next call would take it for whole.
 int solver_init(mhd_ctx *c, const mhd_solver_opts *o, bool condense) {
   if (c->solver && c->solver->condense == condense) return 0;
   if (c->solver) mhd_solver_free(c);
+  const int rc = solver_build(c, o, condense);
+  if (rc) mhd_solver_free(c);
+  return rc;
+}
+
+int solver_build(mhd_ctx *c, const mhd_solver_opts *o, bool condense) {
   if (c->block_style != 1) {
     c->err = "mhd_newton_solve needs the Badia2024 block numbering (spaces.block_style = 1)";
     return -1;

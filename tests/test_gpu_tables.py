@@ -129,3 +129,24 @@ def test_dofs_in_no_cell_stay_zero(precision):
     err = np.linalg.norm(np.delete(sol[1], range(n1, n1 + extra)) - sol[0]) / np.linalg.norm(sol[0])
     print(f"[tables] dofs in no cell, precision={precision}: {sol[1][n1:n1 + extra]}, others {err:.2e}", flush=True)
     assert np.all(sol[1][n1:n1 + extra] == 0.0) and err < 1e-7  # 1e-10 times the condition number's part
+
+
+def test_a_refused_table_is_refused_again():
+    """A solver that was refused half-way leaves nothing that a second call takes
+    for a solver."""
+    import gridapmhd_amd as g
+    from gridapmhd_amd import adjoint
+    sp, phys = adjoint.inlet_duct((2, 2, 2), 10.0, 5.0, 0.05)
+    cd = sp.cell_dofs.copy()
+    cd[0, 82], cd[0, 83] = cd[0, 83], cd[0, 82]                # pressure dofs out of order
+    ctx = g._lib.context_from_spaces(dataclasses.replace(sp, cell_dofs=cd), phys)
+    try:
+        x = np.zeros(sp.ndofs)
+        o = ctx.default_opts()
+        ctx.jacobian(x)
+        for call in (lambda: ctx.precond_setup(o), lambda: ctx.precond_setup(o), lambda: ctx.newton_solve(x, o),
+                     lambda: ctx.linear_solve(x, x, o)):
+            with pytest.raises(g._lib.MhdError, match="p dofs of a cell must be consecutive"):
+                call()
+    finally:
+        ctx.close()
