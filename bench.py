@@ -96,12 +96,13 @@ def time_events(fn, reps, stream):
     return s.elapsed_time(e) / 1e3 / reps
 
 
-def cpu_baseline(sp, phys, ctx, counts, residuals_per_step, log):
+def cpu_baseline(sp, phys, ctx, coarsest, counts, residuals_per_step, log):
     """CPU price of one FP64 Newton step of the same duct on the host cores:
     the oracle's element kernels (assembly into the duct's own CSC pattern by
     binary search) and the solver's sparse, patch, dense and vector kernels,
     each timed on a bounded sample at the real sizes, times the per-step
-    operation counts of the FP64 GPU solve."""
+    operation counts of the FP64 GPU solve (`coarsest`: the spaces of the level
+    that is solved with a dense inverse, or None)."""
     sys.path.insert(0, os.path.join(ROOT, "tests"))
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
     import cases
@@ -116,6 +117,8 @@ def cpu_baseline(sp, phys, ctx, counts, residuals_per_step, log):
     n1 = sp.nfree["u"] + sp.nfree["j"]
     rt = cb.rates(orc, colptr, rowval, n1, sp.ndofs, log=log)
     del colptr, rowval
+    if coarsest is not None:
+        counts = cb.executed_dense(counts, coarsest.nfree["u"] + coarsest.nfree["j"], coarsest.ncells)
     t, parts = cb.compose(rt, counts, orc.ncells, residuals_per_step)
     host = cb.host_info()
     samp = rt["cells_sampled"]
@@ -478,7 +481,9 @@ def main():
     cpu = None
     if not args.no_cpu:
         log("CPU baseline (oracle element kernels + CPU solver kernels) ...")
-        cpu = cpu_baseline(sp, phys, ctx, results["fp64"]["op_counts_per_step"],
+        dense = levels > 1 and args.coarse_iters == 0
+        coarsest = sp._multigrid_cache[(0, 1)]["chain"][levels - 1] if dense else None
+        cpu = cpu_baseline(sp, phys, ctx, coarsest, results["fp64"]["op_counts_per_step"],
                            results["fp64"]["residuals_per_step"], log)
         log(f"cpu: {cpu}")
 

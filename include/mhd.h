@@ -299,9 +299,10 @@ int mhd_smoother_info(mhd_ctx *ctx, int64_t *npatch, int64_t *patch_dim, int64_t
  *      linear combinations, minimal-residual coarse steps)
  *   7  cells of the coarse-level Jacobian assemblies (preconditioner set-up)
  *   8  sum of dim^3 over the inverted patches (set-up)
- *   9  sum of n^3 over the dense coarsest inversions (n: the level's [u,j] dofs,
- *      of which the cells' interior current dofs are eliminated; an inverse whose
- *      block Gauss-Jordan check fails and is redone by the pivoted LU counts twice)
+ *   9  sum of n^3 over the dense coarsest inversions, n all [u,j] dofs of the
+ *      level (the block that is inverted has the cells' interior current dofs
+ *      eliminated, 12 per cell: the executed size is below n); an inverse whose
+ *      block Gauss-Jordan check fails and is redone by the pivoted LU counts twice
  *   10 outer FGMRES iterations
  * reset != 0 zeroes the counts after reading them. */
 #define MHD_NOPS 11

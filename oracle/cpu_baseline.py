@@ -197,6 +197,13 @@ def rates(orc, colptr, rowval, n1, nfree, log=print, cell_budget_s=6.0, patch_di
     return out
 
 
+def executed_dense(counts, n1, ncells):
+    """`counts` with the dense coarsest inversions at the size they are executed
+    at: mhd_op_counts counts them by the level's n1 [u,j] dofs, of which the 12
+    interior current dofs of each of its `ncells` cells are eliminated first."""
+    return dict(counts, setup_dense_dim3=counts["setup_dense_dim3"] * ((n1 - 12 * ncells) / n1) ** 3)
+
+
 def compose(rt, counts, ncells, residuals_per_step):
     """Seconds of one FP64 Newton step on the CPU: the measured per-operation
     times of ``rates`` times the per-step operation counts of the GPU solve."""
