@@ -463,29 +463,26 @@ struct FaceLDS {
   double W[NQF];
   double ndn[NQF];           // +-1 / (det J |J^-T n^|): s.n = sgn * rt_d * ndn
   double n[NQF][3];
-  double psi[NQF][36][3];
   double gpsi[NQF][36][9];   // [i][k] = d psi_k / d x_i
-  double jn[NQF], jnn[NQF];
+  double jnn[NQF];           // n.(grad j).n of the state
   double xl[NJ];
   double xyz[24];
   int32_t g[NJ];
-  int64_t rp[NJ];
 };
 
+// geometry of a face and, with a state x, the current on it
 __device__ void stage_face(FaceLDS &S, int f, const double *__restrict__ xyz, const int32_t *__restrict__ dofs,
                            const int8_t *__restrict__ sign, const double *__restrict__ dir,
                            const double *__restrict__ x, const FaceTables *__restrict__ F,
-                           const int32_t *__restrict__ fcell, const int8_t *__restrict__ flf,
-                           const int64_t *__restrict__ rowptr, int &cell, int &lf) {
+                           const int32_t *__restrict__ fcell, const int8_t *__restrict__ flf, int &cell, int &lf) {
   const int tid = threadIdx.x, nt = blockDim.x;
   cell = fcell[f];
   lf = flf[f];
   if (tid < 24) S.xyz[tid] = xyz[(int64_t)cell * 24 + tid];
-  if (tid < NJ) {
+  if (x && tid < NJ) {
     const int32_t g = dofs[(int64_t)cell * NDOF + OFF_J + tid];
     S.g[tid] = g;
-    S.xl[tid] = g >= 0 ? x[g] : dir[-g - 1];
-    S.rp[tid] = (g >= 0 && rowptr) ? rowptr[g] : -1;
+    S.xl[tid] = g >= 0 ? x[g] : dir[-(int64_t)g - 1];
   }
   __syncthreads();
   __shared__ double Jq[NQF][9], Jiq[NQF][9], detq[NQF];
@@ -534,8 +531,6 @@ __device__ void stage_face(FaceLDS &S, int f, const double *__restrict__ xyz, co
     const double sgn = r < 24 ? (sign ? (double)sign[(int64_t)cell * 6 + (r >> 2)] : 1.0) : 1.0;
     const double id = sgn / detq[q];
     const double *J = Jq[q], *Ji = Jiq[q];
-    const double *rt = F->rt[lf][q][r];
-    for (int k = 0; k < 3; ++k) S.psi[q][r][k] = id * (J[3 * k + 0] * rt[0] + J[3 * k + 1] * rt[1] + J[3 * k + 2] * rt[2]);
     // grad psi [i][k] = id * sum_l J[k][l] sum_m drt[l][m] Ji[m][i]  (affine push-forward)
     for (int i = 0; i < 3; ++i)
       for (int k = 0; k < 3; ++k) {
@@ -549,22 +544,16 @@ __device__ void stage_face(FaceLDS &S, int f, const double *__restrict__ xyz, co
       }
   }
   __syncthreads();
-  if (tid < NQF) {
+  if (x && tid < NQF) {
     const int q = tid;
     const double *n = S.n[q];
-    const int d = 2 - lf / 2;
-    double jn = 0.0, jnn = 0.0;
-    for (int r = 4 * lf; r < 4 * lf + 4; ++r) {
-      const double sgn = sign ? (double)sign[(int64_t)cell * 6 + lf] : 1.0;
-      jn += S.xl[r] * sgn * F->rt[lf][q][r][d] * S.ndn[q];
-    }
+    double jnn = 0.0;
     for (int r = 0; r < 36; ++r) {
       const double *gs = S.gpsi[q][r];
       double t = 0.0;
       for (int i = 0; i < 3; ++i) t += n[i] * (gs[3 * i + 0] * n[0] + gs[3 * i + 1] * n[1] + gs[3 * i + 2] * n[2]);
       jnn += S.xl[r] * t;
     }
-    S.jn[q] = jn;
     S.jnn[q] = jnn;
   }
   __syncthreads();
@@ -580,7 +569,7 @@ __global__ __launch_bounds__(64) void k_face_dcw(int nfaces, const double *__res
   __shared__ FaceLDS S;
   for (int f = blockIdx.x; f < nfaces; f += gridDim.x) {
     int cell, lf;
-    stage_face(S, f, xyz, dofs, sign, dir, x, F, fcell, flf, nullptr, cell, lf);
+    stage_face(S, f, xyz, dofs, sign, dir, x, F, fcell, flf, cell, lf);
     const int a = 4 * lf + threadIdx.x;
     if (threadIdx.x < 4 && S.g[a] >= 0) {
       const double tau = ftau[f];
@@ -600,8 +589,7 @@ __global__ __launch_bounds__(64) void k_face_dcw(int nfaces, const double *__res
 // linear and depends on the geometry and the face's parameters only, so they
 // are computed once per context (1.2 KB per face).
 __global__ __launch_bounds__(64) void k_face_matrix(int nfaces, const double *__restrict__ xyz,
-                                                    const int32_t *__restrict__ dofs, const double *__restrict__ dir,
-                                                    const double *__restrict__ x, const FaceTables *__restrict__ F,
+                                                    const FaceTables *__restrict__ F,
                                                     const int32_t *__restrict__ fcell, const int8_t *__restrict__ flf,
                                                     const double *__restrict__ ftau, const double *__restrict__ fcw,
                                                     const double *__restrict__ fjw, double *__restrict__ K,
@@ -609,7 +597,7 @@ __global__ __launch_bounds__(64) void k_face_matrix(int nfaces, const double *__
   __shared__ FaceLDS S;
   for (int f = blockIdx.x; f < nfaces; f += gridDim.x) {
     int cell, lf;
-    stage_face(S, f, xyz, dofs, nullptr, dir, x, F, fcell, flf, nullptr, cell, lf);
+    stage_face(S, f, xyz, nullptr, nullptr, nullptr, nullptr, F, fcell, flf, cell, lf);
     const double tau = ftau[f], cw = fcw[f], jw = fjw[f];
     const int dax = 2 - lf / 2;
     for (int idx = threadIdx.x; idx < 4 * NJ; idx += blockDim.x) {
@@ -1229,11 +1217,8 @@ int mhd_build_face_matrices(mhd_ctx *c) {
   MHD_HIP(hipMalloc(&c->d_fK, sizeof(double) * nf * 4 * NJ));
   MHD_HIP(hipMalloc(&c->d_fc, sizeof(double) * nf * 4));
   if (c->nfaces <= 0) return 0;
-  // the state that the staging reads plays no part in the matrices
-  MHD_HIP(hipMemsetAsync(c->d_x, 0, sizeof(double) * std::max<int64_t>(c->n, 1), c->stream));
   hipLaunchKernelGGL(k_face_matrix, dim3((unsigned)std::min(c->nfaces, 1 << 20)), dim3(64), 0, c->stream, c->nfaces,
-                     c->d_xyz, c->d_dofs, c->d_dir, c->d_x, c->d_fref, c->d_fcell, c->d_flf, c->d_ftau, c->d_fcw,
-                     c->d_fjw, c->d_fK, c->d_fc);
+                     c->d_xyz, c->d_fref, c->d_fcell, c->d_flf, c->d_ftau, c->d_fcw, c->d_fjw, c->d_fK, c->d_fc);
   MHD_HIP(hipGetLastError());
   return 0;
 }

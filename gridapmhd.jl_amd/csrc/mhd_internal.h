@@ -48,9 +48,6 @@ struct FaceTables {
   double dq2[6][NQF][27][3];     // Q2 reference gradients (skeleton stabilisation)
 };
 
-// Skeleton stabilisation: the velocity nodes of a face are the 27 of its first
-// cell (slots 0..26) and those of the second cell not shared with the first
-// (slot 27 + local node); SKEL_NONE marks the unused slots.
 // mhd_spmv_d applies the form cell by cell from this many nonzeros on; smaller
 // matrices are streamed.  Two launches of a cell's serial chain against one
 // pass over the values: 192 cells and 1.6M nonzeros 13.2 against 7.4 us, 480 and
@@ -59,6 +56,9 @@ struct FaceTables {
 // have no such line: their grouped streams take 21 us on 48 cells, applied 14.)
 constexpr int64_t APPLY_NNZ = 5000000;
 
+// Skeleton stabilisation: the velocity nodes of a face are the 27 of its first
+// cell (slots 0..26) and those of the second cell not shared with the first
+// (slot 27 + local node); SKEL_NONE marks the unused slots.
 constexpr int SKEL_SLOTS = 54;
 constexpr int SKEL_MAX_ROW = 8192;  // longest CSR row of a stabilised Jacobian (64 KiB of LDS)
 constexpr int SKEL_DOFS = 3 * SKEL_SLOTS;   // [component][slot]

@@ -33,7 +33,7 @@
 #include <cstring>
 #include <type_traits>
 
-#include "mhd_internal.h"
+#include "mhd_cell.h"
 
 using namespace mhd;
 
@@ -149,29 +149,21 @@ __device__ inline double csr_row_dot(int64_t p0, int64_t e, const int32_t *__res
   return (a0 + a1) + (a2 + a3);
 }
 
-// MODE 0: full rows.  MODE 1: A11 prefix [rowptr, split).  MODE 2: y = v - suffix [split, rowptr+1) . x
-// MODE 3: y = v - prefix . x
-template <class MV, class TX, class TY, int LPR, int MODE>
-__global__ __launch_bounds__(256) void k_spmv_seg(int64_t nrows, const int64_t *__restrict__ rowptr,
-                                                  const int64_t *__restrict__ split, const int32_t *__restrict__ colind,
-                                                  const MV *__restrict__ val, const TX *__restrict__ x,
-                                                  const TY *__restrict__ v, TY *__restrict__ y) {
+// y = v - (the columns from split on) . x: the p and phi columns of the [u,j] rows
+template <int LPR>
+__global__ __launch_bounds__(256) void k_spmv_suffix(int64_t nrows, const int64_t *__restrict__ rowptr,
+                                                     const int64_t *__restrict__ split,
+                                                     const int32_t *__restrict__ colind,
+                                                     const double *__restrict__ val, const double *__restrict__ x,
+                                                     const double *__restrict__ v, double *__restrict__ y) {
   const int64_t gid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const int64_t row = gid / LPR;
   const int lane = threadIdx.x % LPR;
   double acc = 0.0;
-  if (row < nrows) {
-    int64_t b = rowptr[row], e = rowptr[row + 1];
-    if (MODE == 1 || MODE == 3) e = split[row];
-    if (MODE == 2) b = split[row];
-    acc = csr_row_dot<LPR>(b + lane, e, colind, val, x);
-  }
+  if (row < nrows) acc = csr_row_dot<LPR>(split[row] + lane, rowptr[row + 1], colind, val, x);
 #pragma unroll
   for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_down(acc, off, LPR);
-  if (row < nrows && lane == 0) {
-    if (MODE == 2 || MODE == 3) y[row] = (TY)((double)v[row] - acc);
-    else y[row] = (TY)acc;
-  }
+  if (row < nrows && lane == 0) y[row] = v[row] - acc;
 }
 
 // Rows that share one column list (the 3 components of a velocity node, the 4
@@ -307,13 +299,6 @@ constexpr int BGJ_B = 96;
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
 
-// Orders the LDS accesses of one wave's lanes (no other wave is involved).
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ inline double read_lane(double v, int lane) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
   const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
@@ -365,13 +350,13 @@ __device__ inline void wave_inverse(double *A, int lda, double *prow, int *pk, i
     mask |= 1u << p;
     if (lane == 0) pk[k] = p;
     if (h == hk) a[kk] = 0.0;
-    wave_sync();
+    wave_order();
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const double pr = prow[16 * h + j];
       a[j] = r == p ? pr : fma(-f, pr, a[j]);
     }
-    wave_sync();
+    wave_order();
   }
   // A^-1[k][pk[c]] = S[pk[k]][c]
 #pragma unroll
@@ -2716,7 +2701,7 @@ int precond(mhd_ctx *c, const double *v, double *z, int prec) {
                                        c->stream))) return rc;
   } else {
     constexpr int LPR = 16;
-    hipLaunchKernelGGL((k_spmv_seg<double, double, double, LPR, 2>), dim3((unsigned)((S->n1 * LPR + 255) / 256)),
+    hipLaunchKernelGGL((k_spmv_suffix<LPR>), dim3((unsigned)((S->n1 * LPR + 255) / 256)),
                        dim3(256), 0, c->stream, S->n1, c->d_rowptr, S->d_split, c->d_colind, c->d_val, z, v, rhs1);
     MHD_HIP(hipGetLastError());
   }
