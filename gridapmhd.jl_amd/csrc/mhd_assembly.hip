@@ -132,7 +132,7 @@ __device__ inline void store_tile(const JacCell &S, const d4_t &acc, double scal
 // Jacobian of one cell per workgroup and turn, on FP64 MFMA tiles (16x16x4) in
 // reference space: every factor that is the same for all cells (reference
 // values and gradients) sits in LDS tables loaded once per workgroup, and a
-// cell brings 57 weights per quadrature point.  With a, b Q2 nodes, r, s RT1
+// cell brings 47 weights per quadrature point.  With a, b Q2 nodes, r, s RT1
 // dofs of the axes d, d' (one nonzero reference component each):
 //   uu(c,d) = delta_cd S + N^{cd} + zeta_u D_c^T M^-1 D_d
 //     S   = sum_q [d_0 a, d_1 a, d_2 a, a] . mq [d_l b]                    (K = 27 x 4)
@@ -143,12 +143,13 @@ __device__ inline void store_tile(const JacCell &S, const d4_t &acc, double scal
 //   jphi / phij = sum_q ws q1 div r                                      (K = 27)
 // The first version mapped the 27 + 36 basis functions to physical space at
 // every point: half of a cell's 124 K cycles went into that staging and jj took
-// K = 27 x 4.  At 64 x 64 x 8 the kernel went from 3.4 to 1.93 ms (22 TFLOP/s of
-// matrix instructions, the matrix unit 45 % busy), at 8 x 8 x 3 from 52 to 34 us,
-// one cell's serial chain.  It is bound by latency at two waves a SIMD (225
+// K = 27 x 4.  At 64 x 64 x 8 the kernel went from 3.34 to 1.73 ms (33.7 TFLOP/s
+// of matrix instructions, the matrix unit 45 % busy), at 8 x 8 x 3 from 52 to 34
+// us, one cell's serial chain.  Up to 2,048 cells every workgroup takes one cell
+// and loads the tables for it alone.  It is bound by latency at two waves a SIMD (225
 // VGPRs): two accumulator chains in flight in the uu job instead of three cost
 // 6 %.  Writing the rows of one cell's own dofs straight into the CSR values
-// was tried: 1.93 -> 2.74 ms with a look-up for every row (2.34 for the p, phi
+// was tried, on a version of 1.93 ms: 2.74 ms with a look-up for every row (2.34 for the p, phi
 // and interior j rows alone), more than the sums save (2.20 -> 1.65, 1.76 ms).
 template <int MODE>
 __global__ __launch_bounds__(WG, 2) void k_cell_jacobian(int ncells, const int32_t *__restrict__ cells,
@@ -675,10 +676,12 @@ __device__ inline void row_segment(int a, int &start, int &len) {
 // rows have one or two holders, too little to keep in flight for a wave that
 // ends each row before it loads the next, so a wave runs through rows with the
 // next row's first RA_BATCH segments already loading, and a row of one holder,
-// which has no sums, goes to its place without the LDS: 2.19 -> 2.09 ms at
-// 64 x 64 x 8 (8.2 GB, 3.9 TB/s; 4.3 with the parts of cache lines beside the
-// segments, against 4.9 of a copy), 186 -> 148 us at 21 x 17 x 5 with the
-// skeleton term.  One round of workgroups (7 fit a CU by their LDS).
+// which has no sums, goes to its place without the LDS.  That pays where the
+// skeleton entries lengthen a row's work, 186 -> 148 us at 21 x 17 x 5; at 64 x
+// 64 x 8 without them it makes no difference to a wave per row and turn: 2.10 ->
+// 2.09 ms (8.2 GB, 3.9 TB/s; 4.3 with the parts of cache lines beside the
+// segments, against 4.9 of a copy).  Of the 2,048 workgroups 1,792 are resident
+// at once there (7 fit a CU by the LDS of their rows).
 constexpr int RA_WAVES = 4;
 constexpr int RA_BATCH = 4;
 constexpr int RA_BLOCKS = 256 * 8;

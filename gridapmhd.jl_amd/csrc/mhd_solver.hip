@@ -718,7 +718,8 @@ constexpr int PATCH_MAX = GJLarge::NMAX;  // unknowns of the largest vertex star
 
 // Static condensation of the vertex patches.  The 12 interior RT1 dofs of a
 // cell couple to the cell's own dofs only, and the star of a vertex that holds
-// one of a cell's other [u,j] dofs holds the whole cell.  With D the 12 x 12
+// one of a cell's other [u,j] dofs holds the whole cell (cells of which that is
+// not so are left out, see build_condensation).  With D the 12 x 12
 // interior block of cell c (the RT1 mass plus zeta_j div-div: symmetric
 // positive definite for zeta_j >= 0), eliminating the interior dofs of every
 // patch therefore gives exactly
@@ -729,7 +730,7 @@ constexpr int PATCH_MAX = GJLarge::NMAX;  // unknowns of the largest vertex star
 // them not interior to a cell: 129^2 / 225^2 = 33 % of the patch entries are
 // left, and 2 x 105 x 12 + 12^2 coupling entries per cell.  One FP32 application
 // at 64 x 64 x 8 (33,800 stars) went from 1.21 ms (6.5 GB of 225 x 225 inverses)
-// to 0.53 ms (2.6 GB in all), FP64 on 13 x 11 x 5 cells from 67 to 42 us.
+// to 0.56 ms (2.5 GB in all), FP64 on 13 x 11 x 5 cells from 67 to 39 us.
 constexpr int NI = 12, NB = NU + 24;   // interior dofs of a cell; its other [u,j] dofs, local index l
 __device__ inline int bdof_local(int l) { return l < NU ? l : l + (OFF_J - NU); }
 // row of F: the three components of a node side by side, as their dofs are
@@ -742,7 +743,7 @@ __device__ inline int frow(int l) { return l < NU ? (l % 27) * 3 + l / 27 : l; }
 // none.  E and A_bi in FP64 for the patch matrices (k_patch_build), E, F, G in
 // the precision of the smoother.  Entries are found through the rank map.  One
 // workgroup per cell, a thread per column; 23 KB of values are read and 31 to
-// 42 KB written per cell, small beside the patches (0.94 ms at 32,768 cells).
+// 42 KB written per cell, small beside the patches (0.97 ms at 32,768 cells).
 constexpr int CND_T = 192, CND_W = 2 * NI + NB;  // threads; columns of [D | I | A_ib]
 template <class TE>
 __global__ __launch_bounds__(CND_T) void k_condense(int ncells, const int32_t *__restrict__ dofs,
@@ -851,10 +852,9 @@ __global__ __launch_bounds__(CND_T) void k_condense(int ncells, const int32_t *_
 // entries per patch, where scanning the CSR rows visits 32 K columns).  SCAN:
 // the skeleton term, or an unusual dof or vertex table, couples dofs of a patch
 // beyond those cells; the rows are scanned then, each by a wave whose lanes
-// binary-search the columns among the sorted ids.  One
-// 1024-thread workgroup per patch.  LDSM: the matrix is built in LDS (129 x 129
-// FP64, 133 of the CU's 160 KB) and written once, coalesced; larger patches are
-// built in place in A.  5.1 ms for 33,800 patches; with the rows scanned and the
+// binary-search the columns among the sorted ids.  One 1024-thread workgroup
+// per patch.  LDSM: the matrix is built in LDS (129 x 129 FP64, 133 of the CU's
+// 160 KB) and written once, coalesced; larger patches are built in place in A.  5.1 ms for 33,800 patches; with the rows scanned and the
 // cells taken one after another, each waiting for its loads, 7.5 ms (the full
 // 225 x 225 matrices, scattered into cleared memory, 18 ms).
 template <bool LDSM, bool SCAN>
@@ -1003,10 +1003,9 @@ __global__ __launch_bounds__(1024) void k_patch_build(int PS, const int32_t *__r
 
 // rt_b = r_b - sum over the cells holding b of F_c[b] . r_i(c), FP64 sums;
 // interior dofs of condensed cells are skipped (`map`: where the others go, or
-// null).  Four lanes per dof share its
-// (up to eight) cells, so the chain of dependent loads is at most two cells
-// long: a level of 200 cells takes 5 us (one lane per dof: 11 us), 32,768
-// cells 60 us (F read once, 138 MB).
+// null).  Four lanes per dof share its (up to eight) cells, so the chain of
+// dependent loads is at most two cells long: a level of 200 cells takes 5 us
+// (one lane per dof: 11 us), 32,768 cells 60 us (F read once, 138 MB).
 template <class T, class TE>
 __global__ __launch_bounds__(256) void k_cond_rhs(int64_t n1, const int32_t *__restrict__ crow,
                                                   const int32_t *__restrict__ centry,
@@ -1259,9 +1258,10 @@ __global__ __launch_bounds__(256) void k_cond_inner(int ncells, const int32_t *_
 // rows) and RJ columns (one of every block of TC columns); the last row and
 // column live in LDS.  GJSmall's FP64 tile is 64 values (128 VGPRs) on 256
 // threads, so two to three workgroups share a CU and hide each other's
-// barriers (one per step): 12.4 ms for 33,800 patches (13.2 with three barriers
-// per step), where the full stars took 61 ms on GJLarge's 98 values on 512
-// threads, one workgroup per CU.
+// barriers (one per step): 10.6 ms for 33,800 patches (12.1 with the diagonal
+// read in a step before the matrix, a millisecond more with three barriers per
+// step), where the full stars took 61 ms on GJLarge's 98 values on 512 threads,
+// one workgroup per CU.
 //
 // Elimination step k, with the pivot column saved as f and zeroed and the
 // pivot row p saved as r = a_p,: / a_pk (r_k = 1 / a_pk) and zeroed, updates
@@ -1774,8 +1774,8 @@ __global__ __launch_bounds__(G::T) void k_patch_gj(int PS, int ld, const int32_t
 // the VEC = 16 bytes / sizeof(MP) rows that a lane loads at once, so the
 // ld / VEC lanes of a column and the next columns' lanes read one linear
 // stream; the NG column groups of the workgroup are summed through LDS.  The
-// kernel is bound by that stream: 2.30 GB of FP32 inverses (33,800 stars) in
-// 0.375 ms, 6.1 TB/s.
+// kernel is bound by that stream: 2.36 GB of traffic for the FP32 inverses of
+// 33,800 stars in 0.40 ms, 5.9 TB/s.
 template <class MP>
 struct MatVec {
   static constexpr int VEC = 16 / (int)sizeof(MP);
